@@ -1706,7 +1706,7 @@ template <class T>
 void krylovIteration(const Ctx& C, vol_matrix A, const Plan& P, const Krylov<T>& k, bool isPCG, bool ex) {
     const int n = A->mesh->n;
     const bool fuse = !ex;
-    const int nparts = ex ? RED_BLOCKS_EXACT : RED_BLOCKS;
+    const int nparts = ex ? vec_exact_blocks(n) : RED_BLOCKS;
     const int sellParts = sell_grid_blocks(A->mesh->sell.nslices);
     const Level0<T> L0 = level0(A, (T*)nullptr);
     if (isPCG) {  // LinearSolver.cpp:176-201
@@ -1869,7 +1869,7 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
                         mixed ? ct.innerRelTol : 0.0, mixed && isPCG ? 1 : 0);
     // initial residual and normalisation (LinearSolver.cpp:150-169)
     sell<double>(C, OP_AMUL, XL_PLAIN, V, A->coef.p, A->diag.p, x, nullptr, wA);
-    const int nparts = ex ? RED_BLOCKS_EXACT : RED_BLOCKS;
+    const int nparts = ex ? vec_exact_blocks(n) : RED_BLOCKS;
     vec<double>(C, V_SUM_X, n, ex, x);
     fin(C, FIN_XREF, 1, ex, nparts);
     sell<double>(C, OP_AMUL, XL_UNIFORM, V, A->coef.p, A->diag.p, nullptr, nullptr, pA, 1.0, nullptr, nullptr,

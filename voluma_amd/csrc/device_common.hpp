@@ -141,30 +141,40 @@ __device__ __forceinline__ void exact_add_wave(long long* bins, int* nfFlag, dou
     }
 }
 
-// Carry-normalise bins (Comm.cpp:114-121): afterwards bins[0..70] ∈ [0, 2^32).
-__device__ __forceinline__ void exact_normalize(long long* b) {
-    for (int k = 0; k < NBINS - 1; ++k) {
-        const long long c = b[k] >> 32;
-        b[k] -= c * (1ll << 32);
-        b[k + 1] += c;
+// Carry-normalise bins (Comm.cpp:114-121) lo..hi, the others zero: afterwards each of
+// them is in [0, 2^32). Carries leave the window upwards, so hi grows (a double's pieces
+// end in bin 65 and 2^31 of them carry two bins further, so never to the last bin). A
+// total below zero ends in a carry of −1, which would fill every bin above: it stays the
+// return value.
+__device__ __forceinline__ long long exact_normalize(long long* b, int lo, int& hi) {
+    long long c = 0;
+    for (int k = lo; k < NBINS && (k <= hi || (c != 0 && c != -1)); ++k) {
+        const long long v = (k <= hi ? b[k] : 0) + c;
+        c = v >> 32;
+        b[k] = v - c * (1ll << 32);
+        if (k > hi) hi = k;
     }
+    return c;
 }
 
-// binsToDouble (Comm.cpp:135-156) on a private copy.
-__device__ __forceinline__ double exact_to_double(long long* b, int nfFlag) {
+// binsToDouble (Comm.cpp:135-156) of the bins lo..hi (the others zero; lo > hi: none), which
+// it changes: |total| in canonical bins, converted from the top bin down. Only the bins of
+// the window and the few its carries reach are visited; the others add nothing.
+__device__ __forceinline__ double exact_to_double(long long* b, int lo, int hi, int nfFlag) {
     if (nfFlag) {
         if ((nfFlag & NF_NAN) || ((nfFlag & NF_PINF) && (nfFlag & NF_NINF))) return __longlong_as_double(0x7ff8000000000000ll);
         return (nfFlag & NF_PINF) ? __longlong_as_double(0x7ff0000000000000ll) : __longlong_as_double((long long)0xfff0000000000000ull);
     }
-    exact_normalize(b);
     double sign = 1.0;
-    if (b[NBINS - 1] < 0) {
+    if (exact_normalize(b, lo, hi) < 0) {  // total = Σ b·2^(32k) − 2^(32(hi+1)): negate
         sign = -1.0;
-        for (int k = 0; k < NBINS; ++k) b[k] = -b[k];
-        exact_normalize(b);
+        for (int k = lo; k <= hi; ++k) b[k] = -b[k];
+        b[hi + 1] = 1;
+        ++hi;
+        exact_normalize(b, lo, hi);
     }
     double r = 0.0;
-    for (int k = NBINS - 1; k >= 0; --k)
+    for (int k = hi; k >= lo; --k)
         if (b[k] != 0) r += ldexp((double)b[k], 32 * k - 1074);
     return sign * r;
 }

@@ -760,6 +760,13 @@ __global__ __launch_bounds__(RED_THREADS) void k_vec_fast(VecArgsT<T> A, double*
     }
 }
 
+// Grid of the exact reductions: a block per RED_THREADS rows up to RED_BLOCKS_EXACT, so a
+// small system leaves the finalize few partials.
+int vec_exact_blocks(int n) { return std::max(std::min((n + RED_THREADS - 1) / RED_THREADS, RED_BLOCKS_EXACT), 1); }
+
+// A block's exact partial in one word: non-finite flags and the window of non-zero bins.
+__device__ __forceinline__ int exact_info(int nf, int lo, int hi) { return nf | (lo << 8) | ((hi + 1) << 16); }
+
 template <int OP, int NRED>
 __global__ __launch_bounds__(RED_THREADS) void k_vec_exact(VecArgs A, long long* xpart, int* xnf, int maxBlk) {
     if (!vec_should_run<OP>(A)) return;
@@ -777,14 +784,27 @@ __global__ __launch_bounds__(RED_THREADS) void k_vec_exact(VecArgs A, long long*
         exact_add_wave(bins[0], &nf[0], r0, act);
         if constexpr (NRED > 1) exact_add_wave(bins[1], &nf[1], r1, act);
     }
-    __syncthreads();
-    if (threadIdx.x < NRED) exact_normalize(bins[threadIdx.x]);
+    // the bins as they are (n < 2^31 pieces below 2^32 fit an int64) and the window of the
+    // ones that hold something, so that the finalize need not read the rest
+    __shared__ int lo[NRED], hi[NRED];
+    if (threadIdx.x < NRED) {
+        lo[threadIdx.x] = NBINS;
+        hi[threadIdx.x] = -1;
+    }
     __syncthreads();
     for (int k = threadIdx.x; k < NRED * NBINS; k += blockDim.x) {
         const int q = k / NBINS, bn = k % NBINS;
-        xpart[(size_t(q) * maxBlk + blockIdx.x) * NBINS + bn] = bins[q][bn];
+        const long long v = bins[q][bn];
+        xpart[(size_t(q) * maxBlk + blockIdx.x) * NBINS + bn] = v;
+        if (v != 0) {
+            atomicMin(&lo[q], bn);
+            atomicMax(&hi[q], bn);
+        }
     }
-    if (threadIdx.x < NRED) xnf[threadIdx.x * maxBlk + blockIdx.x] = nf[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x < NRED)
+        xnf[threadIdx.x * maxBlk + blockIdx.x] =
+            exact_info(nf[threadIdx.x], lo[threadIdx.x], hi[threadIdx.x]);
 }
 
 template <int OP, class T>
@@ -796,8 +816,8 @@ static void vec_dispatch(hipStream_t st, const VecArgsT<T>& a, bool exact, const
                              : 0;
     if constexpr (NRED > 0 && std::is_same_v<T, double>) {
         if (exact) {
-            hipLaunchKernelGGL((k_vec_exact<OP, NRED>), dim3(RED_BLOCKS_EXACT), dim3(RED_THREADS), 0, st, a, R.xpart,
-                               R.xnf, R.maxBlkExact);
+            hipLaunchKernelGGL((k_vec_exact<OP, NRED>), dim3(vec_exact_blocks(a.n)), dim3(RED_THREADS), 0, st, a,
+                               R.xpart, R.xnf, R.maxBlkExact);
             return;
         }
     }
@@ -982,9 +1002,22 @@ __device__ __forceinline__ void publish(const DevScalars& S, DevScalars* hostOut
     if (hostOut) *hostOut = S;
 }
 
-__global__ __launch_bounds__(FIN_THREADS) void k_finalize(int op, int nred, int exact, int nparts, const double* part,
-                                                  int maxBlk, const long long* xpart, const int* xnf, int maxBlkExact,
-                                                  DevScalars* Sp, double* result, DevScalars* hostOut) {
+// The scalar step of a finalize on its thread 0, v0 and v1 reduced.
+__device__ __forceinline__ void fin_apply(int op, int nred, double v0, double v1, DevScalars* Sp, double* result,
+                                          DevScalars* hostOut) {
+    if (op == FIN_STORE) {
+        if (result) {
+            result[0] = v0;
+            if (nred > 1) result[1] = v1;
+        }
+        return;
+    }
+    fin_step(op, *Sp, Sp[1], v0, v1);
+    publish(*Sp, hostOut);
+}
+
+__global__ __launch_bounds__(FIN_THREADS) void k_finalize(int op, int nred, int nparts, const double* part, int maxBlk,
+                                                          DevScalars* Sp, double* result, DevScalars* hostOut) {
     DevScalars& S = *Sp;
     if (op == FIN_INNER_START) {  // no reduction: S[1] ← fresh inner solve, or done with S[0]
         if (threadIdx.x == 0) inner_start(S, Sp[1]);
@@ -996,46 +1029,93 @@ __global__ __launch_bounds__(FIN_THREADS) void k_finalize(int op, int nred, int 
     }
     __shared__ double vals[MAX_RED];
     __shared__ double sh[FIN_THREADS / WAVE];
-    __shared__ long long bins[NBINS];
-    __shared__ int nfl;
     for (int q = 0; q < nred; ++q) {
-        if (!exact) {
-            const double t = fin_sum(part + size_t(q) * maxBlk, nparts, sh);
-            if (threadIdx.x == 0) vals[q] = t;
-        } else {
-            if (threadIdx.x == 0) nfl = 0;
-            __syncthreads();
-            if (threadIdx.x < NBINS) {
-                long long s = 0;
-                for (int k = 0; k < nparts; ++k) s += xpart[(size_t(q) * maxBlkExact + k) * NBINS + threadIdx.x];
-                bins[threadIdx.x] = s;
-            }
-            for (int k = threadIdx.x; k < nparts; k += blockDim.x) {
-                const int f = xnf[q * maxBlkExact + k];
-                if (f) atomicOr(&nfl, f);
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) vals[q] = exact_to_double(bins, nfl);
-        }
+        const double t = fin_sum(part + size_t(q) * maxBlk, nparts, sh);
+        if (threadIdx.x == 0) vals[q] = t;
         __syncthreads();
     }
-    if (threadIdx.x != 0) return;
-    const double v0 = vals[0], v1 = nred > 1 ? vals[1] : 0.0;
-    if (op == FIN_STORE) {
-        if (result) {
-            result[0] = v0;
-            if (nred > 1) result[1] = v1;
-        }
+    if (threadIdx.x == 0) fin_apply(op, nred, vals[0], nred > 1 ? vals[1] : 0.0, Sp, result, hostOut);
+}
+
+// The finalize of exact sums. Integer bins add up to the same value in any order, so the
+// blocks' partials are read by the whole workgroup: first the blocks' info words (one per
+// thread, nparts ≤ FINX_THREADS), then only the window of bins any block used, P threads
+// (the window rounded up to a power of two) per partial and FINX_LOADS loads in flight
+// each, a tree over the FINX_THREADS / P groups, and the carries and the conversion over
+// the window on one thread. Latency-bound: two round trips, the tree and ~10 bins in turn.
+// Adding the partials bin by bin on 72 threads and carrying through all 72 bins took 116 µs
+// per launch at 512 partials; a reproducible PCG iteration on 24,480 cells (three of these)
+// went from 375 to 38 µs with this and the smaller grids of vec_exact_blocks.
+constexpr int FINX_THREADS = 512;
+constexpr int FINX_LOADS = 8;
+static_assert(RED_BLOCKS_EXACT <= FINX_THREADS, "one info word per thread");
+__global__ __launch_bounds__(FINX_THREADS) void k_finalize_exact(int op, int nred, int nparts, const long long* xpart,
+                                                                 const int* xnf, int maxBlk, DevScalars* Sp,
+                                                                 double* result, DevScalars* hostOut) {
+    if (op != FIN_STORE && Sp->done) {
+        if (threadIdx.x == 0) publish(*Sp, hostOut);
         return;
     }
-    fin_step(op, S, Sp[1], v0, v1);
-    publish(S, hostOut);
+    __shared__ double vals[MAX_RED];
+    __shared__ long long sum[FINX_THREADS];
+    __shared__ long long bins[NBINS];
+    __shared__ int nfl, lo, hi;
+    const int t = threadIdx.x;
+    for (int q = 0; q < nred; ++q) {
+        if (t == 0) {
+            nfl = 0;
+            lo = NBINS;
+            hi = -1;
+        }
+        __syncthreads();
+        const int f = t < nparts ? xnf[q * maxBlk + t] : exact_info(0, NBINS, -1);
+        const int wlo = wave_min_i((f >> 8) & 0xff), whi = wave_max_i((f >> 16) - 1);
+        if (t % WAVE == 0) {
+            atomicMin(&lo, wlo);
+            atomicMax(&hi, whi);
+        }
+        if (f & 0xff) atomicOr(&nfl, f & 0xff);
+        __syncthreads();
+        const int l = lo, w = hi - lo + 1;
+        int P = 8;
+        while (P < w) P *= 2;  // ≤ 128
+        const int b = t % P, g = t / P, groups = FINX_THREADS / P;
+        long long s = 0;
+        if (b < w) {
+            const long long* src = xpart + size_t(q) * maxBlk * NBINS + l + b;
+            for (int k0 = g; k0 < nparts; k0 += groups * FINX_LOADS) {
+                long long v[FINX_LOADS];
+#pragma unroll
+                for (int u = 0; u < FINX_LOADS; ++u) {
+                    const int k = k0 + u * groups;
+                    v[u] = k < nparts ? src[size_t(k) * NBINS] : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < FINX_LOADS; ++u) s += v[u];
+            }
+        }
+        sum[t] = s;
+        for (int o = groups / 2; o > 0; o /= 2) {
+            __syncthreads();
+            if (g < o) sum[t] += sum[t + o * P];
+        }
+        __syncthreads();
+        if (t < w) bins[l + t] = sum[t];
+        __syncthreads();
+        if (t == 0) vals[q] = exact_to_double(bins, l, hi, nfl);
+        __syncthreads();
+    }
+    if (t == 0) fin_apply(op, nred, vals[0], nred > 1 ? vals[1] : 0.0, Sp, result, hostOut);
 }
 
 void launch_finalize(hipStream_t st, int op, int nred, bool exact, int nparts, const RedScratch& R, DevScalars* S,
                      DevScalars* hostOut) {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, op, nred, exact ? 1 : 0, nparts, R.part, R.maxBlk,
-                       R.xpart, R.xnf, R.maxBlkExact, S, R.result, hostOut);
+    if (exact && op != FIN_INNER_START)
+        hipLaunchKernelGGL(k_finalize_exact, dim3(1), dim3(FINX_THREADS), 0, st, op, nred, nparts, R.xpart, R.xnf,
+                           R.maxBlkExact, S, R.result, hostOut);
+    else
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, op, nred, nparts, R.part, R.maxBlk, S,
+                           R.result, hostOut);
 }
 
 __global__ void k_init_scalars(DevScalars* S, double tol, double relTol, int maxIter, int minIter, int nSweeps, int n,

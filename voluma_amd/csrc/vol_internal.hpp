@@ -105,18 +105,18 @@ enum FinOp : int {
 };
 
 // Reduction scratch: fast mode uses `nblk` double partials per reduced quantity;
-// exact mode uses `nblk` × 72 int64 bins + a non-finite flag per block.
+// exact mode uses `nblk` × 72 int64 bins + one info word per block.
 struct RedScratch {
     double* part = nullptr;     // [maxRed][maxBlk]
     long long* xpart = nullptr; // [maxRed][maxBlkExact][72]
-    int* xnf = nullptr;         // [maxRed][maxBlkExact]
+    int* xnf = nullptr;         // [maxRed][maxBlkExact]: non-finite flags | window of non-zero bins
     double* result = nullptr;   // [maxRed] (FIN_STORE)
     int* arrive = nullptr;      // ticket counter of the last-block finalize (nullable; 0 between launches)
     int maxBlk = 0, maxBlkExact = 0;
 };
 
 constexpr int RED_BLOCKS = 1024;       // grid of fast reduction kernels
-constexpr int RED_BLOCKS_EXACT = 512;  // grid of exact reduction kernels
+constexpr int RED_BLOCKS_EXACT = 512;  // largest grid of exact reduction kernels
 constexpr int RED_THREADS = 256;
 constexpr int MAX_RED = 2;
 
@@ -235,6 +235,7 @@ void launch_finalize(hipStream_t st, int op, int nred, bool exact, int nparts, c
 int vec_has_reduction(int op);
 // blocks of a fast-sum vector op (= partials of its reduction; maxBlk: the scratch's)
 int vec_fast_blocks(int op, int n, int maxBlk);
+int vec_exact_blocks(int n);
 
 void launch_clear_exit(hipStream_t st, DevScalars* S);
 void launch_init_scalars(hipStream_t st, DevScalars* S, double tol, double relTol, int maxIter, int minIter,
