@@ -1,0 +1,82 @@
+"""Triangular sweeps over one and several chunks against the oracle's sequential loops, bit
+for bit (exact sums), on graphs at the edges of the sweep plans: the largest one-chunk
+size and its neighbour, a chain (one row per level), rows of every length the kernels
+treat apart (up to 8, 12 and 20 entries, longer ones, a hub of hundreds), neighbours so
+scattered that a chunk's halo does not fit its LDS, and more sweeps than one launch takes.
+"""
+import numpy as np
+import pytest
+
+import voluma_amd as va
+from oracle import oracle as O
+from voluma_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+def _band(n, deg, width, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.integers(0, n - 1, n * deg // 2)
+    b = np.minimum(a + 1 + rng.integers(0, width, a.size), n - 1)
+    return a, b
+
+
+def _graph(name):
+    rng = np.random.default_rng(5)
+    if name == "chain":
+        n = 8193
+        a, b = np.arange(n - 1), np.arange(1, n)
+    elif name == "one":
+        n, (a, b) = 8192, _band(8192, 6, 300, 1)
+    elif name == "two":
+        n, (a, b) = 8193, _band(8193, 6, 300, 2)
+    elif name == "wide":
+        n, (a, b) = 12345, _band(12345, 14, 900, 3)
+    elif name == "far":  # neighbours anywhere: 4096-cell chunks see over 16,300 other cells
+        n = 30000
+        a, b = _band(n, 16, n, 4)
+    elif name == "hub":
+        n, (a, b) = 9001, _band(9001, 5, 200, 6)
+        a = np.concatenate([a, np.full(400, 4500), rng.integers(0, 4500, 400)])
+        b = np.concatenate([b, 4501 + rng.permutation(4500)[:400], np.full(400, 4500)])
+    else:
+        m = M.box(23, 21, 19)
+        return m.n_cells, m.owner[: m.n_internal], m.neighbour
+    keep = a < b
+    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
+    rng.shuffle(e)  # face order unrelated to cell order
+    flip = rng.random(e.size) < 0.3  # faces owned by the higher cell too
+    l, u = (e // n).astype(np.int32), (e % n).astype(np.int32)
+    return n, np.where(flip, u, l), np.where(flip, l, u)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = va.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("name", ["chain", "one", "two", "wide", "far", "hub", "box"])
+def test_sweeps_bit_exact_vs_oracle(ctx, name):
+    n, own, nei = _graph(name)
+    rng = np.random.default_rng(9)
+    nf = own.size
+    u = -rng.uniform(0.5, 1.5, nf)
+    lo = u * rng.uniform(0.7, 1.3, nf)
+    d = 0.1 + np.bincount(own, np.maximum(-u, -lo), n) + np.bincount(nei, np.maximum(-u, -lo), n)
+    b = rng.uniform(-1, 1, n)
+    x0 = rng.uniform(-1, 1, n)
+    lm = va.LduMesh(ctx, n, own, nei)
+    om = O.LduMesh(n, own, nei)
+    A, N = va.LduMatrix(lm, d, u), va.LduMatrix(lm, d, u, lo)
+    for solver, pre, sym, sweeps, mx in (("GaussSeidel", "none", True, 1, 2), ("GaussSeidel", "none", False, 2, 4),
+                                         ("GaussSeidel", "none", True, 5, 5), ("symGaussSeidel", "none", False, 1, 2),
+                                         ("PCG", "DIC", True, 1, 3), ("PBiCGStab", "DILU", False, 1, 3)):
+        xo, po = om.solve(d, u, None if sym else lo, b, x0=x0, solver=solver, preconditioner=pre, tolerance=1e-30,
+                          max_iter=mx, n_sweeps=sweeps, mode=O.MODE_EXACT)
+        x = x0.copy()
+        p = va.solve_ldu(A if sym else N, b, x, va.SolverControls(solver, pre, 1e-30, 0.0, mx, nSweeps=sweeps,
+                                                                  sums=va.SUMS_EXACT))
+        assert p.iterations == po["iterations"] and p.finalResidual == po["finalResidual"], (solver, sweeps)
+        assert np.array_equal(x, xo), (solver, sweeps)

@@ -106,10 +106,12 @@ struct vol_mesh_s {
     int nb = -1;
     DevBuf<int> bOff, bList;
     DevBuf<int> dOwn, dNei;  // device owner/neighbour, uploaded on first use
-    // level schedules and neighbour lists of the triangular sweeps (DIC/DILU,
-    // Gauss–Seidel), built on first use
+    // plans of the triangular sweeps, built on first use: the DIC/DILU rows (entry source:
+    // face and side), and Gauss–Seidel rows per (GAMG level, backward, sweeps) with the
+    // SELL or CSR slot as entry source
     std::mutex sweepMu;
-    bool sweepReady = false;
+    std::unique_ptr<SweepPlanDev> diluF, diluB;
+    std::map<std::tuple<int, int, int>, std::unique_ptr<SweepPlanDev>> gsPlans;
     // geometry of the explicit corrector operators (vol_mesh_set_geometry) and their
     // staging buffers for host pointers
     bool geomSet = false;
@@ -118,38 +120,12 @@ struct vol_mesh_s {
     DevBuf<double> gV, gSf, gMagSf, gW, gD, gSkew;
     DevBuf<double> fst[8], fout, fgls;
     DevBuf<int> fsti;
-    LevelOrderDev ordF;  // forward level order of level 0 (DIC/DILU factor)
-    DevBuf<int> lowOff, lowCol, lowSrc, upOff, upCol, upSrc;
-    LevelEllDev diluF, diluB;  // substitution rows (entry source: list index)
-    LevelEllDev gsF, gsB;      // Gauss–Seidel rows of level 0 (entry source: SELL slot)
-    // Gauss–Seidel GAMG smoother: rows of the coarse GAMG levels 1 .. nL−2 (index =
-    // GAMG level; level 0 uses gsF/gsB)
-    struct LevelOrder {
-        LevelEllDev F, B;
-    };
-    bool gsLevelsReady = false;
-    std::vector<std::unique_ptr<LevelOrder>> gsLev;
-    // k consecutive Gauss–Seidel sweeps of one direction as one level schedule, per
-    // (GAMG level, backward, k); built on first use
-    std::map<std::tuple<int, int, int>, std::unique_ptr<LevelEllDev>> gsMulti;
-    SweepView sweepView() const {
-        SweepView v;
-        v.lowOff = lowOff.p;
-        v.lowCol = lowCol.p;
-        v.lowSrc = lowSrc.p;
-        v.upOff = upOff.p;
-        v.upCol = upCol.p;
-        v.upSrc = upSrc.p;
-        return v;
-    }
 };
 
 struct MatLevel {
     DevBuf<double> diag, rD, Fu, Fl, coef, bufA, bufB, r, x;
     DevBuf<double> z;  // ω·(r·rD) of the restricted residual: the first smoothing from zero
     DevBuf<float> diag32, rD32, coef32, bufA32, bufB32, r32, x32, z32;  // mixed precision
-    DevBuf<double> gsCF, gsCB;  // Gauss–Seidel smoother coefficients (LevelEll layouts)
-    DevBuf<float> gsCF32, gsCB32;
     DevBuf<double> coefR;  // the level's rows in restriction order (LevelDev::rrCsr)
     DevBuf<float> coefR32;
 };
@@ -173,23 +149,19 @@ struct vol_matrix_s {
     DevBuf<int> status;
     // FP32 copies for mixed precision, built lazily after each vol_matrix_set
     bool mixedReady = false, mixedGamg = false;
-    // DIC/DILU factor (per cell) and substitution coefficients (per list entry), built
+    // DIC/DILU factor (per cell) and substitution coefficients (per plan entry), built
     // lazily after each vol_matrix_set; FP32 copies for mixed precision
     bool diluReady = false, dilu32Ready = false;
-    DevBuf<double> dluD, dluR, dluPf, dluPb, dluEf, dluEb;  // Ef/Eb: pf/pb in the LevelEll layouts
+    DevBuf<double> dluD, dluR, dluEf, dluEb;
     DevBuf<float> dluR32, dluEf32, dluEb32;
-    // Gauss–Seidel coefficients in the LevelEll layouts: level 0 (solver and smoother)
-    // and the coarse levels (smoother), FP32 copies for mixed precision
-    bool gsReady = false, gsLevReady = false, gs32Ready = false;
-    DevBuf<double> gsCF, gsCB;
-    std::map<std::tuple<int, int, int>, DevBuf<double>> gsMultiCoef;  // per gsMulti schedule
-    DevBuf<float> gsCF32, gsCB32;
+    // Gauss–Seidel coefficients per entry of the mesh's gsPlans, FP32 ones for mixed
+    // precision; gathered on first use after each vol_matrix_set
+    std::map<std::tuple<int, int, int>, DevBuf<double>> gsCoef;
+    std::map<std::tuple<int, int, int>, DevBuf<float>> gsCoef32;
     DevBuf<float> coef32, diag32, rD32;
     DevBuf<TailLevel32> tail32;
     DevBuf<float> ir, iw, ip, iq, ie, ir0, iy, iAy, is, iz, it;  // inner-solve vectors
     DevBuf<float> iz0;  // inner PCG: ω·(r·rD) kept with the inner residual
-    DevBuf<double> diluTmp;  // sync-free DILU: the forward substitution's result
-    DevBuf<float> diluTmp32;
     // solve work vectors
     DevBuf<double> vx, vb, vr, vw, vp, vq, wA, pA, r0, y, Ay, s, z, t;
     DevBuf<double> hx, hy;  // staging for host-pointer calls
@@ -523,89 +495,6 @@ void toFloat(hipStream_t st, const double* a, float* w, size_t n) {
 
 // FP32 copies of the level-0 matrix and, with GAMG, of every coarse level and the tail
 // descriptors (the coarsest LU stays FP64). Values are rounded from the FP64 ones.
-// Level schedules of the triangular sweeps (sweep_kernels.hip). Lower list of cell u:
-// its neighbours l < u in ascending (l, face) order, the order of the reference's
-// (u, l)-sorted face list (LinearSolver.cpp:29-51); upper list of cell l: its neighbours
-// u > l in descending (u, face) order, the order of the backward face loop.
-void buildSweep(vol_mesh m) {
-    std::lock_guard<std::mutex> guard(m->sweepMu);
-    if (m->sweepReady) return;
-    const int n = m->n, nf = m->nf;
-    std::vector<int> lowOff(n + 1, 0), upOff(n + 1, 0);
-    for (int f = 0; f < nf; ++f) {
-        const int o = m->own[f], e = m->nei[f];
-        ++lowOff[std::max(o, e) + 1];
-        ++upOff[std::min(o, e) + 1];
-    }
-    for (int c = 0; c < n; ++c) {
-        lowOff[c + 1] += lowOff[c];
-        upOff[c + 1] += upOff[c];
-    }
-    // entries (neighbour, face); side of the list's own row: 0 when it owns the face
-    std::vector<std::pair<int, int>> low(nf), up(nf);
-    {
-        std::vector<int> fl(lowOff.begin(), lowOff.end() - 1), fu(upOff.begin(), upOff.end() - 1);
-        for (int f = 0; f < nf; ++f) {
-            const int o = m->own[f], e = m->nei[f];
-            const int l = std::min(o, e), u = std::max(o, e);
-            low[fl[u]++] = {l, f};
-            up[fu[l]++] = {u, f};
-        }
-    }
-    std::vector<int> lowCol(nf), lowSrc(nf), upCol(nf), upSrc(nf), levF(n, 0), levB(n, 0);
-    for (int c = 0; c < n; ++c) {
-        std::sort(low.begin() + lowOff[c], low.begin() + lowOff[c + 1]);
-        std::sort(up.begin() + upOff[c], up.begin() + upOff[c + 1], std::greater<>());
-        for (int k = lowOff[c]; k < lowOff[c + 1]; ++k) {
-            const int f = low[k].second;
-            lowCol[k] = low[k].first;
-            lowSrc[k] = (f << 1) | (m->own[f] == c ? 0 : 1);
-            levF[c] = std::max(levF[c], levF[low[k].first] + 1);
-        }
-        for (int k = upOff[c]; k < upOff[c + 1]; ++k) {
-            const int f = up[k].second;
-            upCol[k] = up[k].first;
-            upSrc[k] = (f << 1) | (m->own[f] == c ? 0 : 1);
-        }
-    }
-    for (int c = n - 1; c >= 0; --c)
-        for (int k = upOff[c]; k < upOff[c + 1]; ++k) levB[c] = std::max(levB[c], levB[upCol[k]] + 1);
-    auto order = [n](const std::vector<int>& lev, std::vector<int>& off, std::vector<int>& perm) {
-        const int nl = n ? *std::max_element(lev.begin(), lev.end()) + 1 : 0;
-        off.assign(nl + 1, 0);
-        for (int c = 0; c < n; ++c) ++off[lev[c] + 1];
-        for (int L = 0; L < nl; ++L) off[L + 1] += off[L];
-        std::vector<int> fill(off.begin(), off.end() - 1);
-        perm.assign(n, 0);
-        for (int c = 0; c < n; ++c) perm[fill[lev[c]]++] = c;
-    };
-    std::vector<int> permF, permB, offF, offB;
-    order(levF, offF, permF);
-    order(levB, offB, permB);
-    hipStream_t st = m->ctx->stream;
-    m->ordF.build(offF, permF, st);
-    std::vector<int> idx(nf);
-    for (int k = 0; k < nf; ++k) idx[k] = k;
-    m->diluF.build(offF, permF, lowOff, lowCol, idx, st);
-    m->diluB.build(offB, permB, upOff, upCol, idx, st);
-    {
-        std::vector<int> ro, rc, rs;
-        sellRows(m->sell, ro, rc, rs);
-        m->gsF.build(offF, permF, ro, rc, rs, st);
-        m->gsB.build(offB, permB, ro, rc, rs, st);
-    }
-    m->lowOff.upload(lowOff, st);
-    m->upOff.upload(upOff, st);
-    if (nf) {
-        m->lowCol.upload(lowCol, st);
-        m->lowSrc.upload(lowSrc, st);
-        m->upCol.upload(upCol, st);
-        m->upSrc.upload(upSrc, st);
-    }
-    HIPCHECK(hipStreamSynchronize(st));
-    m->sweepReady = true;
-}
-
 // Forward / backward level order of a graph given by its edges (l[k] < u[k]): cells by
 // level, then by index; offF/offB hold the level offsets.
 void levelOrder(int n, const std::vector<int>& l, const std::vector<int>& u, std::vector<int>& offF,
@@ -645,74 +534,98 @@ void levelOrder(int n, const std::vector<int>& l, const std::vector<int>& u, std
     order(levB, offB, permB);
 }
 
-// Level orders of the coarse GAMG levels for the Gauss–Seidel smoother.
-void buildGsLevels(vol_mesh m) {
-    buildSweep(m);
+// Plans of the DIC/DILU sweeps (sweep_kernels.hip). Forward rows: a cell's neighbours
+// l < u in ascending (l, face) order, the order of the reference's (u, l)-sorted face list
+// (LinearSolver.cpp:29-51); backward rows: its neighbours u > l in descending (u, face)
+// order, the order of the backward face loop.
+void buildDiluPlans(vol_mesh m) {
     std::lock_guard<std::mutex> guard(m->sweepMu);
-    if (m->gsLevelsReady) return;
-    const int nL = int(m->lv.size());
-    m->gsLev.clear();
-    m->gsLev.resize(std::max(nL, 1));
-    for (int k = 1; k + 1 < nL; ++k) {
-        auto o = std::make_unique<vol_mesh_s::LevelOrder>();
-        std::vector<int> pf, pb, of, ob, ro, rc, rs;
-        levelOrder(m->H[k].n, m->H[k].l, m->H[k].u, of, pf, ob, pb);
-        sellRows(m->lv[k]->sell, ro, rc, rs);
-        o->F.build(of, pf, ro, rc, rs, m->ctx->stream);
-        o->B.build(ob, pb, ro, rc, rs, m->ctx->stream);
-        m->gsLev[k] = std::move(o);
+    if (m->diluF) return;
+    const int n = m->n, nf = m->nf;
+    std::vector<int> lowOff(n + 1, 0), upOff(n + 1, 0), l(nf), u(nf);
+    for (int f = 0; f < nf; ++f) {
+        l[f] = std::min(m->own[f], m->nei[f]);
+        u[f] = std::max(m->own[f], m->nei[f]);
+        ++lowOff[u[f] + 1];
+        ++upOff[l[f] + 1];
     }
-    HIPCHECK(hipStreamSynchronize(m->ctx->stream));
-    m->gsLevelsReady = true;
+    for (int c = 0; c < n; ++c) {
+        lowOff[c + 1] += lowOff[c];
+        upOff[c + 1] += upOff[c];
+    }
+    std::vector<std::pair<int, int>> low(nf), up(nf);  // (neighbour, face)
+    {
+        std::vector<int> fl(lowOff.begin(), lowOff.end() - 1), fu(upOff.begin(), upOff.end() - 1);
+        for (int f = 0; f < nf; ++f) {
+            low[fl[u[f]]++] = {l[f], f};
+            up[fu[l[f]]++] = {u[f], f};
+        }
+    }
+    std::vector<int> lowCol(nf), lowSrc(nf), upCol(nf), upSrc(nf);
+    for (int c = 0; c < n; ++c) {
+        std::sort(low.begin() + lowOff[c], low.begin() + lowOff[c + 1]);
+        std::sort(up.begin() + upOff[c], up.begin() + upOff[c + 1], std::greater<>());
+        for (int k = lowOff[c]; k < lowOff[c + 1]; ++k) {
+            lowCol[k] = low[k].first;
+            lowSrc[k] = (low[k].second << 1) | (m->own[low[k].second] == c ? 0 : 1);
+        }
+        for (int k = upOff[c]; k < upOff[c + 1]; ++k) {
+            upCol[k] = up[k].first;
+            upSrc[k] = (up[k].second << 1) | (m->own[up[k].second] == c ? 0 : 1);
+        }
+    }
+    std::vector<int> permF, permB, offF, offB;
+    levelOrder(n, l, u, offF, permF, offB, permB);
+    hipStream_t st = m->ctx->stream;
+    auto F = std::make_unique<SweepPlanDev>(), B = std::make_unique<SweepPlanDev>();
+    F->build(n, offF, permF, lowOff, lowCol, lowSrc, sweepChunks(n, offF, permF, false), 0, false, st);
+    B->build(n, offB, permB, upOff, upCol, upSrc, sweepChunks(n, offB, permB, false), 0, false, st);
+    m->diluB = std::move(B);
+    m->diluF = std::move(F);
 }
 
-// DIC/DILU factor of the matrix (LinearSolver.cpp:66-78) on the forward levels.
+// The mailbox of `sweeps` sweeps over n cells (several chunks) and the tickets of up to
+// SWEEP_TICKETS launches made ready in stream order.
+template <class T> T* sweepMailbox(vol_context c, hipStream_t st, int n, int sweeps, const int* done) {
+    const size_t m = size_t(n) * sweeps;
+    c->sweepMail.alloc((m * sizeof(T) + sizeof(double) - 1) / sizeof(double));
+    T* mail = reinterpret_cast<T*>(c->sweepMail.p);
+    launch_sweep_prepare<T>(st, m, mail, c->sweepFault.p + 1, done);
+    return mail;
+}
+
+// DIC/DILU factor of the matrix (LinearSolver.cpp:66-78) and the substitutions' entries.
 void buildDilu(vol_matrix A) {
     vol_mesh m = A->mesh;
-    buildSweep(m);
-    hipStream_t st = m->ctx->stream;
-    const size_t n = m->n, nf = m->nf;
-    A->dluD.alloc(n);
-    A->dluR.alloc(n);
-    A->dluPf.alloc(std::max<size_t>(nf, 1));
-    A->dluPb.alloc(std::max<size_t>(nf, 1));
-    launch_dilu_factor(st, m->sweepView(), m->ordF.view(), A->diag.p, A->upper.p,
-                       A->symmetric ? A->upper.p : A->lower.p, A->dluD.p, A->dluR.p, A->dluPf.p, A->dluPb.p);
-    A->dluEf.alloc(std::max<size_t>(m->diluF.nEntries, 1));
-    A->dluEb.alloc(std::max<size_t>(m->diluB.nEntries, 1));
-    launch_gather_entries<double>(st, m->diluF.nEntries, m->diluF.src.p, A->dluPf.p, A->dluEf.p);
-    launch_gather_entries<double>(st, m->diluB.nEntries, m->diluB.src.p, A->dluPb.p, A->dluEb.p);
+    buildDiluPlans(m);
+    vol_context c = m->ctx;
+    hipStream_t st = c->stream;
+    const SweepPlanDev &F = *m->diluF, &B = *m->diluB;
+    A->dluD.alloc(m->n);
+    A->dluR.alloc(m->n);
+    A->dluEf.alloc(F.nEntries);
+    A->dluEb.alloc(B.nEntries);
+    const double* lower = A->symmetric ? A->upper.p : A->lower.p;
+    launch_dilu_entries(st, F.v, F.src.p, A->upper.p, lower, nullptr, A->dluEf.p);
+    SweepArgs<double> a;
+    a.coef = A->dluEf.p;
+    a.diag = A->diag.p;
+    a.x = A->dluD.p;
+    if (F.v.nChunks > 1) {
+        a.mail = sweepMailbox<double>(c, st, m->n, 1, nullptr);
+        a.ticket = c->sweepFault.p + 1;
+        a.fault = c->sweepFault.p;
+    }
+    launch_sweep<double>(st, SW_FAC, false, F.v, a, 1, nullptr);
+    VecArgs v;
+    v.n = m->n;
+    v.a = A->dluD.p;
+    v.w = A->dluR.p;
+    launch_vec(st, V_RECIP, v, false, c->red);
+    launch_dilu_entries(st, F.v, F.src.p, A->upper.p, lower, A->dluR.p, A->dluEf.p);
+    launch_dilu_entries(st, B.v, B.src.p, A->upper.p, lower, A->dluR.p, A->dluEb.p);
     A->diluReady = true;
     A->dilu32Ready = false;
-}
-
-// Gauss–Seidel coefficients of the matrix in the LevelEll layouts: level 0, and the
-// coarse GAMG levels when the GAMG smoother needs them.
-void buildGs(vol_matrix A, bool gamgLevels) {
-    vol_mesh m = A->mesh;
-    buildSweep(m);
-    hipStream_t st = m->ctx->stream;
-    if (!A->gsReady) {
-        A->gsCF.alloc(std::max<size_t>(m->gsF.nEntries, 1));
-        A->gsCB.alloc(std::max<size_t>(m->gsB.nEntries, 1));
-        launch_gather_entries<double>(st, m->gsF.nEntries, m->gsF.src.p, A->coef.p, A->gsCF.p);
-        launch_gather_entries<double>(st, m->gsB.nEntries, m->gsB.src.p, A->coef.p, A->gsCB.p);
-        A->gsReady = true;
-        A->gs32Ready = false;
-    }
-    if (gamgLevels && !A->gsLevReady) {
-        const int nL = int(m->lv.size());
-        for (int k = 1; k + 1 < nL; ++k) {
-            const vol_mesh_s::LevelOrder& o = *m->gsLev[k];
-            MatLevel& M = *A->L[k];
-            M.gsCF.alloc(std::max<size_t>(o.F.nEntries, 1));
-            M.gsCB.alloc(std::max<size_t>(o.B.nEntries, 1));
-            launch_gather_entries<double>(st, o.F.nEntries, o.F.src.p, M.coef.p, M.gsCF.p);
-            launch_gather_entries<double>(st, o.B.nEntries, o.B.src.p, M.coef.p, M.gsCB.p);
-        }
-        A->gsLevReady = true;
-        A->gs32Ready = false;
-    }
 }
 
 // k consecutive Gauss–Seidel sweeps over a graph (edges l[e] < u[e]) as one level
@@ -777,10 +690,12 @@ void multiSweepOrder(int n, const std::vector<int>& l, const std::vector<int>& u
         for (int s = 0; s < k; ++s) perm[fill[lev[size_t(s) * n + c]]++] = c;
 }
 
-// The k-sweep schedule of GAMG level lvl (0: the mesh) and direction, built on first use.
-const LevelEllDev& gsMultiEll(vol_mesh m, int lvl, bool backward, int k) {
+// The plan of Gauss–Seidel sweeps of GAMG level lvl (0: the mesh) in one direction, built
+// on first use: with one chunk the k sweeps as one pipelined schedule, else a single sweep
+// (k = 1).
+const SweepPlanDev& gsPlan(vol_mesh m, int lvl, bool backward, int k) {
     std::lock_guard<std::mutex> guard(m->sweepMu);
-    auto& slot = m->gsMulti[{lvl, backward ? 1 : 0, k}];
+    auto& slot = m->gsPlans[{lvl, backward ? 1 : 0, k}];
     if (slot) return *slot;
     std::vector<int> l, u;
     int n;
@@ -800,48 +715,34 @@ const LevelEllDev& gsMultiEll(vol_mesh m, int lvl, bool backward, int k) {
     std::vector<int> off, perm, ro, rc, rs;
     multiSweepOrder(n, l, u, backward, k, off, perm);
     sellRows(lvl == 0 ? m->sell : m->lv[lvl]->sell, ro, rc, rs);
-    auto e = std::make_unique<LevelEllDev>();
-    e->build(off, perm, ro, rc, rs, m->ctx->stream);
+    int width = 0;
+    for (int c = 0; c < n; ++c) width = std::max(width, ro[c + 1] - ro[c]);
+    auto e = std::make_unique<SweepPlanDev>();
+    e->build(n, off, perm, ro, rc, rs, sweepChunks(n, off, perm, width > 8), backward ? -1 : 1, true, m->ctx->stream);
     slot = std::move(e);
     return *slot;
 }
 
-// The matrix's coefficients in that schedule's layout (level coefficients gathered by the
-// schedule's entry sources), built after each change of the matrix.
-const double* gsMultiCoef(vol_matrix A, int lvl, bool backward, int k) {
-    const LevelEllDev& E = gsMultiEll(A->mesh, lvl, backward, k);
-    auto& buf = A->gsMultiCoef[{lvl, backward ? 1 : 0, k}];
-    if (!buf.p) {
-        buf.alloc(std::max<size_t>(E.nEntries, 1));
-        launch_gather_entries<double>(A->mesh->ctx->stream, E.nEntries, E.src.p,
-                                      lvl == 0 ? A->coef.p : A->L[lvl]->coef.p, buf.p);
-    }
-    return buf.p;
-}
-
-void buildGs32(vol_matrix A) {
-    vol_mesh m = A->mesh;
-    hipStream_t st = m->ctx->stream;
-    A->gsCF32.alloc(std::max<size_t>(m->gsF.nEntries, 1));
-    A->gsCB32.alloc(std::max<size_t>(m->gsB.nEntries, 1));
-    launch_gather_entries<float>(st, m->gsF.nEntries, m->gsF.src.p, A->coef32.p, A->gsCF32.p);
-    launch_gather_entries<float>(st, m->gsB.nEntries, m->gsB.src.p, A->coef32.p, A->gsCB32.p);
-    const int nL = int(m->lv.size());
-    for (int k = 1; k + 1 < nL; ++k) {
-        const vol_mesh_s::LevelOrder& o = *m->gsLev[k];
-        MatLevel& M = *A->L[k];
-        M.gsCF32.alloc(std::max<size_t>(o.F.nEntries, 1));
-        M.gsCB32.alloc(std::max<size_t>(o.B.nEntries, 1));
-        launch_gather_entries<float>(st, o.F.nEntries, o.F.src.p, M.coef32.p, M.gsCF32.p);
-        launch_gather_entries<float>(st, o.B.nEntries, o.B.src.p, M.coef32.p, M.gsCB32.p);
-    }
-    A->gs32Ready = true;
+// The matrix's coefficients in that plan's layout, gathered after each change of the matrix.
+template <class T> const T* gsPlanCoef(vol_matrix A, const SweepPlanDev& E, int lvl, bool backward, int k) {
+    const std::tuple<int, int, int> key{lvl, backward ? 1 : 0, k};
+    auto gather = [&](DevBuf<T>& buf, const T* from) {
+        if (!buf.p) {
+            buf.alloc(E.nEntries);
+            launch_gather_entries<T>(A->mesh->ctx->stream, E.nEntries, E.src.p, from, buf.p);
+        }
+        return buf.p;
+    };
+    if constexpr (std::is_same_v<T, float>)
+        return gather(A->gsCoef32[key], lvl == 0 ? A->coef32.p : A->L[lvl]->coef32.p);
+    else
+        return gather(A->gsCoef[key], lvl == 0 ? A->coef.p : A->L[lvl]->coef.p);
 }
 
 void buildDilu32(vol_matrix A) {
     vol_mesh m = A->mesh;
     hipStream_t st = m->ctx->stream;
-    const size_t n = m->n, ef = std::max<size_t>(m->diluF.nEntries, 1), eb = std::max<size_t>(m->diluB.nEntries, 1);
+    const size_t n = m->n, ef = m->diluF->nEntries, eb = m->diluB->nEntries;
     A->dluR32.alloc(n);
     A->dluEf32.alloc(ef);
     A->dluEb32.alloc(eb);
@@ -931,10 +832,8 @@ void matrixFinish(vol_matrix A) {
     A->mixedReady = false;
     A->diluReady = false;
     A->dilu32Ready = false;
-    A->gsReady = false;
-    A->gsLevReady = false;
-    A->gs32Ready = false;
-    A->gsMultiCoef.clear();
+    A->gsCoef.clear();
+    A->gsCoef32.clear();
     A->set = true;
 }
 
@@ -1560,31 +1459,30 @@ bool vcycle(const Ctx& C, vol_matrix A, const Plan& P, int l, const T* r, T* xou
     return push != nullptr;
 }
 
-// After a solve with sync-free sweeps (stream synchronised): a wait that ran past its
-// limit voids the results.
-void checkSweepFault(vol_context c, hipStream_t st) {
-    int f = 0;
-    HIPCHECK(hipMemcpyAsync(&f, c->sweepFault.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHECK(hipStreamSynchronize(st));
-    if (f) {
-        HIPCHECK(hipMemsetAsync(c->sweepFault.p, 0, sizeof(int), st));
-        HIPCHECK(hipStreamSynchronize(st));
-        throw VolError(VOL_ERR_HIP, "sync-free sweep: a wait for a neighbour's value timed out");
-    }
-}
-
-// `sweeps` sync-free Gauss–Seidel sweeps of x (in place from the caller's view):
-// alternately x → tmp and tmp → x, and a copy back after an odd count.
+// k Gauss–Seidel sweeps of x on a level; fromZero: x is taken as zero.
 template <class T>
-void gsSweepsFree(const Ctx& C, const LevelEll& E, bool backward, const T* coef, const T* diag, const T* b, T* x, T* tmp,
-                  int n, int sweeps) {
-    T* src = x;
-    T* dst = tmp;
-    for (int s = 0; s < sweeps; ++s) {
-        launch_gs_sweep_free<T>(C.st, E, backward, coef, diag, b, src, dst, C.c->sweepFault.p, C.done);
-        std::swap(src, dst);
+void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T* diag, const T* b, T* x, int n,
+              bool fromZero) {
+    const bool one = n <= SWEEP_ONE_CELLS;
+    const SweepPlanDev& E = gsPlan(A->mesh, lvl, backward, one ? k : 1);
+    SweepArgs<T> a;
+    a.coef = gsPlanCoef<T>(A, E, lvl, backward, one ? k : 1);
+    a.b = b;
+    a.diag = diag;
+    a.x = x;
+    a.zero = fromZero;
+    if (one) {
+        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, 1, C.done);
+        return;
     }
-    if (src != x) vec<T>(C, V_COPY, n, false, src, nullptr, nullptr, nullptr, x);
+    a.ticket = C.c->sweepFault.p + 1;
+    a.fault = C.c->sweepFault.p;
+    for (int s = 0; s < k; s += SWEEP_MAX_SWEEPS) {
+        const int q = std::min(k - s, SWEEP_MAX_SWEEPS);
+        a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
+        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, q, C.done);
+        a.zero = false;
+    }
 }
 
 // One V-cycle at level l with the reference's Gauss–Seidel smoother (GAMG.cpp:403-443):
@@ -1601,47 +1499,14 @@ template <class T> void vcycleGS(const Ctx& C, vol_matrix A, const Plan& P, int 
     const SellView V = l == 0 ? m->sell.view() : D.sell.view();
     const LevelPtrs<T> L = levelPtrs(A, l, (T*)nullptr);
     const int n = l == 0 ? m->n : D.n;
-    const LevelEll sF = l == 0 ? m->gsF.view() : m->gsLev[l]->F.view();
-    const LevelEll sB = l == 0 ? m->gsB.view() : m->gsLev[l]->B.view();
-    const T *cF, *cB;
-    if constexpr (std::is_same_v<T, float>) {
-        cF = l == 0 ? A->gsCF32.p : A->L[l]->gsCF32.p;
-        cB = l == 0 ? A->gsCB32.p : A->L[l]->gsCB32.p;
-    } else {
-        cF = l == 0 ? A->gsCF.p : A->L[l]->gsCF.p;
-        cB = l == 0 ? A->gsCB.p : A->L[l]->gsCB.p;
-    }
-    launch_fill_zero<T>(C.st, n, xout, C.done);
-    if (C.c->freeSweeps) {  // sync-free sweeps alternating between xout and bufB
-        gsSweepsFree<T>(C, sF, false, cF, L.diag, r, xout, L.bufB, n, P.nPre);
-    } else if constexpr (std::is_same_v<T, double>) {  // the sweeps as one pipelined schedule
-        if (P.nPre > 1) {
-            launch_gs_sweep<T>(C.st, gsMultiEll(m, l, false, P.nPre).view(), gsMultiCoef(A, l, false, P.nPre),
-                               L.diag, r, xout, C.done);
-        } else {
-            for (int s = 0; s < P.nPre; ++s) launch_gs_sweep<T>(C.st, sF, cF, L.diag, r, xout, C.done);
-        }
-    } else {
-        for (int s = 0; s < P.nPre; ++s) launch_gs_sweep<T>(C.st, sF, cF, L.diag, r, xout, C.done);
-    }
+    gsSweeps<T>(C, A, l, false, P.nPre, L.diag, r, xout, n, true);
     sell<T>(C, OP_RESID, XL_PLAIN, V, L.coef, L.diag, xout, r, L.bufA, P.omega, nullptr, nullptr, nullptr, nullptr,
             nullptr, L.rD);
     const LevelPtrs<T> LC = levelPtrs(A, l + 1, (T*)nullptr);
     restrictLevel(C, m->lv[l + 1]->n, D, L.bufA, LC.r);
     vcycleGS<T>(C, A, P, l + 1, LC.r, LC.x);
     launch_prolong<T>(C.st, n, D.agg.p, LC.x, xout, C.done);
-    if (C.c->freeSweeps) {
-        gsSweepsFree<T>(C, sB, true, cB, L.diag, r, xout, L.bufB, n, P.nPost);
-    } else if constexpr (std::is_same_v<T, double>) {
-        if (P.nPost > 1) {
-            launch_gs_sweep<T>(C.st, gsMultiEll(m, l, true, P.nPost).view(), gsMultiCoef(A, l, true, P.nPost),
-                               L.diag, r, xout, C.done);
-        } else {
-            for (int s = 0; s < P.nPost; ++s) launch_gs_sweep<T>(C.st, sB, cB, L.diag, r, xout, C.done);
-        }
-    } else {
-        for (int s = 0; s < P.nPost; ++s) launch_gs_sweep<T>(C.st, sB, cB, L.diag, r, xout, C.done);
-    }
+    gsSweeps<T>(C, A, l, true, P.nPost, L.diag, r, xout, n, false);
 }
 
 template <class T>
@@ -1662,20 +1527,24 @@ void precondApply(const Ctx& C, vol_matrix A, const Plan& P, const T* r, T* w, i
             ef = A->dluEf.p;
             eb = A->dluEb.p;
         }
-        if (C.c->freeSweeps) {
-            T* tmp;
-            if constexpr (std::is_same_v<T, float>) {
-                A->diluTmp32.alloc(n);
-                tmp = A->diluTmp32.p;
-            } else {
-                A->diluTmp.alloc(n);
-                tmp = A->diluTmp.p;
-            }
-            launch_dilu_apply_free<T>(C.st, m->diluF.view(), m->diluB.view(), rD, ef, eb, r, tmp, w,
-                                      C.c->sweepFault.p, C.done);
-        } else {
-            launch_dilu_apply<T>(C.st, m->diluF.view(), m->diluB.view(), rD, ef, eb, r, w, C.done);
+        const SweepPlan &F = m->diluF->v, &B = m->diluB->v;
+        SweepArgs<T> a;
+        a.coef = ef;
+        a.rD = rD;
+        a.b = r;
+        a.x = w;
+        if (F.nChunks == 1) {
+            launch_dilu_one<T>(C.st, F, B, a, eb, C.done);
+            return;
         }
+        a.mail = sweepMailbox<T>(C.c, C.st, n, 2, C.done);
+        a.ticket = C.c->sweepFault.p + 1;
+        a.fault = C.c->sweepFault.p;
+        launch_sweep<T>(C.st, SW_FWD, false, F, a, 1, C.done);
+        a.coef = eb;
+        a.mail += n;
+        ++a.ticket;
+        launch_sweep<T>(C.st, SW_BWD, true, B, a, 1, C.done);
     } else
         vec<T>(C, V_SCALE, n, false, r, nullptr, nullptr, nullptr, w, nullptr, nullptr,
                P.precond == "diagonal" ? level0(A, (T*)nullptr).rD : nullptr);
@@ -1885,16 +1754,12 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
     readScalars(c, C.S, hs);
     if (!hs.done) {
         if (P.precond == "GAMG" && !A->gamgReady) buildGamgCoeffs(A);
-        if (P.precond == "GAMG" && P.gamgGS) buildGsLevels(m);
-        if ((P.precond == "GAMG" && P.gamgGS) || isGS) buildGs(A, P.precond == "GAMG" && P.gamgGS);
         const bool dilu = (isPCG || isBi) && (P.precond == "DIC" || P.precond == "DILU");
         if (dilu && !A->diluReady) buildDilu(A);
         if (dilu && mixed && !A->dilu32Ready) buildDilu32(A);
-        if (isGS) buildSweep(m);
         const int maxLoops = std::max(ct.maxIter, 1) + 2;
         if (mixed) {
             if (!A->mixedReady || (P.precond == "GAMG" && !A->mixedGamg)) buildMixed(A, P.precond == "GAMG");
-            if (P.precond == "GAMG" && P.gamgGS && !A->gs32Ready) buildGs32(A);
             for (DevBuf<float>* v : {&A->ir, &A->iw, &A->ip, &A->iq, &A->ie}) v->alloc(n);
             if (isBi)
                 for (DevBuf<float>* v : {&A->ir0, &A->iy, &A->iAy, &A->is, &A->iz, &A->it}) v->alloc(n);
@@ -1966,23 +1831,13 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
             A->vw.alloc(n);
             const bool sym = P.solver == "symGaussSeidel";
             runLoop(c, C, maxLoops, [&] {
+                if (isGS && !sym)
+                    gsSweeps<double>(C, A, 0, false, ct.nSweeps, A->diag.p, b, x, n, false);
                 for (int sw = 0; sw < ct.nSweeps; ++sw) {
-                    if (isGS && c->freeSweeps) {  // x → vw (forward), then vw → x (backward) or a copy
-                        int* f = c->sweepFault.p;
-                        launch_gs_sweep_free<double>(st, m->gsF.view(), false, A->gsCF.p, A->diag.p, b, x, A->vw.p, f,
-                                                     C.done);
-                        if (sym)
-                            launch_gs_sweep_free<double>(st, m->gsB.view(), true, A->gsCB.p, A->diag.p, b, A->vw.p, x,
-                                                         f, C.done);
-                        else
-                            vec<double>(C, V_COPY, n, false, A->vw.p, nullptr, nullptr, nullptr, x);
-                        continue;
-                    }
-                    if (isGS) {
-                        launch_gs_sweep<double>(st, m->gsF.view(), A->gsCF.p, A->diag.p, b, x, C.done);
-                        if (sym) launch_gs_sweep<double>(st, m->gsB.view(), A->gsCB.p, A->diag.p, b, x, C.done);
-                        continue;
-                    }
+                    if (isGS && sym)
+                        for (bool backward : {false, true})
+                            gsSweeps<double>(C, A, 0, backward, 1, A->diag.p, b, x, n, false);
+                    if (isGS) continue;
                     sell<double>(C, OP_JACREF, XL_PLAIN, V, A->coef.p, A->diag.p, x, b, A->vw.p);
                     vec<double>(C, V_COPY, n, ex, A->vw.p, nullptr, nullptr, nullptr, x);
                 }
@@ -1991,10 +1846,16 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
                 fin(C, FIN_JAC_NORM, 1, ex, nparts, C.hostOut);
             });
         }
+        const bool chunked = n > SWEEP_ONE_CELLS && (isGS || dilu || (P.precond == "GAMG" && P.gamgGS));
+        if (chunked)
+            HIPCHECK(hipMemcpyAsync(c->hostFault, c->sweepFault.p, sizeof(int), hipMemcpyDeviceToHost, st));
         readScalars(c, C.S, hs);
+        if (chunked && *c->hostFault) {
+            HIPCHECK(hipMemsetAsync(c->sweepFault.p, 0, sizeof(int), st));
+            throw VolError(VOL_ERR_HIP, "triangular sweep: a wait for a neighbour's value timed out");
+        }
         if (!hs.done) throw VolError(VOL_ERR_HIP, "solver loop did not terminate");
     }
-    if (c->freeSweeps && (isGS || P.precond == "DIC" || P.precond == "DILU" || P.gamgGS)) checkSweepFault(c, st);
     collectTiming(c);
     perf.initialResidual = hs.initialResidual;
     perf.finalResidual = hs.finalResidual;
@@ -2201,11 +2062,11 @@ int vol_context_create(int device, vol_context* out) {
     if (const char* e = std::getenv("VOLUMA_LAST_BLOCK_FIN")) c->lastBlockFin = std::string(e) == "1";
     if (const char* e = std::getenv("VOLUMA_FUSED_SELL_DIRECT")) c->fusedSellDirect = std::string(e) == "1";
     if (const char* e = std::getenv("VOLUMA_FUSED_SELL_MAX")) c->fusedSellMax = std::atoi(e);
-    if (const char* e = std::getenv("VOLUMA_SWEEP")) c->freeSweeps = std::string(e) == "free";
-    c->sweepFault.alloc(2);  // fault flag, work counter
-    HIPCHECK(hipMemsetAsync(c->sweepFault.p, 0, 2 * sizeof(int), c->stream));
+    c->sweepFault.alloc(1 + SWEEP_TICKETS);
+    HIPCHECK(hipMemsetAsync(c->sweepFault.p, 0, (1 + SWEEP_TICKETS) * sizeof(int), c->stream));
     c->scal.alloc(2);
-    HIPCHECK(hipHostMalloc((void**)&c->hostScal, 2 * sizeof(DevScalars), hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void**)&c->hostScal, 2 * sizeof(DevScalars) + sizeof(int), hipHostMallocDefault));
+    c->hostFault = reinterpret_cast<int*>(c->hostScal + 2);
     c->ensureScratch(RED_BLOCKS);
     for (hipEvent_t& e : c->loopEv) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     registerScratch(device);

@@ -64,244 +64,41 @@ template <class T> struct DevBuf {
     }
 };
 
-// One level order of the triangular sweeps in host and device form (LevelSched view):
-// offsets and permutation, and the launch groups — runs of consecutive levels of at most
-// SWEEP_RUN_MAX cells (one workgroup) and single larger levels (a grid each).
-struct LevelOrderDev {
-    std::vector<int> off, grp;
-    std::vector<char> run;
-    DevBuf<int> perm, offD;
-    void build(const std::vector<int>& offH, const std::vector<int>& permH, hipStream_t st) {
-        off = offH;
-        const int nl = int(off.size()) - 1;
-        grp.clear();
-        run.clear();
-        for (int L = 0; L < nl;) {
-            grp.push_back(L);
-            if (off[L + 1] - off[L] > SWEEP_RUN_MAX) {
-                run.push_back(0);
-                ++L;
-            } else {
-                run.push_back(1);
-                while (L < nl && off[L + 1] - off[L] <= SWEEP_RUN_MAX) ++L;
-            }
-        }
-        grp.push_back(std::max(nl, 0));
-        perm.upload(permH, st);
-        offD.upload(off, st);
-    }
-    LevelSched view() const {
-        LevelSched v;
-        v.perm = perm.p;
-        v.offD = offD.p;
-        v.offH = off.data();
-        v.nLev = int(off.size()) - 1;
-        v.grpH = grp.data();
-        v.grpRunH = run.data();
-        v.nGrp = int(grp.size()) - 1;
-        return v;
-    }
-};
-
-// Level-ordered ELL rows of a triangular sweep (LevelEll view). Rows are given as a
-// CSR by cell (rowOff, rowCol, rowSrc: neighbour and coefficient source index of each
-// entry, in the sweep's order); src keeps the source index of every entry (−1 padding)
-// for the per-matrix coefficient gather.
-struct LevelEllDev {
-    std::vector<int> off, width, base, grp, runOff, runCnt;
-    std::vector<char> kind;
-    DevBuf<int> cell, slot, runCells, col, src, offD, widthD, baseD;
-    DevBuf<int2> waves;  // sync-free sweeps: (level, first row) per wavefront
-    DevBuf<int> runBaseD;  // per level: first runCells entry of its run (−1: not in a run)
-    int nWaves = 0;
+// A triangular sweep's plan on the device; src keeps the source of every entry for the
+// per-matrix coefficients.
+struct SweepPlanDev {
+    DevBuf<int> chunkOff, stepOff, haloOff, halo, cell, col, col2, src;
+    DevBuf<SweepStep> steps;
     size_t nEntries = 0;
-    void build(const std::vector<int>& levOff, const std::vector<int>& perm, const std::vector<int>& rowOff,
-               const std::vector<int>& rowCol, const std::vector<int>& rowSrc, hipStream_t st) {
-        off = levOff;
-        const int nl = int(off.size()) - 1;
-        width.assign(std::max(nl, 0), 0);
-        base.assign(std::max(nl, 0), 0);
-        size_t total = 0;
-        for (int L = 0; L < nl; ++L) {
-            if (off[L + 1] <= off[L]) throw VolError(VOL_ERR_INVALID_ARGUMENT, "empty sweep level");
-            int w = 0;
-            for (int i = off[L]; i < off[L + 1]; ++i) w = std::max(w, rowOff[perm[i] + 1] - rowOff[perm[i]]);
-            width[L] = w;
-            base[L] = int(total);
-            total += size_t(w) * size_t(off[L + 1] - off[L]);
-        }
-        if (total >= (size_t(1) << 31)) throw VolError(VOL_ERR_INVALID_ARGUMENT, "sweep rows exceed 2^31 entries");
-        nEntries = total;
-        {  // wavefronts of one level each, in level order (the sync-free sweeps' work order)
-            std::vector<int2> wv;
-            for (int L = 0; L < nl; ++L)
-                for (int t0 = 0; t0 < off[L + 1] - off[L]; t0 += WAVE) wv.push_back(make_int2(L, t0));
-            nWaves = int(wv.size());
-            waves.upload(wv, st);
-        }
-        // at least one entry, so a sweep's stand-in reads of entry 0 stay in bounds
-        std::vector<int> ec(std::max<size_t>(total, 1), -1), es(total, -1);
-        for (int L = 0; L < nl; ++L) {
-            const int size = off[L + 1] - off[L];
-            for (int t = 0; t < size; ++t) {
-                const int c = perm[off[L] + t];
-                for (int k = 0; k < rowOff[c + 1] - rowOff[c]; ++k) {
-                    const size_t e = size_t(base[L]) + size_t(k) * size + t;
-                    ec[e] = rowCol[rowOff[c] + k];
-                    es[e] = rowSrc[rowOff[c] + k];
-                }
-            }
-        }
-        grp.clear();
-        kind.clear();
-        auto kindOf = [&](int L) {
-            const int size = off[L + 1] - off[L];
-            return size <= 256 ? ELL_RUN256 : size <= 512 ? ELL_RUN512 : size <= 1024 ? ELL_RUN1024 : ELL_GRID;
-        };
-        for (int L = 0; L < nl;) {
-            if (kindOf(L) == ELL_GRID) {
-                grp.push_back(L);
-                kind.push_back(char(ELL_GRID));
-                ++L;
-                continue;
-            }
-            // a stretch of run levels [L, R): segments of one class, a segment of fewer
-            // than 16 levels merged into a neighbour (the merged run takes the larger
-            // class), each segment cut into runs of at most ELL_RUN_LEVELS levels
-            int R = L;
-            while (R < nl && kindOf(R) != ELL_GRID) ++R;
-            std::vector<int> segS, segK;
-            for (int i = L; i < R; ++i)
-                if (segK.empty() || segK.back() != kindOf(i)) {
-                    segS.push_back(i);
-                    segK.push_back(kindOf(i));
-                }
-            segS.push_back(R);
-            for (bool merged = true; merged && segK.size() > 1;) {
-                merged = false;
-                for (size_t g = 0; g < segK.size(); ++g) {
-                    if (segS[g + 1] - segS[g] >= 16) continue;
-                    const size_t a = g > 0 ? g - 1 : 0;  // merge segments a and a + 1
-                    segK[a] = std::max(segK[a], segK[a + 1]);
-                    segK.erase(segK.begin() + long(a) + 1);
-                    segS.erase(segS.begin() + long(a) + 1);
-                    merged = true;
-                    break;
-                }
-            }
-            for (size_t g = 0; g < segK.size(); ++g)
-                for (int s0 = segS[g]; s0 < segS[g + 1]; s0 += ELL_RUN_LEVELS) {
-                    grp.push_back(s0);
-                    kind.push_back(char(segK[g]));
-                }
-            L = R;
-        }
-        grp.push_back(std::max(nl, 0));
-        // LDS-resident runs: a run takes consecutive levels while the cells its rows
-        // write or read fit RUN_LDS_CELLS slots (a level that alone does not fit is swept
-        // as a grid level); slots in first-appearance order (a row's cell, then its
-        // neighbours), run rows' entries and own cells re-coded as slots
-        std::vector<int> slotv(std::max<size_t>(perm.size(), 1), 0), cells;
-        std::vector<int> runBase(std::max(nl, 1), -1);  // entries of run levels hold slots
-        {
-            std::vector<int> g2, ro, rn;
-            std::vector<char> k2;
-            std::unordered_map<int, int> map, seen;
-            std::vector<int> fresh;
-            auto close = [&](int L, char k, int start, int cnt) {
-                g2.push_back(L);
-                k2.push_back(k);
-                ro.push_back(start);
-                rn.push_back(cnt);
-            };
-            for (size_t g = 0; g + 1 < grp.size(); ++g) {
-                const int A = grp[g], B = grp[g + 1];
-                if (kind[g] == char(ELL_GRID)) {
-                    close(A, kind[g], int(cells.size()), 0);
-                    continue;
-                }
-                for (int L = A; L < B;) {
-                    map.clear();
-                    const int start = int(cells.size());
-                    int R = L;
-                    for (; R < B; ++R) {
-                        fresh.clear();
-                        seen.clear();
-                        for (int i = off[R]; i < off[R + 1]; ++i) {
-                            const int c = perm[i];
-                            auto take = [&](int q) {
-                                if (!map.count(q) && seen.emplace(q, 0).second) fresh.push_back(q);
-                            };
-                            take(c);
-                            for (int k = rowOff[c]; k < rowOff[c + 1]; ++k) take(rowCol[k]);
-                        }
-                        if (map.size() + fresh.size() > size_t(RUN_LDS_CELLS)) break;
-                        for (int q : fresh) {
-                            map.emplace(q, int(cells.size()) - start);
-                            cells.push_back(q);
-                        }
-                    }
-                    if (R == L) {  // one level alone exceeds the slots
-                        close(L, char(ELL_GRID), start, 0);
-                        ++L;
-                        continue;
-                    }
-                    close(L, kind[g], start, int(cells.size()) - start);
-                    for (int Lq = L; Lq < R; ++Lq) {
-                        const int size = off[Lq + 1] - off[Lq];
-                        runBase[Lq] = start;
-                        for (int t = 0; t < size; ++t) {
-                            const int c = perm[off[Lq] + t];
-                            slotv[off[Lq] + t] = map.at(c);
-                            for (int k = 0; k < rowOff[c + 1] - rowOff[c]; ++k) {
-                                const size_t e = size_t(base[Lq]) + size_t(k) * size + t;
-                                ec[e] = map.at(ec[e]);
-                            }
-                        }
-                    }
-                    L = R;
-                }
-            }
-            g2.push_back(std::max(nl, 0));
-            grp = std::move(g2);
-            kind = std::move(k2);
-            runOff = std::move(ro);
-            runCnt = std::move(rn);
-        }
-        cell.upload(perm, st);
-        slot.upload(slotv, st);
-        if (cells.empty()) cells.push_back(0);
-        runCells.upload(cells, st);
-        runBaseD.upload(runBase, st);
-        col.upload(ec, st);
-        src.upload(es, st);
-        offD.upload(off, st);
-        widthD.upload(width, st);
-        baseD.upload(base, st);
-        HIPCHECK(hipStreamSynchronize(st));
-    }
-    LevelEll view() const {
-        LevelEll v;
+    SweepPlan v;  // valid while this lives
+    void build(int n, const std::vector<int>& off, const std::vector<int>& perm, const std::vector<int>& rowOff,
+               const std::vector<int>& rowCol, const std::vector<int>& rowSrc, int nChunks, int oldSide, bool again,
+               hipStream_t st) {
+        const SweepPlanHost H = buildSweepPlan(n, off, perm, rowOff, rowCol, rowSrc, nChunks, oldSide, again);
+        chunkOff.upload(H.chunkOff, st);
+        stepOff.upload(H.stepOff, st);
+        cell.upload(H.cell, st);
+        steps.upload(H.steps, st);
+        col.upload(H.col, st);
+        if (!H.col2.empty()) col2.upload(H.col2, st);
+        v.col2 = col2.p;
+        src.upload(H.src, st);
+        nEntries = H.col.size();
+        v.chunkOff = chunkOff.p;
+        v.stepOff = stepOff.p;
+        v.steps = steps.p;
         v.cell = cell.p;
-        v.slot = slot.p;
-        v.runCells = runCells.p;
-        v.runOffH = runOff.data();
-        v.runCntH = runCnt.data();
         v.col = col.p;
-        v.offD = offD.p;
-        v.widthD = widthD.p;
-        v.baseD = baseD.p;
-        v.offH = off.data();
-        v.widthH = width.data();
-        v.baseH = base.data();
-        v.nLev = int(off.size()) - 1;
-        v.grpH = grp.data();
-        v.grpKindH = kind.data();
-        v.nGrp = int(grp.size()) - 1;
-        v.waves = waves.p;
-        v.nWaves = nWaves;
-        v.runBaseD = runBaseD.p;
-        return v;
+        v.n = n;
+        v.nChunks = H.nChunks;
+        v.nSteps = int(H.steps.size());
+        haloOff.upload(H.haloOff, st);
+        halo.upload(H.halo, st);
+        v.haloOff = haloOff.p;
+        v.halo = halo.p;
+        v.maxSlots = H.maxSlots;
+        v.maxWidth = H.maxWidth;
+        HIPCHECK(hipStreamSynchronize(st));
     }
 };
 
@@ -960,12 +757,11 @@ struct vol_context_s {
     // SELL levels also in the packed SELL form (SellView::colS): the coarse levels of a
     // mesh, and every level of a batch (VOLUMA_SELL_PAIRS=0: slot-major only)
     bool sellPairs = true;
-    // triangular sweeps (Gauss–Seidel, DIC/DILU substitutions) in their sync-free form,
-    // one launch per sweep (VOLUMA_SWEEP=free; the same bits; measured slower than the
-    // default level-scheduled launches); sweepFault: [0] set by a sync-free wait that ran
-    // past its limit, [1] the sync-free sweeps' work counter
-    bool freeSweeps = false;
+    // triangular sweeps over several chunks: [0] set by a wait that ran past its limit,
+    // then the chunk tickets; pinned copy of the flag read with a solve's scalars
     DevBuf<int> sweepFault;
+    int* hostFault = nullptr;
+    DevBuf<double> sweepMail;  // their mailbox
     RedScratch red;
     DevBuf<double> part, result;
     DevBuf<long long> xpart;

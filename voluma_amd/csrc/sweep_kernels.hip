@@ -1,30 +1,39 @@
-// Level-scheduled triangular sweeps: the DIC/DILU preconditioner (factor, forward and
-// backward substitution, LinearSolver.cpp:56-105), the Gauss–Seidel solver sweeps
+// Triangular sweeps: the DIC/DILU preconditioner (factor, forward and backward
+// substitution, LinearSolver.cpp:56-105), the Gauss–Seidel solver sweeps
 // (LinearSolver.cpp:238-264) and the Gauss–Seidel GAMG smoother (GAMG.cpp:363-384).
 //
 // The reference runs these loops one cell (or one face) at a time. A cell's update reads
-// only neighbours with a smaller index (forward) or a larger one (backward), so cells
-// are grouped into levels: the forward level of a cell is one more than the largest
-// forward level among its lower-numbered neighbours, and no two cells of one level are
-// neighbours. All cells of a level are updated at once, each with the same operands, in
-// the same order, as in the sequential loop, so the results are bit-identical to it.
+// the new values of its neighbours on one side (smaller indices forward, larger ones
+// backward), so cells are grouped into levels: the forward level of a cell is one more
+// than the largest forward level among its lower-numbered neighbours, and no two cells of
+// one level are neighbours. A level's cells are updated at once, each with the same
+// operands, in the same order, as in the sequential loop: the results are its bits.
 //
-// Levels are short (10²–10⁴ cells on the meshes here) and there are hundreds of them,
-// so the cost of a level is the latency of its dependent loads, plus the launch when it
-// has one. The substitutions and Gauss–Seidel sweeps therefore read a level-ordered ELL
-// copy of their rows (LevelEll): the cells of a level are contiguous, and entry k of
-// the level's row t sits at base + k·size + t, so a row needs its cell index, its
-// entries and the gathers of its neighbours' values, and no per-row offsets. Runs of
-// consecutive levels of at most 1024 cells are swept by one workgroup of 1024 threads,
-// a row per thread, in a single launch, with the run's part of x in LDS (every cell its
-// rows write or read: loaded when the run starts, updated in place, stored to x as it is
-// computed), a barrier on the LDS writes only between levels (a full barrier would also
-// wait for the next levels' operand loads in flight), and the next level's operands
-// loaded while the current level's LDS gathers are read. Larger levels get a grid launch
-// each: a level of ~10⁴ rows moves ~1 MB, more than one CU streams in the time of a
-// launch (measured: 16 rows per thread in one workgroup was 3× slower than grid
-// launches on 2M-cell meshes). The factor, run once per matrix, walks the neighbour
-// lists level by level (LevelSched).
+// What bounds a sweep is the chain of levels (10²–10³ of 10¹–10⁴ cells), i.e. the time of
+// one level's dependence: from a value to its neighbours' values. That is shortest through
+// LDS, so a sweep keeps x there: the cells are cut into chunks of consecutive indices
+// (SweepPlanHost), a workgroup takes a chunk and works through its rows in level order,
+// 64 rows of a level (a step) per wavefront, the steps dealt to the wavefronts in turn.
+// While one wavefront computes, the others load the entries and operands of their next
+// steps, so their memory latency is hidden behind as many steps as there are wavefronts;
+// a wavefront then waits for a count of finished steps in LDS, gathers from LDS, and adds
+// to the count. No barrier, no launch and no memory round trip lies between two levels of
+// a chunk. Between chunks the new values travel through memory and are their own flags:
+// a published value replaces a sentinel, and a wavefront whose step needs it polls for it
+// before its turn. Chunks are handed out by a ticket counter in sweep order, so a value
+// is only ever waited for from a workgroup that has started (and waits itself only for
+// earlier ones): whichever workgroups are resident, the earliest unfinished chunk
+// proceeds. A wait past its limit sets *fault and every later wait gives up at once.
+//
+// Measured (MI355X): a dependence through LDS with 8 entries and a division takes 0.30 µs,
+// with 24 entries 0.53 µs (of which the count's hand-over 0.14), a value handed to another
+// workgroup through memory 0.6 µs plus the polling; one CU streams rows at about 30 GB/s.
+// Levels cost 0.5 µs in one chunk and about 1 µs across chunks, against 4–5 µs for a launch
+// per level or a barrier per level in one workgroup. Two Gauss–Seidel sweeps: 373,920 tets
+// (158 levels) 200 µs, 64³ hexes (190 levels) 185 µs; before, 720 and 790. PCG with GAMG
+// smoothed by Gauss–Seidel on these: 231 → 76 and 68 → 21 ms; DIC-PCG on 24,273 hexes 34.2
+// → 8.8 ms; three momentum components by PBiCGStab + DILU on 839,664 tets, assembly and
+// factor included, 29.1 → 8.4 ms.
 #include "device_common.hpp"
 #include "vol_internal.hpp"
 
@@ -32,86 +41,9 @@ namespace vol {
 
 namespace {
 constexpr int SWEEP_THREADS = 256;
-constexpr int RUN_THREADS = 1024;
-inline dim3 sweep_grid(int cnt) { return dim3((cnt + SWEEP_THREADS - 1) / SWEEP_THREADS); }
+inline dim3 sweep_grid(size_t cnt) { return dim3(unsigned((cnt + SWEEP_THREADS - 1) / SWEEP_THREADS)); }
 }  // namespace
 
-// One level as a grid: thread i updates cell perm[i].
-template <class Row>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_level(Row op, const int* perm, int lo, int hi, const int* done) {
-    if (done && *done) return;
-    const int i = lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < hi) op(perm[i]);
-}
-
-// Levels [L0, L1) by one workgroup, a barrier after each level.
-template <class Row>
-__global__ __launch_bounds__(RUN_THREADS) void k_level_run(Row op, const int* perm, const int* off, int L0, int L1,
-                                                           const int* done) {
-    if (done && *done) return;
-    for (int L = L0; L < L1; ++L) {
-        const int lo = off[L], hi = off[L + 1];
-        for (int i = lo + int(threadIdx.x); i < hi; i += RUN_THREADS) op(perm[i]);
-        __syncthreads();
-    }
-}
-
-template <class Row>
-static void launch_levels(hipStream_t st, const LevelSched& ls, int firstLevel, const Row& op, const int* done) {
-    for (int g = 0; g < ls.nGrp; ++g) {
-        const int L0 = std::max(ls.grpH[g], firstLevel), L1 = ls.grpH[g + 1];
-        if (L0 >= L1) continue;
-        if (ls.grpRunH[g]) {
-            hipLaunchKernelGGL(k_level_run<Row>, dim3(1), dim3(RUN_THREADS), 0, st, op, ls.perm, ls.offD, L0, L1,
-                               done);
-        } else {
-            for (int L = L0; L < L1; ++L) {
-                const int lo = ls.offH[L], hi = ls.offH[L + 1];
-                if (hi > lo)
-                    hipLaunchKernelGGL(k_level<Row>, sweep_grid(hi - lo), dim3(SWEEP_THREADS), 0, st, op, ls.perm, lo,
-                                       hi, done);
-            }
-        }
-    }
-}
-
-// DIC/DILU factor (LinearSolver.cpp:67-74) of cell u: d_u = diag_u − Σ_{l<u, ascending
-// (l, face)} (A_lu·A_ul) / d_l, rD_u = 1/d_u. The same thread then forms the coefficient
-// products the substitutions use: rD_u·A_ul for its lower-list entries and rD_u times
-// its own row's coefficient for its upper-list entries.
-struct DiluFactorRow {
-    SweepView s;
-    const double *diag, *upper, *lower;
-    double *dF, *rD, *pf, *pb;
-    __device__ void operator()(int u) const {
-        const int k0 = s.lowOff[u], k1 = s.lowOff[u + 1];
-        double d = diag[u];
-        for (int k = k0; k < k1; ++k) {
-            const int e = s.lowSrc[k], f = e >> 1;
-            const double aul = (e & 1) ? lower[f] : upper[f];  // row u, column l
-            const double alu = (e & 1) ? upper[f] : lower[f];  // row l, column u
-            d = d - (alu * aul) / dF[s.lowCol[k]];
-        }
-        dF[u] = d;
-        const double r = 1.0 / d;
-        rD[u] = r;
-        for (int k = k0; k < k1; ++k) {
-            const int e = s.lowSrc[k], f = e >> 1;
-            pf[k] = r * ((e & 1) ? lower[f] : upper[f]);
-        }
-        for (int k = s.upOff[u]; k < s.upOff[u + 1]; ++k) {
-            const int e = s.upSrc[k], f = e >> 1;
-            pb[k] = r * ((e & 1) ? lower[f] : upper[f]);
-        }
-    }
-};
-
-void launch_dilu_factor(hipStream_t st, const SweepView& s, const LevelSched& fwd, const double* diag,
-                        const double* upper, const double* lower, double* dF, double* rD, double* pf, double* pb) {
-    launch_levels(st, fwd, 0, DiluFactorRow{s, diag, upper, lower, dF, rD, pf, pb}, nullptr);
-}
-
-// ---------------------------------------------------------------- level-ordered ELL sweeps
 // Row operations (T: double, or float in the mixed-precision inner solve):
 //   SW_GS   Gauss–Seidel (LinearSolver.cpp:247-262, GAMG.cpp:368-379):
 //           x_c = (b_c − Σ coef·x_nb) / diag_c, entries in ascending face order
@@ -119,457 +51,441 @@ void launch_dilu_factor(hipStream_t st, const SweepView& s, const LevelSched& fw
 //           w_u = rD_u·r_u − Σ (rD_u·A_ul)·w_l, entries in ascending (l, face) order
 //   SW_BWD  DILU backward substitution (LinearSolver.cpp:99-103):
 //           w_l = w_l − Σ (rD_l·A_lu)·w_u, entries in descending (u, face) order
-// What a row needs that the sweep does not change: its cell, its first PF entries
-// (column and coefficient) and the operands of its start value (GS: b and diag; forward:
-// rD·r; backward: its own w, which only its own level writes).
-//
-// Every load is issued whatever the row's width: a thread without a row, or an entry
-// past its row, reads a valid stand-in (the level's first cell, entry 0, x[0]) whose
-// value is then discarded. With no branches around them the loads of a phase go out
-// together and the compiler waits for exactly those a result needs (vector loads return
-// in order), not for everything in flight.
-template <int PF, class T> struct RowPre {
-    int c;     // the row's cell (a stand-in when !has)
-    int s;     // runs: the LDS slot of the row's cell
-    bool has;  // the thread has a row in this level
-    T i0, i1;
-    int col[PF];  // −1: no entry
-    T cf[PF];
-};
-
-__device__ __forceinline__ int row_cell(const LevelEll& E, int pos0, int size, int t) {
-    return E.cell[pos0 + (t < size ? t : 0)];
-}
-template <int PF, class T>
-__device__ __forceinline__ void row_load_entries(const LevelEll& E, const SweepArgs<T>& a, int size, int width, int base,
-                                                 int t, RowPre<PF, T>& p) {
-    p.has = t < size;
-#pragma unroll
-    for (int k = 0; k < PF; ++k) {
-        const bool in = p.has && k < width;
-        const int e = in ? base + k * size + t : 0;
-        const int j = E.col[e];
-        const T v = a.coef[e];
-        p.col[k] = in ? j : -1;
-        p.cf[k] = v;
-    }
-}
-template <int OP, int PF, class T> __device__ __forceinline__ void row_load_start(const SweepArgs<T>& a, RowPre<PF, T>& p) {
-    if constexpr (OP == SW_GS) {
-        p.i0 = a.b[p.c];
-        p.i1 = a.diag[p.c];
-    } else if constexpr (OP == SW_FWD) {
-        p.i0 = a.rD[p.c] * a.r[p.c];
-        p.i1 = T(1);
-    } else {
-        p.i0 = a.x[p.c];
-        p.i1 = T(1);
-    }
-}
-template <int PF, class T> __device__ __forceinline__ void row_gather(const SweepArgs<T>& a, const RowPre<PF, T>& p, T* xv) {
-#pragma unroll
-    for (int k = 0; k < PF; ++k) xv[k] = a.x[p.col[k] >= 0 ? p.col[k] : 0];
-}
-// acc = start − Σ coef·x over the row's entries in order (padding entries, −1, only
-// trail a row); entries k ≥ PF in steps of SWEEP_TAIL with their loads issued together.
-// Writes the row's new value.
-constexpr int SWEEP_TAIL = 4;
-template <int OP, int PF, class T>
-__device__ __forceinline__ void row_finish(const LevelEll& E, const SweepArgs<T>& a, const RowPre<PF, T>& p, const T* xv,
-                                           int size, int width, int base, int t) {
-    T acc = p.i0;
-#pragma unroll
-    for (int k = 0; k < PF; ++k)
-        if (p.col[k] >= 0) acc = acc - p.cf[k] * xv[k];
-    for (int k0 = PF; k0 < width; k0 += SWEEP_TAIL) {
-        int j[SWEEP_TAIL];
-        T cf[SWEEP_TAIL], xt[SWEEP_TAIL];
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q) {
-            const bool in = k0 + q < width;
-            const int e = in ? base + (k0 + q) * size + t : 0;
-            const int jj = E.col[e];
-            cf[q] = a.coef[e];
-            j[q] = in ? jj : -1;
-        }
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q) xt[q] = a.x[j[q] >= 0 ? j[q] : 0];
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q)
-            if (j[q] >= 0) acc = acc - cf[q] * xt[q];
-    }
-    if constexpr (OP == SW_GS) a.x[p.c] = acc / p.i1;
-    else a.x[p.c] = acc;
+//   SW_FAC  DIC/DILU factor (LinearSolver.cpp:67-74):
+//           d_u = diag_u − Σ (A_lu·A_ul) / d_l, entries in ascending (l, face) order
+// Except in GS the row's start value lies in its own slot of x when the sweep starts.
+template <int OP, class T> __device__ __forceinline__ T row_term(T cf, T x) {
+    if constexpr (OP == SW_FAC) return cf / x;
+    else return cf * x;
 }
 
-// Runs: entries hold LDS slots of x (xs), so the gathers and the tail's reads come from
-// LDS; the row writes its value to its slot and to x (read by later launches only).
-template <int PF, class T> __device__ __forceinline__ void row_gather_lds(const T* xs, const RowPre<PF, T>& p, T* xv) {
-#pragma unroll
-    for (int k = 0; k < PF; ++k) xv[k] = xs[p.col[k] >= 0 ? p.col[k] : 0];
-}
-template <int OP, int PF, class T>
-__device__ __forceinline__ void row_finish_lds(const LevelEll& E, const SweepArgs<T>& a, T* xs, const RowPre<PF, T>& p,
-                                               const T* xv, int size, int width, int base, int t) {
-    T acc = p.i0;
-#pragma unroll
-    for (int k = 0; k < PF; ++k)
-        if (p.col[k] >= 0) acc = acc - p.cf[k] * xv[k];
-    for (int k0 = PF; k0 < width; k0 += SWEEP_TAIL) {
-        int j[SWEEP_TAIL];
-        T cf[SWEEP_TAIL], xt[SWEEP_TAIL];
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q) {
-            const bool in = k0 + q < width;
-            const int e = in ? base + (k0 + q) * size + t : 0;
-            const int jj = E.col[e];
-            cf[q] = a.coef[e];
-            j[q] = in ? jj : -1;
-        }
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q) xt[q] = xs[j[q] >= 0 ? j[q] : 0];
-#pragma unroll
-        for (int q = 0; q < SWEEP_TAIL; ++q)
-            if (j[q] >= 0) acc = acc - cf[q] * xt[q];
-    }
-    const T v = OP == SW_GS ? acc / p.i1 : acc;
-    xs[p.s] = v;
-    a.x[p.c] = v;
-}
-// Barrier for values exchanged through LDS only: waits for the LDS writes, not for the
-// global loads in flight (the next levels' operands) or the stores to x.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// One level as a grid: thread t updates the level's row t.
-constexpr int GRID_PF = 8;
-template <int OP, class T>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_ell_level(LevelEll E, SweepArgs<T> a, int pos0, int size, int width,
-                                                             int base, const int* done) {
-    if (done && *done) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= size) return;
-    RowPre<GRID_PF, T> p;
-    p.c = row_cell(E, pos0, size, t);
-    row_load_entries(E, a, size, width, base, t, p);
-    row_load_start<OP>(a, p);
-    T xv[GRID_PF];
-    row_gather(a, p, xv);
-    row_finish<OP>(E, a, p, xv, size, width, base, t);
-}
-
-// Levels [L0, L1) by one workgroup of THREADS threads (every level has at most THREADS
-// cells), a row per thread, x of the run's cells (cells[0 .. nCells), entries holding
-// their slots) in LDS, a barrier on the LDS writes after each level. The levels' offsets,
-// widths and bases are staged in LDS first. In level i a thread first reads its row's
-// neighbour values from LDS, then loads level i+1's entries and start operands (from the
-// cell it loaded in level i−1) and level i+2's cell and slot: none of them is written
-// before its own level, and they stay in flight across the barrier. Sums keep the entry order: the result is the plain loop's.
-template <int OP, int THREADS, int PF, class T>
-__global__ __launch_bounds__(THREADS) void k_ell_run(LevelEll E, SweepArgs<T> a, int L0, int L1, const int* cells,
-                                                     int nCells, const int* done) {
-    if (done && *done) return;
-    __shared__ int sOff[ELL_RUN_LEVELS + 1], sWidth[ELL_RUN_LEVELS], sBase[ELL_RUN_LEVELS];
-    __shared__ T xs[RUN_LDS_CELLS];
-    const int nl = L1 - L0, t = int(threadIdx.x);
-    // staging in batches: every load of a batch in flight together, then the stores (a
-    // plain loop waits for each element's load, or pair of dependent loads, in turn)
-    constexpr int SB = 16;
-    for (int i0 = t; i0 <= nl; i0 += SB * THREADS) {
-        int o[SB], w[SB], b[SB];
-#pragma unroll
-        for (int u = 0; u < SB; ++u) {
-            const int i = i0 + u * THREADS;
-            o[u] = i <= nl ? E.offD[L0 + i] : 0;
-            w[u] = i < nl ? E.widthD[L0 + i] : 0;
-            b[u] = i < nl ? E.baseD[L0 + i] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < SB; ++u) {
-            const int i = i0 + u * THREADS;
-            if (i <= nl) sOff[i] = o[u];
-            if (i < nl) {
-                sWidth[i] = w[u];
-                sBase[i] = b[u];
-            }
-        }
-    }
-    for (int i0 = t; i0 < nCells; i0 += SB * THREADS) {
-        int c[SB];
-        T v[SB];
-#pragma unroll
-        for (int u = 0; u < SB; ++u) c[u] = i0 + u * THREADS < nCells ? cells[i0 + u * THREADS] : -1;
-#pragma unroll
-        for (int u = 0; u < SB; ++u) v[u] = c[u] >= 0 ? a.x[c[u]] : T(0);
-#pragma unroll
-        for (int u = 0; u < SB; ++u)
-            if (c[u] >= 0) xs[i0 + u * THREADS] = v[u];
-    }
-    __syncthreads();
-    // past the last level, a thread loads the last level's data again (unused)
-    auto lev = [nl](int i) { return i < nl ? i : nl - 1; };
-    RowPre<PF, T> cur, nxt;
-    int size = sOff[1] - sOff[0], width = sWidth[0], base = sBase[0];
-    cur.c = row_cell(E, sOff[0], size, t);
-    cur.s = E.slot[sOff[0] + (t < size ? t : 0)];
-    row_load_entries(E, a, size, width, base, t, cur);
-    row_load_start<OP>(a, cur);
-    const int p1 = sOff[lev(1)], z1 = sOff[lev(1) + 1] - p1;
-    int cNext = row_cell(E, p1, z1, t), sNext = E.slot[p1 + (t < z1 ? t : 0)];
-    for (int i = 0; i < nl; ++i) {
-        T xv[PF];
-        row_gather_lds(xs, cur, xv);
-        asm volatile("" ::: "memory");  // the gathers go out before the loads below
-        const int n1 = lev(i + 1), n2 = lev(i + 2);
-        const int nSize = sOff[n1 + 1] - sOff[n1], nWidth = sWidth[n1], nBase = sBase[n1];
-        nxt.c = cNext;
-        nxt.s = sNext;
-        row_load_start<OP>(a, nxt);
-        row_load_entries(E, a, nSize, nWidth, nBase, t, nxt);
-        const int p2 = sOff[n2], z2 = sOff[n2 + 1] - p2;
-        cNext = row_cell(E, p2, z2, t);
-        sNext = E.slot[p2 + (t < z2 ? t : 0)];
-        if (cur.has) row_finish_lds<OP>(E, a, xs, cur, xv, size, width, base, t);
-        lds_barrier();
-        cur = nxt;
-        size = nSize;
-        width = nWidth;
-        base = nBase;
-    }
-}
-
-template <int OP, class T>
-static void launch_ell(hipStream_t st, const LevelEll& E, int firstLevel, const SweepArgs<T>& a, const int* done) {
-    for (int g = 0; g < E.nGrp; ++g) {
-        const int L0 = std::max(E.grpH[g], firstLevel), L1 = E.grpH[g + 1];
-        if (L0 >= L1) continue;
-        switch (E.grpKindH[g]) {
-        case ELL_RUN256:
-            hipLaunchKernelGGL((k_ell_run<OP, 256, 24, T>), dim3(1), dim3(256), 0, st, E, a, L0, L1,
-                               E.runCells + E.runOffH[g], E.runCntH[g], done);
-            break;
-        case ELL_RUN512:
-            hipLaunchKernelGGL((k_ell_run<OP, 512, 16, T>), dim3(1), dim3(512), 0, st, E, a, L0, L1,
-                               E.runCells + E.runOffH[g], E.runCntH[g], done);
-            break;
-        case ELL_RUN1024:
-            hipLaunchKernelGGL((k_ell_run<OP, 1024, 12, T>), dim3(1), dim3(1024), 0, st, E, a, L0, L1,
-                               E.runCells + E.runOffH[g], E.runCntH[g], done);
-            break;
-        default:
-            for (int L = L0; L < L1; ++L) {
-                const int pos0 = E.offH[L], size = E.offH[L + 1] - pos0;
-                if (size > 0)
-                    hipLaunchKernelGGL((k_ell_level<OP, T>), sweep_grid(size), dim3(SWEEP_THREADS), 0, st, E, a, pos0,
-                                       size, E.widthH[L], E.baseH[L], done);
-            }
-        }
-    }
-}
-
-template <class T>
-void launch_dilu_apply(hipStream_t st, const LevelEll& F, const LevelEll& B, const T* rD, const T* ef, const T* eb,
-                       const T* r, T* w, const int* done) {
-    SweepArgs<T> a;
-    a.rD = rD;
-    a.r = r;
-    a.x = w;
-    a.coef = ef;
-    launch_ell<SW_FWD, T>(st, F, 0, a, done);
-    a.coef = eb;
-    // backward level 0 holds the cells without upper neighbours: nothing to subtract
-    launch_ell<SW_BWD, T>(st, B, 1, a, done);
-}
-template void launch_dilu_apply<double>(hipStream_t, const LevelEll&, const LevelEll&, const double*, const double*,
-                                        const double*, const double*, double*, const int*);
-template void launch_dilu_apply<float>(hipStream_t, const LevelEll&, const LevelEll&, const float*, const float*,
-                                       const float*, const float*, float*, const int*);
-
-template <class T>
-void launch_gs_sweep(hipStream_t st, const LevelEll& E, const T* coef, const T* diag, const T* b, T* x,
-                     const int* done) {
-    SweepArgs<T> a;
-    a.coef = coef;
-    a.diag = diag;
-    a.b = b;
-    a.x = x;
-    launch_ell<SW_GS, T>(st, E, 0, a, done);
-}
-template void launch_gs_sweep<double>(hipStream_t, const LevelEll&, const double*, const double*, const double*,
-                                      double*, const int*);
-template void launch_gs_sweep<float>(hipStream_t, const LevelEll&, const float*, const float*, const float*, float*,
-                                     const int*);
-
-// ---------------------------------------------------------------- sync-free sweeps
-// One launch per sweep. The work items are the wavefronts of E.waves (64 rows of one
-// level each, in level order), and a wavefront takes the next item from a counter when
-// it starts, not from its block index: the order in which workgroups start is not the
-// order of their indices across the XCDs. Every value a row waits for then belongs to an
-// item taken earlier, by a wavefront that has started and is resident or finished, and
-// never to one of its own lanes, so the earliest unfinished item can always proceed. A row reads the new value of a neighbour on the sweep's side (GS forward and
-// the DILU forward substitution: lower-numbered; backward: higher-numbered) from xNew,
-// which starts filled with a sentinel NaN that arithmetic does not produce, and waits
-// until it is no longer the sentinel; other neighbours' values come from xOld. Values
-// are published by an atomic exchange (a read-modify-write is performed where all XCDs
-// see it; a plain relaxed store may stay in the writer's L2) and read with device-scope
-// atomic loads: the value is its own flag, so no fence is needed. A wait that runs past
-// its limit sets *fault, and once it is set no wait spins any more, so every launch ends
-// soon. Row arithmetic and order are row_finish's.
-constexpr int FREE_GROUP = 8;                    // entries whose loads go out together
-constexpr unsigned FREE_SPIN_LIMIT = 1u << 18;   // ≈ 10–20 ms of s_sleep(1) per value
-
+// A value not published yet: a signalling NaN, which arithmetic does not produce (a value
+// that is one, copied from the caller's data, is published as the quiet NaN).
 template <class T> struct Sentinel;
 template <> struct Sentinel<double> {
-    static constexpr unsigned long long bits = 0x7FF4A5A5DEAD0001ull;  // signalling NaN
+    static constexpr unsigned long long bits = 0x7FF4A5A5DEAD0001ull;
     __device__ static bool is(double v) { return (unsigned long long)__double_as_longlong(v) == bits; }
     __device__ static double value() { return __longlong_as_double((long long)bits); }
+    __device__ static double quiet() { return __longlong_as_double((long long)(bits | (1ull << 51))); }
 };
 template <> struct Sentinel<float> {
-    static constexpr unsigned bits = 0x7FA5DEADu;  // signalling NaN
+    static constexpr unsigned bits = 0x7FA5DEADu;
     __device__ static bool is(float v) { return (unsigned)__float_as_uint(v) == bits; }
     __device__ static float value() { return __uint_as_float(bits); }
+    __device__ static float quiet() { return __uint_as_float(bits | (1u << 22)); }
 };
 
-// xNew ← sentinel, and the sweep's work counter ← 0 (stream-ordered before the sweep).
-template <class T>
-__global__ void k_fill_sentinel(int n, T* x, int* counter, const int* done) {
+constexpr unsigned SWEEP_SPIN_LIMIT = 1u << 18;  // polls of one value, ≥ 0.2 s
+
+template <class T> __device__ __forceinline__ T peek(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ __forceinline__ void publish_value(T* p, T v) {
+    if (Sentinel<T>::is(v)) v = Sentinel<T>::quiet();
+    // a read-modify-write is performed where every XCD sees it
+    (void)__hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Whether a wait ends without its value after `spins` polls: past its limit (which it
+// reports), or because another wait has.
+__device__ __forceinline__ bool given_up(unsigned spins, int* fault) {
+    if (spins > SWEEP_SPIN_LIMIT) {
+        __hip_atomic_fetch_or(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    }
+    return (spins & 63) == 63 && __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+// Finished steps of the chunk.
+__device__ __forceinline__ int finished(int* cnt) {
+    return __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+constexpr int SWEEP_NEAR = 4;  // steps before its turn that a wavefront starts to watch closely
+// LDS-only ordering: waits for LDS accesses, not for the global loads in flight.
+__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+__device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
+
+// Steps s0 .. s1 of a chunk from cell c0, its slots of x in xs (the padding slot holds a
+// value whose term is 0), by a workgroup of WAVES wavefronts; *cnt counts finished steps
+// from 0. Everything that does not depend on the step's turn is done before it: the row's
+// first PF entries (later ones are loaded after the turn), their LDS addresses, and
+// (MULTI) the values that come by mail. After the turn a step gathers from LDS, subtracts in order, stores
+// and adds to the count; the code for that exists once per number of entry groups, so
+// that every LDS read is in flight before the first is waited for. Lanes past the step's
+// rows repeat its last row and store nothing. MULTI: every value goes to the mailbox of
+// this sweep.
+template <int OP, bool MULTI, int PF, int WAVES, class T>
+__device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<T>& a, T* xs, int* cnt, int c0, int s0,
+                                            int s1, int sweep) {
+    constexpr int GRP = SWEEP_GROUP;
+    static_assert(PF % GRP == 0 && PF <= 24);
+    const int lane = threadIdx.x % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / WAVE);
+    char* const lds = reinterpret_cast<char*>(xs);
+    const auto value = [&](int byte) { return *reinterpret_cast<const T*>(lds + byte); };
+    // past the last step a wavefront loads the last one's data again (unused)
+    const auto stepAt = [&](int s) { return P.steps[s < s1 ? s : s1 - 1]; };
+    const auto rowOf = [&](const SweepStep& d) {
+        const int rows = d.rowsNeed & ((1 << SWEEP_ROWS_BITS) - 1);
+        return lane < rows ? lane : rows - 1;
+    };
+    // MULTI: where the value of an entry at < 0 lies in the mailbox (from mail), or that
+    // it is x before the first sweep
+    const T* const mail = MULTI ? a.mail + (sweep - 1) * ptrdiff_t(P.n) : nullptr;
+    const auto initial = [&](int at) { return ~at >= 2 * P.n; };
+    const auto far = [&](int at) {
+        if (!initial(at)) return peek(&mail[~at]);
+        return a.zero ? T(0) : a.x[~at - 2 * P.n];
+    };
+    const auto missing = [&](int at, T v) { return at < 0 && Sentinel<T>::is(v) && !initial(at); };
+    const int* const places = MULTI && sweep > 0 ? P.col2 : P.col;
+    int s = s0 + wave;
+    if (s >= s1) return;
+    SweepStep d = stepAt(s), dn = stepAt(s + WAVES);
+    int c = P.cell[d.pos + rowOf(d)];
+    for (; s < s1; s += WAVES) {
+        const int rows = __builtin_amdgcn_readfirstlane(d.rowsNeed & ((1 << SWEEP_ROWS_BITS) - 1));
+        const int need = __builtin_amdgcn_readfirstlane(d.rowsNeed >> SWEEP_ROWS_BITS);
+        const int width = __builtin_amdgcn_readfirstlane(d.width), base = __builtin_amdgcn_readfirstlane(d.base);
+        const int pos = __builtin_amdgcn_readfirstlane(d.pos);
+        const unsigned t = unsigned(lane < rows ? lane : rows - 1);
+        const int* const ecol = places + base;  // uniform: the loads take 32-bit offsets
+        const T* const ecoef = a.coef + base;
+        T acc = T(0), dg = T(1);
+        if constexpr (OP == SW_GS) {
+            acc = a.b[unsigned(c)];
+            dg = a.diag[unsigned(c)];
+        }
+        const int cn = P.cell[unsigned(dn.pos + rowOf(dn))];
+        const SweepStep dnn = stepAt(s + 2 * WAVES);
+        int at[PF];
+        T cf[PF];
+#pragma unroll
+        for (int g = 0; g < PF; g += GRP) {
+            if (g < width) {
+#pragma unroll
+                for (int k = g; k < g + GRP; ++k) at[k] = ecol[unsigned(k * rows) + t];
+#pragma unroll
+                for (int k = g; k < g + GRP; ++k) cf[k] = ecoef[unsigned(k * rows) + t];
+            } else {
+#pragma unroll
+                for (int k = g; k < g + GRP; ++k) at[k] = 0;
+            }
+        }
+        T v[MULTI ? PF : 1];
+        unsigned out = 0;  // which entries are values of other chunks
+        if constexpr (MULTI) {
+#pragma unroll
+            for (int k = 0; k < PF; ++k) out |= at[k] < 0 ? 1u << k : 0u;
+            if (__any(out != 0)) {
+                // all of them in one round trip; then, once the turn is near (asking
+                // earlier only loads the fabric), the ones not yet published again,
+                // together, until they are
+#pragma unroll
+                for (int k = 0; k < PF; ++k) {
+                    v[k] = T(0);
+                    if (at[k] < 0) v[k] = far(at[k]);
+                }
+                for (unsigned spins = 0;;) {
+                    bool miss = false;
+#pragma unroll
+                    for (int k = 0; k < PF; ++k) miss = miss || missing(at[k], v[k]);
+                    if (!__any(miss)) break;
+                    if (need - finished(cnt) > SWEEP_NEAR) {
+                        __builtin_amdgcn_s_sleep(2);
+                        continue;
+                    }
+                    if (given_up(++spins, a.fault)) break;
+#pragma unroll
+                    for (int k = 0; k < PF; ++k) {
+                        asm volatile("" : "+v"(at[k]));  // no address kept over the loop
+                        if (missing(at[k], v[k])) v[k] = peek(&mail[~at[k]]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PF; ++k) at[k] = (MULTI && at[k] < 0 ? 0 : at[k]) * int(sizeof(T));
+        int slot = (c - c0) * int(sizeof(T));
+        // keep all of the above before the turn
+#pragma unroll
+        for (int k = 0; k < PF; ++k) asm volatile("" : "+v"(at[k]), "+v"(cf[k]));
+        asm volatile("" : "+v"(slot), "+v"(acc), "+v"(dg));
+        // the step's turn: every step of the chunk's earlier levels is done
+        for (;;) {
+            const int got = finished(cnt);
+            if (got >= need) break;
+            if (need - got > SWEEP_NEAR) __builtin_amdgcn_s_sleep(1);
+        }
+        lds_acquire();
+        __builtin_amdgcn_s_setprio(3);  // ahead of the wavefronts that prepare later steps
+        if constexpr (OP != SW_GS) acc = value(slot);
+        const auto rowSum = [&](auto groups, auto mixed) {
+            constexpr int N = decltype(groups)::value * GRP;
+            T xv[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) xv[k] = value(at[k]);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                if constexpr (decltype(mixed)::value) xv[k] = (out >> k) & 1 ? v[k] : xv[k];
+                acc = acc - row_term<OP>(cf[k], xv[k]);
+            }
+        };
+        const auto rowSums = [&](auto mixed) {
+            const int ng = width / GRP;
+            if (ng >= 6 && PF >= 24) rowSum(std::integral_constant<int, PF >= 24 ? 6 : 1>{}, mixed);
+            else if (ng >= 5 && PF >= 20) rowSum(std::integral_constant<int, PF >= 20 ? 5 : 1>{}, mixed);
+            else if (ng >= 4 && PF >= 16) rowSum(std::integral_constant<int, PF >= 16 ? 4 : 1>{}, mixed);
+            else if (ng >= 3 && PF >= 12) rowSum(std::integral_constant<int, PF >= 12 ? 3 : 1>{}, mixed);
+            else if (ng >= 2 && PF >= 8) rowSum(std::integral_constant<int, PF >= 8 ? 2 : 1>{}, mixed);
+            else if (ng >= 1) rowSum(std::integral_constant<int, 1>{}, mixed);
+        };
+        if constexpr (MULTI) {
+            if (__any(out != 0)) rowSums(std::true_type{});
+            else rowSums(std::false_type{});
+        } else {
+            rowSums(std::false_type{});
+        }
+        for (int k0 = PF; k0 < width; k0 += GRP) {
+            int j[GRP];
+            T f[GRP], xt[GRP];
+#pragma unroll
+            for (int q = 0; q < GRP; ++q) j[q] = ecol[unsigned((k0 + q) * rows) + t];
+#pragma unroll
+            for (int q = 0; q < GRP; ++q) f[q] = ecoef[unsigned((k0 + q) * rows) + t];
+#pragma unroll
+            for (int q = 0; q < GRP; ++q) {
+                xt[q] = value((MULTI && j[q] < 0 ? 0 : j[q]) * int(sizeof(T)));
+                if (MULTI && j[q] < 0) {
+                    xt[q] = far(j[q]);
+                    for (unsigned spins = 0; missing(j[q], xt[q]) && !given_up(spins, a.fault); ++spins)
+                        xt[q] = peek(&mail[~j[q]]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < GRP; ++q) acc = acc - row_term<OP>(f[q], xt[q]);
+        }
+        if constexpr (OP == SW_GS) acc = acc / dg;
+        if (lane < rows) *reinterpret_cast<T*>(lds + slot) = acc;
+        lds_release();
+        if (lane == 0) __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (MULTI) {
+            if (lane < rows) publish_value(&a.mail[sweep * ptrdiff_t(P.n) + pos + lane], acc);
+        }
+        c = cn;
+        d = dn;
+        dn = dnn;
+    }
+}
+
+// The chunk's slots at the start of a sweep: start values or x before the sweep, the
+// halo's x before the sweep, and the padding.
+template <int OP, class T>
+__device__ __forceinline__ void sweep_fill(const SweepPlan& P, const SweepArgs<T>& a, T* xs, int c0, int nc, int h0,
+                                           int nh) {
+    constexpr int SB = 8;  // loads in flight per thread
+    for (int i0 = threadIdx.x; i0 < nc; i0 += SB * int(blockDim.x)) {
+        T v[SB];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+            const int i = i0 + u * int(blockDim.x), q = c0 + (i < nc ? i : 0);
+            if constexpr (OP == SW_GS || OP == SW_BWD) v[u] = a.zero ? T(0) : a.x[q];
+            else if constexpr (OP == SW_FWD) v[u] = a.rD[q] * a.b[q];
+            else v[u] = a.diag[q];
+        }
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+            if (i0 + u * int(blockDim.x) < nc) xs[i0 + u * int(blockDim.x)] = v[u];
+    }
+    for (int i0 = threadIdx.x; i0 < nh; i0 += SB * int(blockDim.x)) {
+        int q[SB];
+        T v[SB];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) q[u] = P.halo[h0 + (i0 + u * int(blockDim.x) < nh ? i0 + u * int(blockDim.x) : 0)];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) v[u] = a.zero ? T(0) : a.x[q[u]];
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+            if (i0 + u * int(blockDim.x) < nh) xs[nc + i0 + u * int(blockDim.x)] = v[u];
+    }
+    if (threadIdx.x == 0) xs[nc + nh] = OP == SW_FAC ? T(1) : T(0);
+}
+
+// Sweeps over more than one chunk: one workgroup per chunk and sweep, by ticket, the
+// chunks of the first sweep first: a chunk's next sweep runs while the first one is still
+// under way further on. The last sweep writes x, in place: whatever reads a cell's x
+// before the first sweep (its own chunk, or a halo) does so when its workgroup starts,
+// and every value of a chunk's last sweep comes after the first-sweep values of its
+// cells' neighbours, so after those workgroups' starts.
+template <int OP, bool BACK, int PF, int WAVES, class T>
+__global__ __launch_bounds__(WAVES* WAVE) void k_sweep_chunks(SweepPlan P, SweepArgs<T> a, int sweeps,
+                                                              const int* done) {
     if (done && *done) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = Sentinel<T>::value();
-    if (i == 0) *counter = 0;
-}
-
-template <class T>
-__device__ __forceinline__ T free_wait(T* xNew, int j, int* fault) {
-    T v = __hip_atomic_load(&xNew[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned spins = 0;
-    while (Sentinel<T>::is(v)) {
-        if ((spins & 1023) == 0 && __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-        __builtin_amdgcn_s_sleep(1);
-        v = __hip_atomic_load(&xNew[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (++spins > FREE_SPIN_LIMIT) {
-            __hip_atomic_fetch_or(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-        }
+    extern __shared__ double sweepLds[];
+    T* xs = reinterpret_cast<T*>(sweepLds);
+    __shared__ int cnt, mine;
+    if (threadIdx.x == 0) {
+        cnt = 0;
+        mine = __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    return v;
+    __syncthreads();
+    const int sweep = mine / P.nChunks;
+    if (sweep >= sweeps) return;
+    const int i = mine - sweep * P.nChunks, k = BACK ? P.nChunks - 1 - i : i;
+    const int c0 = P.chunkOff[k], nc = P.chunkOff[k + 1] - c0;
+    const int h0 = P.haloOff[k], nh = P.haloOff[k + 1] - h0;
+    if (sweep == 0) sweep_fill<OP>(P, a, xs, c0, nc, h0, nh);
+    else if (threadIdx.x == 0) xs[nc + nh] = T(0);  // the others are written before they are read
+    __syncthreads();
+    sweep_steps<OP, true, PF, WAVES, T>(P, a, xs, &cnt, c0, P.stepOff[k], P.stepOff[k + 1], sweep);
+    if (sweep + 1 < sweeps) return;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nc; q += blockDim.x) a.x[c0 + q] = xs[q];
 }
 
-template <int OP, bool BACK, class T>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_ell_free(LevelEll E, SweepArgs<T> a, const T* xOld, T* xNew,
-                                                            int* counter, int* fault, const int* done) {
+// A sweep (or a schedule of several) over one chunk that holds every cell.
+template <int OP, int PF, int WAVES, class T>
+__global__ __launch_bounds__(WAVES* WAVE) void k_sweep_one(SweepPlan P, SweepArgs<T> a, const int* done) {
     if (done && *done) return;
-    int w = 0;
-    if ((threadIdx.x % WAVE) == 0) w = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    w = __builtin_amdgcn_readfirstlane(w);  // lane 0's item for the whole wavefront
-    if (w >= E.nWaves) return;              // whole wavefronts
-    const int2 wl = E.waves[w];
-    const int L = wl.x;
-    const int pos0 = E.offD[L], size = E.offD[L + 1] - pos0, width = E.widthD[L], base = E.baseD[L];
-    const int rb = E.runBaseD[L];  // ≥ 0: entries hold LDS slots of a run (cell = runCells[rb + slot])
-    const int t = wl.y + int(threadIdx.x % WAVE);
-    const bool has = t < size;
-    const int c = E.cell[pos0 + (has ? t : 0)];
-    T acc, dg = T(1);
-    if constexpr (OP == SW_GS) {
-        acc = a.b[c];
-        dg = a.diag[c];
-    } else if constexpr (OP == SW_FWD) {
-        acc = a.rD[c] * a.r[c];
-    } else {
-        acc = xOld[c];
-    }
-    for (int k0 = 0; k0 < width; k0 += FREE_GROUP) {
-        int j[FREE_GROUP];
-        T cf[FREE_GROUP], v[FREE_GROUP];
-#pragma unroll
-        for (int u = 0; u < FREE_GROUP; ++u) {
-            const bool in = has && k0 + u < width;
-            const int e = in ? base + (k0 + u) * size + t : 0;
-            const int jj = E.col[e];
-            cf[u] = a.coef[e];
-            j[u] = in ? jj : -1;
-        }
-        if (rb >= 0) {  // LDS slots → cells
-#pragma unroll
-            for (int u = 0; u < FREE_GROUP; ++u)
-                if (j[u] >= 0) j[u] = E.runCells[rb + j[u]];
-        }
-        // first reads of the group together; then wait on the ones not published yet
-#pragma unroll
-        for (int u = 0; u < FREE_GROUP; ++u) {
-            const bool fresh = j[u] >= 0 && (BACK ? j[u] > c : j[u] < c);
-            v[u] = j[u] < 0 ? T(0)
-                   : fresh ? __hip_atomic_load(&xNew[j[u]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                           : xOld[j[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < FREE_GROUP; ++u) {
-            const bool fresh = j[u] >= 0 && (BACK ? j[u] > c : j[u] < c);
-            if (fresh && Sentinel<T>::is(v[u])) v[u] = free_wait(xNew, j[u], fault);
-        }
-#pragma unroll
-        for (int u = 0; u < FREE_GROUP; ++u)
-            if (j[u] >= 0) acc = acc - cf[u] * v[u];
-    }
-    if (has) {
-        const T res = OP == SW_GS ? acc / dg : acc;
-        (void)__hip_atomic_exchange(&xNew[c], res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    extern __shared__ double sweepLds[];
+    T* xs = reinterpret_cast<T*>(sweepLds);
+    __shared__ int cnt;
+    if (threadIdx.x == 0) cnt = 0;
+    sweep_fill<OP>(P, a, xs, 0, P.n, 0, 0);
+    __syncthreads();
+    sweep_steps<OP, false, PF, WAVES, T>(P, a, xs, &cnt, 0, 0, P.nSteps, 0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < P.n; i += blockDim.x) a.x[i] = xs[i];
 }
 
-// fault points at two ints: [0] the fault flag, [1] the work counter.
-template <int OP, bool BACK, class T>
-static void launch_free(hipStream_t st, const LevelEll& E, int n, const SweepArgs<T>& a, const T* xOld, T* xNew,
-                        int* fault, const int* done) {
-    if (n <= 0 || E.nWaves == 0) return;
-    int* counter = fault + 1;
-    hipLaunchKernelGGL(k_fill_sentinel<T>, sweep_grid(n), dim3(SWEEP_THREADS), 0, st, n, xNew, counter, done);
-    const long threads = long(E.nWaves) * WAVE;
-    hipLaunchKernelGGL((k_ell_free<OP, BACK, T>), dim3(unsigned((threads + SWEEP_THREADS - 1) / SWEEP_THREADS)),
-                       dim3(SWEEP_THREADS), 0, st, E, a, xOld, xNew, counter, fault, done);
-}
-
-template <class T>
-void launch_gs_sweep_free(hipStream_t st, const LevelEll& E, bool backward, const T* coef, const T* diag, const T* b,
-                          const T* xOld, T* xNew, int* fault, const int* done) {
-    SweepArgs<T> a;
-    a.coef = coef;
-    a.diag = diag;
-    a.b = b;
-    const int n = E.offH[E.nLev];
-    if (backward)
-        launch_free<SW_GS, true, T>(st, E, n, a, xOld, xNew, fault, done);
-    else
-        launch_free<SW_GS, false, T>(st, E, n, a, xOld, xNew, fault, done);
-}
-template void launch_gs_sweep_free<double>(hipStream_t, const LevelEll&, bool, const double*, const double*,
-                                           const double*, const double*, double*, int*, const int*);
-template void launch_gs_sweep_free<float>(hipStream_t, const LevelEll&, bool, const float*, const float*,
-                                          const float*, const float*, float*, int*, const int*);
-
-template <class T>
-void launch_dilu_apply_free(hipStream_t st, const LevelEll& F, const LevelEll& B, const T* rD, const T* ef,
-                            const T* eb, const T* r, T* tmp, T* w, int* fault, const int* done) {
-    SweepArgs<T> a;
-    a.rD = rD;
-    a.r = r;
-    a.coef = ef;
-    const int n = F.offH[F.nLev];
-    launch_free<SW_FWD, false, T>(st, F, n, a, nullptr, tmp, fault, done);  // tmp: forward result
+// Both DIC/DILU substitutions over one chunk, w staying in LDS between them.
+template <int PF, int WAVES, class T>
+__global__ __launch_bounds__(WAVES* WAVE) void k_dilu_one(SweepPlan F, SweepPlan B, SweepArgs<T> a, const T* eb,
+                                                          const int* done) {
+    if (done && *done) return;
+    extern __shared__ double sweepLds[];
+    T* xs = reinterpret_cast<T*>(sweepLds);
+    __shared__ int cnt[2];
+    if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
+    sweep_fill<SW_FWD>(F, a, xs, 0, F.n, 0, 0);
+    __syncthreads();
+    sweep_steps<SW_FWD, false, PF, WAVES, T>(F, a, xs, &cnt[0], 0, 0, F.nSteps, 0);
+    __syncthreads();
     a.coef = eb;
-    launch_free<SW_BWD, true, T>(st, B, n, a, tmp, w, fault, done);  // every cell, level 0 included
+    sweep_steps<SW_BWD, false, PF, WAVES, T>(B, a, xs, &cnt[1], 0, 0, B.nSteps, 0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < F.n; i += blockDim.x) a.x[i] = xs[i];
 }
-template void launch_dilu_apply_free<double>(hipStream_t, const LevelEll&, const LevelEll&, const double*,
-                                             const double*, const double*, const double*, double*, double*, int*,
-                                             const int*);
-template void launch_dilu_apply_free<float>(hipStream_t, const LevelEll&, const LevelEll&, const float*, const float*,
-                                            const float*, const float*, float*, float*, int*, const int*);
 
-// Per-entry coefficients of a LevelEll from their source array: out[e] = from[src[e]]
+// Mailbox values ← sentinel and tickets ← 0.
+template <class T> __global__ void k_sweep_prepare(size_t m, T* mail, int* tickets, const int* done) {
+    if (done && *done) return;
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < m) mail[i] = Sentinel<T>::value();
+    if (i < SWEEP_TICKETS) tickets[i] = 0;
+}
+
+template <class T> void launch_sweep_prepare(hipStream_t st, size_t m, T* mail, int* tickets, const int* done) {
+    hipLaunchKernelGGL(k_sweep_prepare<T>, sweep_grid(std::max<size_t>(m, SWEEP_TICKETS)), dim3(SWEEP_THREADS), 0, st,
+                       m, mail, tickets, done);
+}
+template void launch_sweep_prepare<double>(hipStream_t, size_t, double*, int*, const int*);
+template void launch_sweep_prepare<float>(hipStream_t, size_t, float*, int*, const int*);
+
+// Launch with dynamic LDS beyond the default limit.
+template <auto Kernel, class... A>
+static void launch_lds(int blocks, int threads, size_t lds, hipStream_t st, A... args) {
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            int((SWEEP_MAX_SLOTS + 1) * sizeof(double)));
+    (void)attr;
+    hipLaunchKernelGGL(Kernel, dim3(blocks), dim3(threads), lds, st, args...);
+}
+
+// Rows of at most 8 entries (mesh cells) run 16 wavefronts; longer ones (coarse GAMG
+// levels) 8, whose registers hold up to 24 entries each (20 with the values of other
+// chunks beside them; entries past that cost a memory round trip inside the dependence:
+// a level of 5,739 cells with up to 24 took 365 µs with 16 held and 220 with 20).
+template <int OP, bool BACK, class T>
+static void launch_sweep_t(hipStream_t st, const SweepPlan& P, const SweepArgs<T>& a, int sweeps, const int* done) {
+    const size_t lds = (size_t(P.maxSlots) + 1) * sizeof(T);
+    if (P.nChunks > 1) {
+        if (P.maxWidth <= 8)
+            launch_lds<k_sweep_chunks<OP, BACK, 8, 16, T>>(P.nChunks * sweeps, 16 * WAVE, lds, st, P, a, sweeps, done);
+        else if (P.maxWidth <= 12)
+            launch_lds<k_sweep_chunks<OP, BACK, 12, 8, T>>(P.nChunks * sweeps, 8 * WAVE, lds, st, P, a, sweeps, done);
+        else
+            launch_lds<k_sweep_chunks<OP, BACK, 20, 8, T>>(P.nChunks * sweeps, 8 * WAVE, lds, st, P, a, sweeps, done);
+    } else {
+        if (P.maxWidth <= 8)
+            launch_lds<k_sweep_one<OP, 8, 16, T>>(1, 16 * WAVE, lds, st, P, a, done);
+        else
+            launch_lds<k_sweep_one<OP, 24, 8, T>>(1, 8 * WAVE, lds, st, P, a, done);
+    }
+}
+
+template <class T>
+void launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
+                  const int* done) {
+    if (P.n <= 0) return;
+    switch (op) {
+    case SW_GS:
+        if (backward) launch_sweep_t<SW_GS, true, T>(st, P, a, sweeps, done);
+        else launch_sweep_t<SW_GS, false, T>(st, P, a, sweeps, done);
+        break;
+    case SW_FWD: launch_sweep_t<SW_FWD, false, T>(st, P, a, sweeps, done); break;
+    case SW_BWD: launch_sweep_t<SW_BWD, true, T>(st, P, a, sweeps, done); break;
+    default:
+        if constexpr (std::is_same_v<T, double>) launch_sweep_t<SW_FAC, false, T>(st, P, a, sweeps, done);
+        break;
+    }
+}
+template void launch_sweep<double>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<double>&, int, const int*);
+template void launch_sweep<float>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<float>&, int, const int*);
+
+template <class T>
+void launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B, const SweepArgs<T>& a, const T* eb,
+                     const int* done) {
+    if (F.n <= 0) return;
+    const size_t lds = (size_t(F.n) + 1) * sizeof(T);
+    if (std::max(F.maxWidth, B.maxWidth) <= 8)
+        launch_lds<k_dilu_one<8, 16, T>>(1, 16 * WAVE, lds, st, F, B, a, eb, done);
+    else
+        launch_lds<k_dilu_one<24, 8, T>>(1, 8 * WAVE, lds, st, F, B, a, eb, done);
+}
+template void launch_dilu_one<double>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<double>&,
+                                      const double*, const int*);
+template void launch_dilu_one<float>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<float>&,
+                                     const float*, const int*);
+
+// Entries of the DIC/DILU factor and substitutions, a wavefront per step. src[e] is a
+// face with its side of the row's own cell (f << 1 | side, 0: upper, 1: lower holds the
+// row's coefficient). rD null: A_lu·A_ul (factor), else rD_row times the row's own.
+__global__ void k_dilu_entries(SweepPlan P, const int* src, const double* upper, const double* lower, const double* rD,
+                               double* out) {
+    const int s = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x % WAVE;
+    if (s >= P.nSteps) return;
+    const SweepStep d = P.steps[s];
+    const int rows = d.rowsNeed & ((1 << SWEEP_ROWS_BITS) - 1);
+    if (lane >= rows) return;
+    const double r = rD ? rD[P.cell[d.pos + lane]] : 0.0;
+    for (int k = 0; k < d.width; ++k) {
+        const int e = d.base + k * rows + lane, q = src[e], f = q >> 1;
+        double v = 0.0;
+        if (q >= 0) {
+            const double own = (q & 1) ? lower[f] : upper[f];
+            v = rD ? r * own : ((q & 1) ? upper[f] : lower[f]) * own;
+        }
+        out[e] = v;
+    }
+}
+void launch_dilu_entries(hipStream_t st, const SweepPlan& P, const int* src, const double* upper, const double* lower,
+                         const double* rD, double* out) {
+    if (P.nSteps > 0)
+        hipLaunchKernelGGL(k_dilu_entries, sweep_grid(size_t(P.nSteps) * WAVE), dim3(SWEEP_THREADS), 0, st, P, src,
+                           upper, lower, rD, out);
+}
+
+// Per-entry coefficients of a sweep plan from their source array: out[e] = from[src[e]]
 // (0 for padding, src < 0).
 template <class T>
 __global__ void k_gather_entries(size_t n, const int* src, const T* from, T* out) {

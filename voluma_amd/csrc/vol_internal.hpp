@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "sweep_plan.hpp"
+
 namespace vol {
 
 constexpr int WAVE = 64;   // CDNA wavefront
@@ -524,105 +526,48 @@ void launch_boundary_values(hipStream_t st, const FvcGeom& G, int nc, const int*
                             const double* c, double* out);
 void launch_copy_strided(hipStream_t st, long long n, const double* src, int ss, double* dst, int ds, double scale);
 
-// ------------------------------------------------------------------ level-scheduled sweeps
-// Lower / upper neighbour lists of the cells (device arrays). Lower list of cell u: neighbours l < u in ascending (l, face) order;
-// upper list of cell l: neighbours u > l in descending (u, face) order; src = face << 1 |
-// side of the list's own row (0: upper[face], 1: lower[face]).
-struct SweepView {
-    const int* lowOff = nullptr;
-    const int* lowCol = nullptr;
-    const int* lowSrc = nullptr;
-    const int* upOff = nullptr;
-    const int* upCol = nullptr;
-    const int* upSrc = nullptr;
+// ------------------------------------------------------------------ triangular sweeps
+// Device view of a SweepPlanHost.
+struct SweepPlan {
+    const int* chunkOff = nullptr;
+    const int* stepOff = nullptr;
+    const SweepStep* steps = nullptr;
+    const int* cell = nullptr;
+    const int* col = nullptr;
+    const int* col2 = nullptr;  // null: single sweeps only
+    const int* haloOff = nullptr;
+    const int* halo = nullptr;
+    int n = 0, nChunks = 0, nSteps = 0, maxSlots = 0, maxWidth = 0;
 };
-// A level order prepared for launching (DIC/DILU factor): cells of level L are
-// perm[off[L] .. off[L+1]); groups [grp[g], grp[g+1]) of consecutive levels are either
-// a run of levels of at most SWEEP_RUN_MAX cells each, swept by one workgroup in one
-// launch (grpRun[g] = 1), or a single larger level with a grid launch.
-constexpr int SWEEP_RUN_MAX = 1024;
-struct LevelSched {
-    const int* perm = nullptr;   // device
-    const int* offD = nullptr;   // device level offsets (nLev + 1)
-    const int* offH = nullptr;   // host copy of the offsets
-    int nLev = 0;
-    const int* grpH = nullptr;   // host: nGrp + 1 group boundaries (level indices)
-    const char* grpRunH = nullptr;
-    int nGrp = 0;
-};
-// DIC/DILU factor over the forward levels: dF, rD = 1/dF per cell, pf per lower-list
-// entry, pb per upper-list entry
-void launch_dilu_factor(hipStream_t st, const SweepView& s, const LevelSched& fwd, const double* diag,
-                        const double* upper, const double* lower, double* dF, double* rD, double* pf, double* pb);
-// Level-ordered ELL rows of a triangular sweep: positions in level order, the cell at
-// each position, and entry k of row t of level L at base[L] + k·size_L + t (neighbour
-// col, −1 padding; the coefficients come per matrix, in the same layout). Groups
-// [grp[g], grp[g+1]) of levels are one level of more than 1024 cells swept by a grid
-// (ELL_GRID), or a run of at most ELL_RUN_LEVELS consecutive levels swept by one
-// workgroup, a row per thread, whose levels hold at most 256, 512 or 1024 cells
-// (ELL_RUN256 < ELL_RUN512 < ELL_RUN1024: the larger class covers the smaller).
-// A run keeps x in LDS: every cell its rows write or read has a slot there (at most
-// RUN_LDS_CELLS, runCells[runOff[g] ..] in slot order), filled from x when the run
-// starts and updated in place; entries of run rows hold the neighbour's slot instead of
-// its cell, and slot[pos] is the slot of the row's own cell.
-constexpr int ELL_GRID = 0, ELL_RUN256 = 1, ELL_RUN512 = 2, ELL_RUN1024 = 3;
-constexpr int ELL_RUN_LEVELS = 2048;
-constexpr int RUN_LDS_CELLS = 16384;
-struct LevelEll {
-    const int* cell = nullptr;    // device
-    const int* slot = nullptr;    // device: per position, the LDS slot of its cell (runs)
-    const int* runCells = nullptr;  // device: cells of each run's LDS slots
-    const int* runOffH = nullptr;   // host: per group, first entry in runCells
-    const int* runCntH = nullptr;   // host: per group, number of slots (0: grid)
-    const int* col = nullptr;     // device
-    const int* offD = nullptr;    // device: nLev + 1 level offsets
-    const int* widthD = nullptr;  // device: entries per row of each level
-    const int* baseD = nullptr;   // device: first entry of each level
-    const int* offH = nullptr;    // host copies
-    const int* widthH = nullptr;
-    const int* baseH = nullptr;
-    int nLev = 0;
-    const int* grpH = nullptr;
-    const char* grpKindH = nullptr;
-    int nGrp = 0;
-    // sync-free sweeps: per wavefront (64 rows of one level) its level and first row
-    const int2* waves = nullptr;  // device
-    int nWaves = 0;
-    // per level, the first runCells entry of the LDS run it belongs to (−1: none): a run
-    // level's entries hold LDS slots, cell = runCells[runBase + slot]
-    const int* runBaseD = nullptr;  // device
-};
-enum SweepOp { SW_GS = 0, SW_FWD = 1, SW_BWD = 2 };
+constexpr int SWEEP_MAX_SWEEPS = 4;  // of one launch over several chunks
+enum SweepOp { SW_GS = 0, SW_FWD = 1, SW_BWD = 2, SW_FAC = 3 };
 template <class T> struct SweepArgs {
-    const T* coef = nullptr;  // per entry (LevelEll layout)
-    const T* b = nullptr;     // SW_GS
-    const T* diag = nullptr;  // SW_GS
+    const T* coef = nullptr;  // per entry of the plan
+    const T* b = nullptr;     // SW_GS: right-hand side; SW_FWD: r
+    const T* diag = nullptr;  // SW_GS, SW_FAC
     const T* rD = nullptr;    // SW_FWD
-    const T* r = nullptr;     // SW_FWD
-    T* x = nullptr;           // updated in place (w for DILU)
+    T* x = nullptr;           // result; SW_GS, SW_BWD: updated in place
+    bool zero = false;        // SW_GS: x is taken as zero
+    // several chunks only: the mailbox (n values per sweep) and the chunk ticket of this
+    // launch, both made ready by launch_sweep_prepare; the flag of timed-out waits
+    T* mail = nullptr;
+    int* ticket = nullptr;
+    int* fault = nullptr;
 };
-// Sync-free forms of the sweeps (one launch per sweep, no level barriers): a row waits
-// for each neighbour whose new value it reads until that value is published in xNew,
-// which starts filled with a sentinel; values it reads old come from xOld (GS: the
-// neighbours on the other side; backward DILU: its own forward value). The arithmetic of
-// every row is the level-scheduled one, so the bits are too. fault (two device ints):
-// [0] set when a wait ran past its spin limit (the sweep's results are then void), [1]
-// the launch's work counter.
+// m mailbox values and SWEEP_TICKETS tickets made ready
+constexpr int SWEEP_TICKETS = 2;
+template <class T> void launch_sweep_prepare(hipStream_t st, size_t m, T* mail, int* tickets, const int* done);
+// `sweeps` sweeps over several chunks; a one-chunk plan holds its whole schedule (sweeps = 1)
 template <class T>
-void launch_gs_sweep_free(hipStream_t st, const LevelEll& E, bool backward, const T* coef, const T* diag, const T* b,
-                          const T* xOld, T* xNew, int* fault, const int* done);
+void launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
+                  const int* done);
+// Forward and backward substitution of one-chunk plans in one launch (a.coef: forward entries)
 template <class T>
-void launch_dilu_apply_free(hipStream_t st, const LevelEll& F, const LevelEll& B, const T* rD, const T* ef,
-                            const T* eb, const T* r, T* tmp, T* w, int* fault, const int* done);
-// w = M⁻¹ r of DIC/DILU: forward then backward substitution (ef, eb: rD·A products per
-// entry of F and B), every launch a no-op once *done
-template <class T>
-void launch_dilu_apply(hipStream_t st, const LevelEll& F, const LevelEll& B, const T* rD, const T* ef, const T* eb,
-                       const T* r, T* w, const int* done);
-// one Gauss–Seidel pass over the levels of E (forward or backward order)
-template <class T>
-void launch_gs_sweep(hipStream_t st, const LevelEll& E, const T* coef, const T* diag, const T* b, T* x,
+void launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B, const SweepArgs<T>& a, const T* eb,
                      const int* done);
+// Entries of the DIC/DILU factor (rD null) and substitutions in a plan's layout
+void launch_dilu_entries(hipStream_t st, const SweepPlan& P, const int* src, const double* upper, const double* lower,
+                         const double* rD, double* out);
 // out[e] = from[src[e]] (0 where src[e] < 0)
 template <class T> void launch_gather_entries(hipStream_t st, size_t n, const int* src, const T* from, T* out);
 // coarsest solve with the LU factors in the reference's row order (Gauss–Seidel V-cycle)
