@@ -9,6 +9,7 @@ import pytest
 
 import voluma_amd as va
 from helpers import SMALL_MESHES, load_json, load_small, sha
+from voluma_amd import mesh as M
 from voluma_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +120,30 @@ def test_full_size_momentum_tet70(ctx):
             p2 = va.solve_ldu(A, b, x2, va.SolverControls("PBiCGStab", "diagonal", 1e-6, 0.0, 1000, precision=prec))
             assert p2.converged
             assert np.linalg.norm(x2 - x) <= 1e-5 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("face", [None, 0, 262143, 262144, -1])
+def test_single_non_orthogonal_face_is_found(ctx, face):
+    """The correction is switched on by any one corrected face, wherever the scan of the
+    faces (1024 blocks of 256, then on) meets it, and only that face's flux is corrected:
+    γ|S| corr·∇ψ with ∇ψ = (1, 0, 0) of ψ = x on a uniform box."""
+    m = M.box(50)
+    geo = m.geometry()
+    lm, A = _matrix(ctx, m)
+    ni = m.n_internal
+    corr = np.zeros_like(geo["corr"])
+    f = None if face is None else face % ni
+    if f is not None:
+        corr[f] = (1e-3, 0.0, 0.0)
+    bc = np.ones(m.n_boundary, np.int32)  # boundary values of ψ, so that the gradient is exact
+    psi, bv = geo["C"][:, 0].copy(), geo["Cf"][ni:, 0].copy()
+    A.fvm_reset()
+    A.fvm_laplacian(+1, geo["magSf"], geo["ndc"], bc, bv, gamma=2.0,
+                    nonorth={"psi": psi, "w": geo["w"], "Sf": geo["Sf"], "corr": corr, "V": geo["V"]})
+    ffc = A.fvm_get()["ffc"]
+    want = np.zeros(m.n_faces)
+    if f is not None:
+        want[f] = 2.0 * geo["magSf"][f] * 1e-3
+    assert np.allclose(ffc, want, rtol=1e-9, atol=0.0)  # 64-bit sums of six terms: ~1e-13
+    A.close()
+    lm.close()
