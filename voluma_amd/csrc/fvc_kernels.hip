@@ -136,27 +136,81 @@ __global__ void k_fvc_interp_boundary(FvcGeom G, const double* c, const double* 
 }
 
 // ---------------------------------------------------------------- gradients
+// The internal faces of a cell held in registers, for rows of exactly W slots (tets 4,
+// hexes 6): every address is known from the slots, so all loads of a kind go out together
+// instead of one face after the other, and both passes of a least-squares gradient read
+// them once. e < 0: padding (face 0 and the cell itself stand in, the value is not used).
+// 2,058,000 tets: least squares 118 → 71 µs (scalar) and 249 → 120 (vector), Gauss with
+// skew correction 249 → 139, divergence 36 → 28, i.e. 3.5–4.5 TB/s of what the gathers
+// touch; the face-wise kernels (flux 113, interpolate 58) run at the copy rate.
+template <int W> struct CellFaces {
+    int e[W], f[W], other[W];
+    __device__ __forceinline__ CellFaces(const FvcGeom& G, int cell) {
+        const int s0 = (cell / WAVE) * WAVE * W + cell % WAVE;
+#pragma unroll
+        for (int k = 0; k < W; ++k) e[k] = G.S.src[s0 + k * WAVE];
+#pragma unroll
+        for (int k = 0; k < W; ++k) other[k] = G.S.col[s0 + k * WAVE];
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            f[k] = e[k] < 0 ? 0 : e[k] >> 1;
+            other[k] = e[k] < 0 ? cell : other[k];
+        }
+    }
+};
+
 // Weighted least squares (Fvc.h:134-206) per cell: Σ d⊗d/|d|² over its faces, the
 // inverse, then Σ (G·d/|d|²)·Δφ with Δφ = φ_N − φ_P of each internal face and the
 // boundary constraints (value faces: d, φ_b − φ_P; others: the zero normal gradient).
-template <int NC>
-__global__ void k_fvc_grad_ls(FvcGeom G, const double* c, const int* bFix, const double* bVal, double* out) {
+// W > 0: rows of exactly W slots (CellFaces), else any layout.
+template <int NC, int W>
+__global__ __launch_bounds__(FVC_THREADS) void k_fvc_grad_ls(FvcGeom G, const double* c, const int* bFix, const double* bVal, double* out) {
     const int cell = blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= G.n) return;
-    int s0, width, stride;
-    row_span(G.S, cell, s0, width, stride);
     double dd[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) dd[k] = 0.0;
-    for (int k = 0; k < width; ++k) {
-        const int e = G.S.src[s0 + k * stride];
-        if (e < 0) continue;
-        const double* v = G.d + 3 * (e >> 1);
-        const double s = 1.0 / dot3(v, v);
+    int s0 = 0, width = 0, stride = 0;
+    constexpr int H = W > 0 ? W : 1;
+    double vf[H][3], sf[H], dphf[H][NC];
+    int ef[H];
+    if constexpr (W > 0) {
+        const CellFaces<W> F(G, cell);
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
+        for (int k = 0; k < W; ++k)
 #pragma unroll
-            for (int b = 0; b < 3; ++b) dd[3 * a + b] += (v[a] * v[b]) * s;
+            for (int q = 0; q < 3; ++q) vf[k][q] = G.d[3 * size_t(F.f[k]) + q];
+        double own[NC];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) own[q] = c[NC * size_t(cell) + q];
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+#pragma unroll
+            for (int q = 0; q < NC; ++q) dphf[k][q] = c[NC * size_t(F.other[k]) + q];
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            ef[k] = F.e[k];
+#pragma unroll
+            for (int q = 0; q < NC; ++q) dphf[k][q] = (ef[k] & 1) ? own[q] - dphf[k][q] : dphf[k][q] - own[q];
+            sf[k] = 1.0 / dot3(vf[k], vf[k]);
+            if (ef[k] >= 0)
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) dd[3 * a + b] += (vf[k][a] * vf[k][b]) * sf[k];
+        }
+    } else {
+        row_span(G.S, cell, s0, width, stride);
+        for (int k = 0; k < width; ++k) {
+            const int e = G.S.src[s0 + k * stride];
+            if (e < 0) continue;
+            const double* v = G.d + 3 * (e >> 1);
+            const double s = 1.0 / dot3(v, v);
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int b = 0; b < 3; ++b) dd[3 * a + b] += (v[a] * v[b]) * s;
+        }
     }
     for (int k = G.bOff[cell]; k < G.bOff[cell + 1]; ++k) {
         const int bf = G.bList[k];
@@ -174,6 +228,13 @@ __global__ void k_fvc_grad_ls(FvcGeom G, const double* c, const int* bFix, const
     double g[3 * NC];
 #pragma unroll
     for (int k = 0; k < 3 * NC; ++k) g[k] = 0.0;
+    if constexpr (W > 0) {
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            const double vw[3] = {vf[k][0] * sf[k], vf[k][1] * sf[k], vf[k][2] * sf[k]};
+            if (ef[k] >= 0) ls_add<NC>(Gi, vw, dphf[k], g);
+        }
+    }
     for (int k = 0; k < width; ++k) {
         const int slot = s0 + k * stride;
         const int e = G.S.src[slot];
@@ -210,14 +271,56 @@ __global__ void k_fvc_grad_ls(FvcGeom G, const double* c, const int* bFix, const
 // Gauss gradient of a scalar (Fvc.h:213-222, GaussLinear; 223-259, GaussSkew with the
 // least-squares gradient gls): Σ S_f ψ_f over the cell's faces (owner +, neighbour −,
 // boundary +) · (1/V).
-template <bool SKEW>
-__global__ void k_fvc_grad_gauss(FvcGeom G, const double* psi, const double* gls, const int* bFix,
+template <bool SKEW, int W>
+__global__ __launch_bounds__(FVC_THREADS) void k_fvc_grad_gauss(FvcGeom G, const double* psi, const double* gls, const int* bFix,
                                  const double* bVal, double* out) {
     const int cell = blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= G.n) return;
-    int s0, width, stride;
-    row_span(G.S, cell, s0, width, stride);
+    int s0 = 0, width = 0, stride = 0;
     double g[3] = {0.0, 0.0, 0.0};
+    if constexpr (W > 0) {
+        const CellFaces<W> F(G, cell);
+        double w[W], S[W][3], sk[SKEW ? W : 1][3], gn[SKEW ? W : 1][3], pn[W], gp[3] = {0.0, 0.0, 0.0};
+        const double pp = psi[cell];
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            w[k] = G.w[F.f[k]];
+            pn[k] = psi[F.other[k]];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) S[k][q] = G.Sf[3 * size_t(F.f[k]) + q];
+        }
+        if constexpr (SKEW) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) gp[q] = gls[3 * size_t(cell) + q];
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    sk[k][q] = G.skew[3 * size_t(F.f[k]) + q];
+                    gn[k][q] = gls[3 * size_t(F.other[k]) + q];
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            const bool nei = F.e[k] & 1;  // the cell is the face's neighbour
+            double phif = w[k] * (nei ? pn[k] : pp) + (1.0 - w[k]) * (nei ? pp : pn[k]);
+            if constexpr (SKEW) {
+                double gP[3], gN[3], t;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    gP[q] = nei ? gn[k][q] : gp[q];
+                    gN[q] = nei ? gp[q] : gn[k][q];
+                }
+                skew_term<1>(sk[k], w[k], gP, gN, &t);
+                phif = phif + t;
+            }
+            if (F.e[k] >= 0)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) g[q] = nei ? g[q] - S[k][q] * phif : g[q] + S[k][q] * phif;
+        }
+    } else {
+        row_span(G.S, cell, s0, width, stride);
+    }
     for (int k = 0; k < width; ++k) {
         const int slot = s0 + k * stride;
         const int e = G.S.src[slot];
@@ -268,15 +371,32 @@ __global__ void k_fvc_grad_gauss(FvcGeom G, const double* psi, const double* gls
 // ---------------------------------------------------------------- div, surfaceIntegrate
 // Σ F over the cell's faces (owner +, neighbour −, boundary +); DIV: / V (Fvc.h:294-305),
 // else · (1/V) (surfaceIntegrate, Fvc.h:307-318).
-template <int NC, bool DIV>
-__global__ void k_fvc_integrate(FvcGeom G, const double* F, double* out) {
+template <int NC, bool DIV, int W>
+__global__ __launch_bounds__(FVC_THREADS) void k_fvc_integrate(FvcGeom G, const double* F, double* out) {
     const int cell = blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= G.n) return;
-    int s0, width, stride;
-    row_span(G.S, cell, s0, width, stride);
+    int s0 = 0, width = 0, stride = 0;
     double r[NC];
 #pragma unroll
     for (int q = 0; q < NC; ++q) r[q] = 0.0;
+    if constexpr (W > 0) {
+        s0 = (cell / WAVE) * WAVE * W + cell % WAVE;
+        int e[W];
+        double v[W][NC];
+#pragma unroll
+        for (int k = 0; k < W; ++k) e[k] = G.S.src[s0 + k * WAVE];
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+#pragma unroll
+            for (int q = 0; q < NC; ++q) v[k][q] = F[NC * size_t(e[k] < 0 ? 0 : e[k] >> 1) + q];
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+            if (e[k] >= 0)
+#pragma unroll
+                for (int q = 0; q < NC; ++q) r[q] = (e[k] & 1) ? r[q] - v[k][q] : r[q] + v[k][q];
+    } else {
+        row_span(G.S, cell, s0, width, stride);
+    }
     for (int k = 0; k < width; ++k) {
         const int e = G.S.src[s0 + k * stride];
         if (e < 0) continue;
@@ -345,34 +465,51 @@ void launch_fvc_interpolate(hipStream_t st, const FvcGeom& G, int nc, const doub
     }
 }
 
+// f(W) with W the row length held in registers: tets (4) and hexes (6) whose level 0 is
+// plain ELL of that width, 0 for any other layout.
+template <class F> static void by_width(const FvcGeom& G, F&& f) {
+    if (G.S.csrG == 0 && G.S.ellWidth == 4 && G.nf > 0) f(std::integral_constant<int, 4>{});
+    else if (G.S.csrG == 0 && G.S.ellWidth == 6 && G.nf > 0) f(std::integral_constant<int, 6>{});
+    else f(std::integral_constant<int, 0>{});
+}
+
 void launch_fvc_grad_ls(hipStream_t st, const FvcGeom& G, int nc, const double* c, const int* bFix,
                         const double* bVal, double* out) {
     if (G.n <= 0) return;
-    if (nc == 1)
-        hipLaunchKernelGGL(k_fvc_grad_ls<1>, fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, c, bFix, bVal, out);
-    else
-        hipLaunchKernelGGL(k_fvc_grad_ls<3>, fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, c, bFix, bVal, out);
+    by_width(G, [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        if (nc == 1)
+            hipLaunchKernelGGL((k_fvc_grad_ls<1, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, c, bFix, bVal, out);
+        else
+            hipLaunchKernelGGL((k_fvc_grad_ls<3, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, c, bFix, bVal, out);
+    });
 }
 
 void launch_fvc_grad_gauss(hipStream_t st, const FvcGeom& G, bool skew, const double* psi, const double* gls,
                            const int* bFix, const double* bVal, double* out) {
     if (G.n <= 0) return;
-    if (skew)
-        hipLaunchKernelGGL(k_fvc_grad_gauss<true>, fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, psi, gls, bFix, bVal,
-                           out);
-    else
-        hipLaunchKernelGGL(k_fvc_grad_gauss<false>, fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, psi, gls, bFix, bVal,
-                           out);
+    by_width(G, [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        if (skew)
+            hipLaunchKernelGGL((k_fvc_grad_gauss<true, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, psi, gls, bFix,
+                               bVal, out);
+        else
+            hipLaunchKernelGGL((k_fvc_grad_gauss<false, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, psi, gls,
+                               bFix, bVal, out);
+    });
 }
 
 void launch_fvc_integrate(hipStream_t st, const FvcGeom& G, int nc, bool div, const double* F, double* out) {
     if (G.n <= 0) return;
-    if (div)
-        hipLaunchKernelGGL((k_fvc_integrate<1, true>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
-    else if (nc == 1)
-        hipLaunchKernelGGL((k_fvc_integrate<1, false>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
-    else
-        hipLaunchKernelGGL((k_fvc_integrate<3, false>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
+    by_width(G, [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        if (div)
+            hipLaunchKernelGGL((k_fvc_integrate<1, true, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
+        else if (nc == 1)
+            hipLaunchKernelGGL((k_fvc_integrate<1, false, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
+        else
+            hipLaunchKernelGGL((k_fvc_integrate<3, false, W>), fvc_grid(G.n), dim3(FVC_THREADS), 0, st, G, F, out);
+    });
 }
 
 void launch_fvc_flux(hipStream_t st, const FvcGeom& G, const double* U, const double* grad, const int* bFix,
