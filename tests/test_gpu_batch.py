@@ -238,3 +238,29 @@ def test_batch_graph_replay_matches_eager(ctx, small_batch, prec):
             os.environ.pop("VOLUMA_BATCH_GRAPH", None)
         else:
             os.environ["VOLUMA_BATCH_GRAPH"] = old
+
+
+@pytest.mark.parametrize("prec", [va.FP64, va.MIXED])
+@pytest.mark.parametrize("pre,post", [(1, 1), (1, 3), (2, 1), (3, 2)])
+def test_batch_vcycle_sweeps_match_single_system_solver(ctx, pre, post, prec):
+    """Sweep counts of the batched V-cycle (one pre-sweep kept with the residual or the
+    pre-smoothed x, the prolongation pushed into either) over systems whose coarsest levels
+    lie at different depths: the iterations of vol_solve within 1 (other reduction trees)
+    and its solution within 1e-8 at residual 1e-10, FP64 and mixed."""
+    specs = W.batch_specs(n_systems=5, seed=23, n_min=90, n_max=9000, median=900)
+    B, b, meshes = W.batch_system(ctx, specs)
+    assert len(set(B.levels())) > 1
+    ctl = _ctl(precision=prec, gamgPreSweeps=pre, gamgPostSweeps=post)
+    for _ in range(2):  # the second solve starts from the first one's buffers
+        x = np.zeros(B.n_total)
+        perf = B.solve(b, x, ctl)
+    for s, m in enumerate(meshes):
+        lm = va.LduMesh(ctx, m.n_cells, m.owner[: m.n_internal], m.neighbour, m.agglomeration_weights())
+        A = va.LduMatrix(lm, B.diag_h[B.cell_off[s]: B.cell_off[s + 1]], B.upper_h[B.face_off[s]: B.face_off[s + 1]])
+        xs = np.zeros(m.n_cells)
+        ps = va.solve_ldu(A, _slice(B, b, s), xs, ctl)
+        assert perf[s].converged and abs(ps.iterations - perf[s].iterations) <= 1, (s, ps.iterations, perf[s].iterations)
+        assert np.linalg.norm(_slice(B, x, s) - xs) <= 1e-8 * np.linalg.norm(xs), s
+        A.close()
+        lm.close()
+    B.close()

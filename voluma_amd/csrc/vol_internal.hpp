@@ -633,10 +633,20 @@ void launch_bmix(hipStream_t st, int op, const BatchRed& R, const DevScalars* S,
                  float* w2, float* z, double* x, const float* e);
 // Dense assembly + no-pivot LU of every system's coarsest level (one workgroup each).
 void launch_bcoarse_factor(hipStream_t st, const CoarseDesc* D, int nSys, double* lu, double* luT, int* status);
+// Pushed prolongation of the coarsest solves: a system whose coarsest level is l also adds
+// its x to z[l] over the members list[l][off[l][row] ..] of its rows (z[l] null: it does not).
+constexpr int BATCH_PUSH_LEVELS = 16;
+template <class T> struct BatchPush {
+    T* z[BATCH_PUSH_LEVELS] = {};
+    const int* off[BATCH_PUSH_LEVELS] = {};
+    const int* list[BATCH_PUSH_LEVELS] = {};
+};
 // Coarsest substitutions: r and x of system s live at rLev[D.level] + D.rowBase.
 void launch_bcoarse_solve(hipStream_t st, const CoarseDesc* D, int nSys, int maxN, const double* lu,
-                          const double* luT, const double* const* rLev, double* const* xLev, const DevScalars* S);
+                          const double* luT, const double* const* rLev, double* const* xLev, const DevScalars* S,
+                          const BatchPush<double>& push);
 void launch_bcoarse_solve32(hipStream_t st, const CoarseDesc* D, int nSys, int maxN, const double* lu,
-                            const double* luT, const float* const* rLev, float* const* xLev, const DevScalars* S);
+                            const double* luT, const float* const* rLev, float* const* xLev, const DevScalars* S,
+                            const BatchPush<float>& push);
 
 }  // namespace vol
