@@ -80,3 +80,51 @@ def test_sweeps_bit_exact_vs_oracle(ctx, name):
                                                                   sums=va.SUMS_EXACT))
         assert p.iterations == po["iterations"] and p.finalResidual == po["finalResidual"], (solver, sweeps)
         assert np.array_equal(x, xo), (solver, sweeps)
+
+
+def test_values_before_the_sweep_past_the_halo(ctx):
+    """Enough chunks of long scattered rows that a chunk's neighbours do not fit its LDS:
+    what is left of them is read where it lies, from x and from zero."""
+    n = 100_003
+    a, b = _band(n, 16, n, 8)
+    keep = a < b
+    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
+    own, nei = (e // n).astype(np.int32), (e % n).astype(np.int32)
+    rng = np.random.default_rng(10)
+    u = -rng.uniform(0.5, 1.5, e.size)
+    d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
+    rhs, x0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    lm = va.LduMesh(ctx, n, own, nei)
+    om = O.LduMesh(n, own, nei)
+    A = va.LduMatrix(lm, d, u)
+    for start in (x0, np.zeros(n)):
+        xo, _ = om.solve(d, u, None, rhs, x0=start, solver="symGaussSeidel", preconditioner="none", tolerance=1e-30,
+                         max_iter=2, mode=O.MODE_EXACT)
+        x = start.copy()
+        va.solve_ldu(A, rhs, x, va.SolverControls("symGaussSeidel", "none", 1e-30, 0.0, 2, sums=va.SUMS_EXACT))
+        assert np.array_equal(x, xo)
+
+
+@pytest.mark.parametrize("name", ["one", "two"])
+@pytest.mark.parametrize("powers", [(0,), (-398, -402, 0, 398, 402), (-800, 0, 180)])
+def test_row_division_over_the_exponent_range(ctx, name, powers):
+    """Rows scaled by powers of two on both sides of the range in which a step divides with
+    the reciprocal, and zero numerators of both signs: the oracle's quotients bit for bit."""
+    n, own, nei = _graph(name)
+    rng = np.random.default_rng(11)
+    s = 2.0 ** rng.choice(powers, n)
+    u, lo = -rng.uniform(0.5, 1.5, own.size), -rng.uniform(0.5, 1.5, own.size)
+    d = (0.1 + np.bincount(own, -u, n) + np.bincount(nei, -lo, n)) * rng.choice([-1.0, 1.0], n)
+    d, u, lo = d * s, u * s[own], lo * s[nei]
+    b = rng.uniform(-1, 1, n) * s
+    b[: n // 2] = 0.0
+    b[: n // 4] = -0.0
+    lm = va.LduMesh(ctx, n, own, nei)
+    om = O.LduMesh(n, own, nei)
+    for sweeps in (1, 3):
+        xo, _ = om.solve(d, u, lo, b, x0=np.zeros(n), solver="GaussSeidel", preconditioner="none", tolerance=1e-300,
+                         max_iter=sweeps, n_sweeps=sweeps, mode=O.MODE_EXACT)
+        x = np.zeros(n)
+        va.solve_ldu(va.LduMatrix(lm, d, u, lo), b, x, va.SolverControls("GaussSeidel", "none", 1e-300, 0.0, sweeps,
+                                                                        nSweeps=sweeps, sums=va.SUMS_EXACT))
+        assert np.array_equal(x, xo) and np.array_equal(np.signbit(x), np.signbit(xo)), sweeps

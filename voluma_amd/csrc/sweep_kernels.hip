@@ -25,15 +25,19 @@
 // earlier ones): whichever workgroups are resident, the earliest unfinished chunk
 // proceeds. A wait past its limit sets *fault and every later wait gives up at once.
 //
-// Measured (MI355X): a dependence through LDS with 8 entries and a division takes 0.30 µs,
-// with 24 entries 0.53 µs (of which the count's hand-over 0.14), a value handed to another
-// workgroup through memory 0.6 µs plus the polling; one CU streams rows at about 30 GB/s.
-// Levels cost 0.5 µs in one chunk and about 1 µs across chunks, against 4–5 µs for a launch
-// per level or a barrier per level in one workgroup. Two Gauss–Seidel sweeps: 373,920 tets
-// (158 levels) 200 µs, 64³ hexes (190 levels) 185 µs; before, 720 and 790. PCG with GAMG
-// smoothed by Gauss–Seidel on these: 231 → 76 and 68 → 21 ms; DIC-PCG on 24,273 hexes 34.2
-// → 8.8 ms; three momentum components by PBiCGStab + DILU on 839,664 tets, assembly and
-// factor included, 29.1 → 8.4 ms.
+// Measured (MI355X): handing a step over through LDS takes 0.14 µs and a value handed to
+// another workgroup through memory 0.6 µs plus the polling; one CU streams rows at about
+// 30 GB/s. Levels cost 0.4 µs in one chunk and about 0.9 µs across chunks, against 4–5 µs
+// for a launch per level or a barrier per level in one workgroup. Two Gauss–Seidel sweeps,
+// forward and backward: 373,920 tets (158 levels) 163 and 149 µs, 64³ hexes (190 levels)
+// 150 and 141. What a step does after its turn counts fully, what a poll does between two
+// looks counts where chunks wait for each other: with a division after the sum, a wait for
+// the stores before the count, an add per LDS address, branches per entry in the polls and
+// the first look at other chunks' values one round trip each, these took 205 and 185 µs
+// (49,000 agglomerated cells of up to 20 entries 310, now 170). PCG with GAMG smoothed by
+// Gauss–Seidel on these meshes: 235 → 57 and 66 → 18 ms; DIC-PCG on 24,273 hexes 34.6 → 7.6
+// ms; three momentum components by PBiCGStab + DILU on 839,664 tets, assembly and factor
+// included, 28.8 → 6.3 ms.
 #include "device_common.hpp"
 #include "vol_internal.hpp"
 
@@ -98,44 +102,77 @@ __device__ __forceinline__ bool given_up(unsigned spins, int* fault) {
 __device__ __forceinline__ int finished(int* cnt) {
     return __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-constexpr int SWEEP_NEAR = 4;  // steps before its turn that a wavefront starts to watch closely
-// LDS-only ordering: waits for LDS accesses, not for the global loads in flight.
-__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+// One more, by one lane (the compiler would first add up over the wavefront's lanes).
+__device__ __forceinline__ void count_step(int* cnt) {
+    using Count = __attribute__((address_space(3))) int;
+    asm volatile("ds_add_u32 %0, %1" ::"v"((Count*)cnt), "v"(1) : "memory");
+}
+// Steps before its turn that a wavefront starts to watch closely: 2, 4, 8 and 12 make two
+// forward sweeps over 373,920 tets 255, 188, 163 and 159 µs.
+constexpr int SWEEP_NEAR = 8;
+// LDS-only ordering. A wavefront's LDS instructions are performed in the order in which it
+// issues them, so its stores are there for whoever reads its later addition to the count:
+// the compiler's order is all that a release needs (waiting for the stores would put one
+// more LDS round trip into every dependence).
+__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local"); }
 __device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
 
-// Steps s0 .. s1 of a chunk from cell c0, its slots of x in xs (the padding slot holds a
-// value whose term is 0), by a workgroup of WAVES wavefronts; *cnt counts finished steps
+// A step's division a / d, the same bits as `/` in fewer dependent operations: everything
+// that needs only d is done before the step's turn. With y = 1/d correctly rounded and e
+// the next digits of 1/d, q = a·y + a·e is off by less than one unit in the last place, and
+// then q + y·(a − d·q) with fused operations is the correctly rounded quotient (Markstein,
+// Computation of elementary functions on the IBM RISC System/6000 processor, 1990), as long
+// as nothing leaves the normal range: exponents past half of it take `/`.
+template <class T> struct RowDivide {
+    static constexpr T HI = sizeof(T) == 8 ? T(0x1p400) : T(0x1p48f), LO = sizeof(T) == 8 ? T(0x1p-400) : T(0x1p-48f);
+    T d, y, e;
+    bool plain;  // wave-uniform
+    __device__ __forceinline__ static bool outside(T v) { return !(fabs(v) <= HI && fabs(v) >= LO); }
+    __device__ __forceinline__ explicit RowDivide(T dg) : d(dg), y(T(1) / dg) {
+        e = fma(-d, y, T(1)) * y;
+        plain = __any(outside(d));
+    }
+    __device__ __forceinline__ T operator()(T a) const {
+        const T z = a * y, q = fma(a, y, a * e);
+        T x = a == T(0) ? z : fma(fma(-d, q, a), y, q);
+        asm volatile("" : "+v"(x));  // computed beside the test, not after it
+        if (__builtin_expect(plain || __any(a != T(0) && outside(a)), 0)) x = a / d;
+        return x;
+    }
+};
+
+// Steps s0 .. s1 of a chunk from cell c0, its slots of x in xs (pad: the padding slot, whose
+// value has a term of 0), by a workgroup of WAVES wavefronts; *cnt counts finished steps
 // from 0. Everything that does not depend on the step's turn is done before it: the row's
-// first PF entries (later ones are loaded after the turn), their LDS addresses, and
-// (MULTI) the values that come by mail. After the turn a step gathers from LDS, subtracts in order, stores
+// first PF entries (later ones are loaded after the turn), their LDS addresses, the
+// division by the diagonal but for its last four operations, and (MULTI) the terms of the
+// values that come by mail. After the turn a step gathers from LDS, subtracts in order, stores
 // and adds to the count; the code for that exists once per number of entry groups, so
 // that every LDS read is in flight before the first is waited for. Lanes past the step's
-// rows repeat its last row and store nothing. MULTI: every value goes to the mailbox of
-// this sweep.
+// rows repeat its last row. MULTI: every value goes to the mailbox of this sweep.
 template <int OP, bool MULTI, int PF, int WAVES, class T>
-__device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<T>& a, T* xs, int* cnt, int c0, int s0,
-                                            int s1, int sweep) {
+__device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<T>& a, T* xs, int pad, int* cnt, int c0,
+                                            int s0, int s1, int sweep) {
     constexpr int GRP = SWEEP_GROUP;
     static_assert(PF % GRP == 0 && PF <= 24);
     const int lane = threadIdx.x % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / WAVE);
-    char* const lds = reinterpret_cast<char*>(xs);
-    const auto value = [&](int byte) { return *reinterpret_cast<const T*>(lds + byte); };
+    using Lds = __attribute__((address_space(3))) T;
+    const unsigned lds = unsigned(uintptr_t((Lds*)xs));  // an LDS address is a 32-bit integer
+    const auto value = [](unsigned addr) { return *(const Lds*)uintptr_t(addr); };
     // past the last step a wavefront loads the last one's data again (unused)
     const auto stepAt = [&](int s) { return P.steps[s < s1 ? s : s1 - 1]; };
     const auto rowOf = [&](const SweepStep& d) {
         const int rows = d.rowsNeed & ((1 << SWEEP_ROWS_BITS) - 1);
         return lane < rows ? lane : rows - 1;
     };
-    // MULTI: where the value of an entry at < 0 lies in the mailbox (from mail), or that
-    // it is x before the first sweep
+    // MULTI: an entry at < 0 is a value in the mailbox (from mail), or x before the sweep
     const T* const mail = MULTI ? a.mail + (sweep - 1) * ptrdiff_t(P.n) : nullptr;
-    const auto initial = [&](int at) { return ~at >= 2 * P.n; };
-    const auto far = [&](int at) {
-        if (!initial(at)) return peek(&mail[~at]);
-        return a.zero ? T(0) : a.x[~at - 2 * P.n];
+    const auto mailed = [&](int at) { return unsigned(~at) < 2u * unsigned(P.n); };
+    const auto initial = [&](int at) {
+        const T x = a.zero ? T(0) : a.x[~at - 2 * P.n];
+        return Sentinel<T>::is(x) ? Sentinel<T>::quiet() : x;
     };
-    const auto missing = [&](int at, T v) { return at < 0 && Sentinel<T>::is(v) && !initial(at); };
     const int* const places = MULTI && sweep > 0 ? P.col2 : P.col;
     int s = s0 + wave;
     if (s >= s1) return;
@@ -170,24 +207,53 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
                 for (int k = g; k < g + GRP; ++k) at[k] = 0;
             }
         }
-        T v[MULTI ? PF : 1];
-        unsigned out = 0;  // which entries are values of other chunks
-        if constexpr (MULTI) {
+        // as loaded, so that no use of them waits between one group's loads and the next
 #pragma unroll
-            for (int k = 0; k < PF; ++k) out |= at[k] < 0 ? 1u << k : 0u;
-            if (__any(out != 0)) {
+        for (int k = 0; k < PF; ++k) asm volatile("" : "+v"(at[k]));
+        unsigned slot = lds + unsigned(c - c0) * unsigned(sizeof(T));
+        if constexpr (OP != SW_GS) acc = value(slot);  // only this step writes it
+        RowDivide<T> div(dg);
+        unsigned addr[PF];
+#pragma unroll
+        for (int k = 0; k < PF; ++k) {
+            addr[k] = lds + unsigned(MULTI && at[k] < 0 ? pad : at[k]) * unsigned(sizeof(T));
+            asm volatile("" : "+v"(addr[k]));
+        }
+        // MULTI: the term of another chunk's value is put into add, and what is gathered for
+        // it is a product of −0 (the padding's); a value in LDS has −0 there, which leaves
+        // its product as it is: the term is the sum of both. Only one product per entry is
+        // left to do when the values arrive.
+        T add[MULTI ? PF : 1];
+        if constexpr (MULTI) {
+            int lowest = 0;
+#pragma unroll
+            for (int k = 0; k < PF; ++k) {
+                lowest = min(lowest, at[k]);
+                add[k] = -T(0);
+            }
+            if (__any(lowest < 0)) {
+                T v[PF], own[PF];
+#pragma unroll
+                for (int k = 0; k < PF; ++k) {
+                    own[k] = at[k] < 0 ? -T(0) : cf[k];
+                    v[k] = OP == SW_FAC ? T(1) : copysign(T(0), -cf[k]);  // cf·v = −0
+                    asm volatile("" : "+v"(own[k]), "+v"(v[k]));
+                }
                 // all of them in one round trip; then, once the turn is near (asking
                 // earlier only loads the fabric), the ones not yet published again,
                 // together, until they are
 #pragma unroll
-                for (int k = 0; k < PF; ++k) {
-                    v[k] = T(0);
-                    if (at[k] < 0) v[k] = far(at[k]);
+                for (int k = 0; k < PF; ++k)
+                    if (mailed(at[k])) v[k] = peek(&mail[~at[k]]);
+                if (__any(lowest < 0 && !mailed(lowest))) {
+#pragma unroll
+                    for (int k = 0; k < PF; ++k)
+                        if (at[k] < 0 && !mailed(at[k])) v[k] = initial(at[k]);
                 }
                 for (unsigned spins = 0;;) {
                     bool miss = false;
 #pragma unroll
-                    for (int k = 0; k < PF; ++k) miss = miss || missing(at[k], v[k]);
+                    for (int k = 0; k < PF; ++k) miss = miss | Sentinel<T>::is(v[k]);
                     if (!__any(miss)) break;
                     if (need - finished(cnt) > SWEEP_NEAR) {
                         __builtin_amdgcn_s_sleep(2);
@@ -197,18 +263,25 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
 #pragma unroll
                     for (int k = 0; k < PF; ++k) {
                         asm volatile("" : "+v"(at[k]));  // no address kept over the loop
-                        if (missing(at[k], v[k])) v[k] = peek(&mail[~at[k]]);
+                        if (Sentinel<T>::is(v[k])) v[k] = peek(&mail[~at[k]]);
                     }
+                }
+#pragma unroll
+                for (int k = 0; k < PF; ++k) {
+                    const T f = OP != SW_FAC || at[k] < 0 ? cf[k] : -T(0);
+                    add[k] = row_term<OP>(f, v[k]);
+                    cf[k] = own[k];
                 }
             }
         }
-#pragma unroll
-        for (int k = 0; k < PF; ++k) at[k] = (MULTI && at[k] < 0 ? 0 : at[k]) * int(sizeof(T));
-        int slot = (c - c0) * int(sizeof(T));
         // keep all of the above before the turn
 #pragma unroll
-        for (int k = 0; k < PF; ++k) asm volatile("" : "+v"(at[k]), "+v"(cf[k]));
-        asm volatile("" : "+v"(slot), "+v"(acc), "+v"(dg));
+        for (int k = 0; k < PF; ++k) {
+            asm volatile("" : "+v"(addr[k]), "+v"(cf[k]));
+            if constexpr (MULTI) asm volatile("" : "+v"(add[k]));
+        }
+        asm volatile("" : "+v"(slot), "+v"(acc));
+        if constexpr (OP == SW_GS) asm volatile("" : "+v"(div.y), "+v"(div.e));
         // the step's turn: every step of the chunk's earlier levels is done
         for (;;) {
             const int got = finished(cnt);
@@ -217,33 +290,25 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
         }
         lds_acquire();
         __builtin_amdgcn_s_setprio(3);  // ahead of the wavefronts that prepare later steps
-        if constexpr (OP != SW_GS) acc = value(slot);
-        const auto rowSum = [&](auto groups, auto mixed) {
+        const auto rowSum = [&](auto groups) {
             constexpr int N = decltype(groups)::value * GRP;
             T xv[N];
 #pragma unroll
-            for (int k = 0; k < N; ++k) xv[k] = value(at[k]);
+            for (int k = 0; k < N; ++k) xv[k] = value(addr[k]);
 #pragma unroll
             for (int k = 0; k < N; ++k) {
-                if constexpr (decltype(mixed)::value) xv[k] = (out >> k) & 1 ? v[k] : xv[k];
-                acc = acc - row_term<OP>(cf[k], xv[k]);
+                if constexpr (!MULTI) acc = acc - row_term<OP>(cf[k], xv[k]);
+                else if constexpr (OP == SW_FAC) acc = acc - (row_term<OP>(cf[k], xv[k]) + add[k]);
+                else acc = acc - fma(cf[k], xv[k], add[k]);
             }
         };
-        const auto rowSums = [&](auto mixed) {
-            const int ng = width / GRP;
-            if (ng >= 6 && PF >= 24) rowSum(std::integral_constant<int, PF >= 24 ? 6 : 1>{}, mixed);
-            else if (ng >= 5 && PF >= 20) rowSum(std::integral_constant<int, PF >= 20 ? 5 : 1>{}, mixed);
-            else if (ng >= 4 && PF >= 16) rowSum(std::integral_constant<int, PF >= 16 ? 4 : 1>{}, mixed);
-            else if (ng >= 3 && PF >= 12) rowSum(std::integral_constant<int, PF >= 12 ? 3 : 1>{}, mixed);
-            else if (ng >= 2 && PF >= 8) rowSum(std::integral_constant<int, PF >= 8 ? 2 : 1>{}, mixed);
-            else if (ng >= 1) rowSum(std::integral_constant<int, 1>{}, mixed);
-        };
-        if constexpr (MULTI) {
-            if (__any(out != 0)) rowSums(std::true_type{});
-            else rowSums(std::false_type{});
-        } else {
-            rowSums(std::false_type{});
-        }
+        const int ng = width / GRP;
+        if (ng >= 6 && PF >= 24) rowSum(std::integral_constant<int, PF >= 24 ? 6 : 1>{});
+        else if (ng >= 5 && PF >= 20) rowSum(std::integral_constant<int, PF >= 20 ? 5 : 1>{});
+        else if (ng >= 4 && PF >= 16) rowSum(std::integral_constant<int, PF >= 16 ? 4 : 1>{});
+        else if (ng >= 3 && PF >= 12) rowSum(std::integral_constant<int, PF >= 12 ? 3 : 1>{});
+        else if (ng >= 2 && PF >= 8) rowSum(std::integral_constant<int, PF >= 8 ? 2 : 1>{});
+        else if (ng >= 1) rowSum(std::integral_constant<int, 1>{});
         for (int k0 = PF; k0 < width; k0 += GRP) {
             int j[GRP];
             T f[GRP], xt[GRP];
@@ -253,20 +318,20 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
             for (int q = 0; q < GRP; ++q) f[q] = ecoef[unsigned((k0 + q) * rows) + t];
 #pragma unroll
             for (int q = 0; q < GRP; ++q) {
-                xt[q] = value((MULTI && j[q] < 0 ? 0 : j[q]) * int(sizeof(T)));
+                xt[q] = value(lds + unsigned(MULTI && j[q] < 0 ? 0 : j[q]) * unsigned(sizeof(T)));
                 if (MULTI && j[q] < 0) {
-                    xt[q] = far(j[q]);
-                    for (unsigned spins = 0; missing(j[q], xt[q]) && !given_up(spins, a.fault); ++spins)
+                    xt[q] = mailed(j[q]) ? Sentinel<T>::value() : initial(j[q]);
+                    for (unsigned spins = 0; Sentinel<T>::is(xt[q]) && !given_up(spins, a.fault); ++spins)
                         xt[q] = peek(&mail[~j[q]]);
                 }
             }
 #pragma unroll
             for (int q = 0; q < GRP; ++q) acc = acc - row_term<OP>(f[q], xt[q]);
         }
-        if constexpr (OP == SW_GS) acc = acc / dg;
-        if (lane < rows) *reinterpret_cast<T*>(lds + slot) = acc;
+        if constexpr (OP == SW_GS) acc = div(acc);
+        *(Lds*)uintptr_t(slot) = acc;
         lds_release();
-        if (lane == 0) __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (lane == 0) count_step(cnt);
         __builtin_amdgcn_s_setprio(0);
         if constexpr (MULTI) {
             if (lane < rows) publish_value(&a.mail[sweep * ptrdiff_t(P.n) + pos + lane], acc);
@@ -336,7 +401,7 @@ __global__ __launch_bounds__(WAVES* WAVE) void k_sweep_chunks(SweepPlan P, Sweep
     if (sweep == 0) sweep_fill<OP>(P, a, xs, c0, nc, h0, nh);
     else if (threadIdx.x == 0) xs[nc + nh] = T(0);  // the others are written before they are read
     __syncthreads();
-    sweep_steps<OP, true, PF, WAVES, T>(P, a, xs, &cnt, c0, P.stepOff[k], P.stepOff[k + 1], sweep);
+    sweep_steps<OP, true, PF, WAVES, T>(P, a, xs, nc + nh, &cnt, c0, P.stepOff[k], P.stepOff[k + 1], sweep);
     if (sweep + 1 < sweeps) return;
     __syncthreads();
     for (int q = threadIdx.x; q < nc; q += blockDim.x) a.x[c0 + q] = xs[q];
@@ -352,7 +417,7 @@ __global__ __launch_bounds__(WAVES* WAVE) void k_sweep_one(SweepPlan P, SweepArg
     if (threadIdx.x == 0) cnt = 0;
     sweep_fill<OP>(P, a, xs, 0, P.n, 0, 0);
     __syncthreads();
-    sweep_steps<OP, false, PF, WAVES, T>(P, a, xs, &cnt, 0, 0, P.nSteps, 0);
+    sweep_steps<OP, false, PF, WAVES, T>(P, a, xs, P.n, &cnt, 0, 0, P.nSteps, 0);
     __syncthreads();
     for (int i = threadIdx.x; i < P.n; i += blockDim.x) a.x[i] = xs[i];
 }
@@ -368,10 +433,10 @@ __global__ __launch_bounds__(WAVES* WAVE) void k_dilu_one(SweepPlan F, SweepPlan
     if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
     sweep_fill<SW_FWD>(F, a, xs, 0, F.n, 0, 0);
     __syncthreads();
-    sweep_steps<SW_FWD, false, PF, WAVES, T>(F, a, xs, &cnt[0], 0, 0, F.nSteps, 0);
+    sweep_steps<SW_FWD, false, PF, WAVES, T>(F, a, xs, F.n, &cnt[0], 0, 0, F.nSteps, 0);
     __syncthreads();
     a.coef = eb;
-    sweep_steps<SW_BWD, false, PF, WAVES, T>(B, a, xs, &cnt[1], 0, 0, B.nSteps, 0);
+    sweep_steps<SW_BWD, false, PF, WAVES, T>(B, a, xs, B.n, &cnt[1], 0, 0, B.nSteps, 0);
     __syncthreads();
     for (int i = threadIdx.x; i < F.n; i += blockDim.x) a.x[i] = xs[i];
 }

@@ -60,13 +60,22 @@ struct SweepPlanHost {
 // 158 levels: 18 of them in 6144 cells, 8 in 1536, where two sweeps take 340 and 200 µs;
 // 64³ hexes, whose chunks all see about 128 of the 190 levels: 188 and 261); fewer cells
 // only add hops between chunks. Long rows (coarse GAMG levels, few rows a level): 4096.
+// Where that makes at most SWEEP_FEW_CHUNKS chunks, twice as many: a step less per level and
+// chunk is then worth more than the hops (two sweeps, as given and doubled: 16,384 box cells
+// in 6 chunks 54 → 44 µs, 65,536 in 22: 91 → 85, 49,000 agglomerated cells in 12: 206 → 170,
+// 20,000 in 6: 79 → 64; but 262,144 box cells in 86: 150 → 204, 188,000 agglomerated cells
+// in 46: 175 → 203).
 constexpr int SWEEP_ONE_CELLS = 8192;
+constexpr int SWEEP_FEW_CHUNKS = 24;
 inline int sweepChunks(int n, const std::vector<int>& off, const std::vector<int>& perm, bool longRows) {
     if (n <= SWEEP_ONE_CELLS) return 1;
-    auto chunks = [n](int cells) { return (n + cells - 1) / cells; };
+    auto chunks = [n](int cells) {
+        const int nc = (n + cells - 1) / cells;
+        return nc <= SWEEP_FEW_CHUNKS ? 2 * nc : nc;
+    };
     if (longRows) return chunks(4096);
     for (int cells : {6144, 3072}) {
-        const int nc = chunks(cells);
+        const int nc = (n + cells - 1) / cells;
         int64_t runs = 0;  // (level, chunk) pairs
         for (size_t L = 0; L + 1 < off.size(); ++L)
             for (int i = off[L], last = -1; i < off[L + 1]; ++i) {
@@ -74,7 +83,7 @@ inline int sweepChunks(int n, const std::vector<int>& off, const std::vector<int
                 runs += k != last;
                 last = k;
             }
-        if (runs * 128 >= n) return nc;
+        if (runs * 128 >= n) return chunks(cells);
     }
     return chunks(1536);
 }
