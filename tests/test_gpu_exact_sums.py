@@ -56,3 +56,28 @@ def test_exact_sums_of_zeros_and_non_finite(ctx):
     assert np.isinf(p.residualSum)
     v[3] = np.nan
     assert np.isnan(_prologue(ctx, v, np.zeros(n)).residualSum)
+
+
+@pytest.mark.parametrize("pre", ["none", "diagonal"])
+@pytest.mark.parametrize("n", [2, 257, 5000, 256 * 512 + 1])
+def test_pcg_with_diagonal_against_oracle(ctx, n, pre):
+    """Both sums of an iteration's end in one reduction: bits of the oracle's recurrence with
+    exact sums, a stop at every count included; fast sums within their rounding of it."""
+    own, nei = np.arange(n - 1), np.arange(1, n)
+    u = -1.0 - W.splitmix_uniform(n - 1, 5)
+    d = 1.0 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
+    b = 2.0 * W.splitmix_uniform(n, 7) - 1.0
+    om, lm = O.LduMesh(n, own, nei), va.LduMesh(ctx, n, own, nei)
+    A = va.LduMatrix(lm, d, u)
+    for most, least in ((1, 0), (2, 0), (3, 0), (60, 0), (60, 9)):
+        xo, po = om.solve(d, u, None, b, x0=np.zeros(n), solver="PCG", preconditioner=pre, tolerance=1e-9,
+                          max_iter=most, min_iter=least, mode=O.MODE_EXACT)
+        x = np.zeros(n)
+        p = va.solve_ldu(A, b, x, va.SolverControls("PCG", pre, 1e-9, 0.0, most, least, sums=va.SUMS_EXACT))
+        assert p.iterations == po["iterations"] and p.finalResidual == po["finalResidual"]
+        assert np.array_equal(x, xo)
+        xf = np.zeros(n)
+        va.solve_ldu(A, b, xf, va.SolverControls("PCG", pre, 1e-9, 0.0, most, least))
+        # α and β differ by the sums' rounding, n·2^-53 at most, over 60 steps of a system
+        # whose condition number is below 10; x is of order 1
+        assert np.abs(xf - xo).max() <= 60 * 10 * n * 2.0**-53 + 1e-9

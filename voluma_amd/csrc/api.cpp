@@ -1570,16 +1570,29 @@ template <class T> struct Krylov {
     T* z0 = nullptr;                 // ω·(r·rD) kept with r (PCG + Jacobi GAMG, one pre-sweep)
 };
 
-// One PCG or PBiCGStab iteration, every kernel predicated on C.done.
+// PCG without a preconditioner or with the diagonal one, FP64: w and Σ w·r of an iteration
+// come with the residual that the iteration before leaves (one pass over r and one
+// finalize less per iteration), the first ones from here.
+template <class T> void pcgDiagonalStart(const Ctx& C, vol_matrix A, const Plan& P, const Krylov<T>& k, bool ex) {
+    const int n = A->mesh->n;
+    vec<T>(C, V_PRECOND_DOT, n, ex, k.r, nullptr, nullptr, nullptr, k.w, nullptr, nullptr,
+           P.precond == "diagonal" ? level0(A, (T*)nullptr).rD : nullptr);
+    fin(C, FIN_PCG_WRA, 1, ex, ex ? vec_exact_blocks(n) : RED_BLOCKS);
+}
+
+// One PCG or PBiCGStab iteration, every kernel predicated on C.done. withW: k.w and Σ w·r
+// are there (pcgDiagonalStart).
 template <class T>
-void krylovIteration(const Ctx& C, vol_matrix A, const Plan& P, const Krylov<T>& k, bool isPCG, bool ex) {
+void krylovIteration(const Ctx& C, vol_matrix A, const Plan& P, const Krylov<T>& k, bool isPCG, bool ex,
+                     bool withW = false) {
     const int n = A->mesh->n;
     const bool fuse = !ex;
     const int nparts = ex ? vec_exact_blocks(n) : RED_BLOCKS;
     const int sellParts = sell_grid_blocks(A->mesh->sell.nslices);
     const Level0<T> L0 = level0(A, (T*)nullptr);
     if (isPCG) {  // LinearSolver.cpp:176-201
-        if (P.precond == "GAMG" && !P.gamgGS && fuse && A->tailStart != 0) {  // Σ w·r fused into the last sweep
+        if (withW) {
+        } else if (P.precond == "GAMG" && !P.gamgGS && fuse && A->tailStart != 0) {  // Σ w·r fused into the last sweep
             vcycle<T>(C, A, P, 0, k.r, k.w, k.r, redOf(C).part, k.z0);
             fin(C, FIN_PCG_WRA, 1, false, sellParts);
         } else {
@@ -1599,6 +1612,12 @@ void krylovIteration(const Ctx& C, vol_matrix A, const Plan& P, const Krylov<T>&
         } else {
             vec<T>(C, V_DOT, n, ex, k.q, k.p);
             fin(C, FIN_PCG_WAPA, 1, ex, nparts);
+        }
+        if (withW) {
+            vec<T>(C, V_PCG_XRW, n, ex, k.p, k.q, nullptr, nullptr, k.w, k.x, k.r,
+                   P.precond == "diagonal" ? L0.rD : nullptr);
+            fin(C, FIN_PCG_NORM_WRA, 2, ex, ex ? nparts : vec_fast_blocks(V_PCG_XRW, n, redOf(C).maxBlk), C.hostOut);
+            return;
         }
         vec<T>(C, V_PCG_XR, n, ex, k.p, k.q, nullptr, nullptr, k.z0, k.x, k.r, k.z0 ? L0.rD : nullptr, P.omega);
         fin(C, FIN_PCG_NORM, 1, ex, ex ? nparts : vec_fast_blocks(V_PCG_XR, n, redOf(C).maxBlk), C.hostOut);
@@ -1826,7 +1845,9 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
             } else if (P.precond != "GAMG") {
                 launch_fill_zero<double>(st, n, k.p, nullptr);
             }
-            runLoop(c, C, maxLoops, [&] { krylovIteration<double>(C, A, P, k, isPCG, ex); });
+            const bool withW = isPCG && P.precond != "GAMG" && !dilu;
+            if (withW) pcgDiagonalStart<double>(C, A, P, k, ex);
+            runLoop(c, C, maxLoops, [&] { krylovIteration<double>(C, A, P, k, isPCG, ex, withW); });
         } else {  // Jacobi and Gauss–Seidel solvers, LinearSolver.cpp:238-278
             A->vw.alloc(n);
             const bool sym = P.solver == "symGaussSeidel";

@@ -656,7 +656,7 @@ void launch_sell_coef(hipStream_t st, const SellView& S, const double* upper, co
 // without a reduction; other reductions use RED_BLOCKS blocks.
 int vec_fast_blocks(int op, int n, int maxBlk) {
     const int rows = std::max((n + RED_THREADS - 1) / RED_THREADS, 1);
-    if (op == V_PCG_XR) return std::max(std::min({rows, 4 * RED_BLOCKS, maxBlk}), 1);
+    if (op == V_PCG_XR || op == V_PCG_XRW) return std::max(std::min({rows, 4 * RED_BLOCKS, maxBlk}), 1);
     if (vec_has_reduction(op) > 0) return RED_BLOCKS;
     return std::min(rows, 4 * RED_BLOCKS);
 }
@@ -664,7 +664,7 @@ int vec_fast_blocks(int op, int n, int maxBlk) {
 int vec_has_reduction(int op) {
     switch (op) {
     case V_SUM_X: case V_PRECOND_DOT: case V_DOT: case V_PCG_XR: case V_BI_S: case V_BMINUSAX_NORM: return 1;
-    case V_INIT: case V_BI_DOT2: return 2;
+    case V_INIT: case V_BI_DOT2: case V_PCG_XRW: return 2;
     case V_BI_XR: return 1;
     default: return 0;
     }
@@ -700,6 +700,14 @@ __device__ __forceinline__ void vec_elem(const VecArgsT<T>& A, int i, double& r0
         A.y[i] = r;
         if (A.w) A.w[i] = T(A.omega) * (r * A.rD[i]);
         r0 = fabs(double(r));
+    } else if constexpr (OP == V_PCG_XRW) {  // a = p, b = q; x = x, y = r, w = w
+        A.x[i] = T(ld(A.x, i) + S->alpha * ld(A.a, i));
+        const T r = T(ld(A.y, i) - S->alpha * ld(A.b, i));
+        const T w = T(A.rD ? ld(A.rD, i) * double(r) : double(r));
+        A.y[i] = r;
+        A.w[i] = w;
+        r0 = fabs(double(r));
+        r1 = double(w) * double(r);
     } else if constexpr (OP == V_BI_P) {  // a = r, b = Ay; x = p
         A.x[i] = T(S->iterations == 0 ? ld(A.a, i) : ld(A.a, i) + S->beta * (ld(A.x, i) - S->omegaB * ld(A.b, i)));
     } else if constexpr (OP == V_SCALE) {
@@ -813,7 +821,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_vec_exact(VecArgs A, long long*
 
 template <int OP, class T>
 static void vec_dispatch(hipStream_t st, const VecArgsT<T>& a, bool exact, const RedScratch& R) {
-    constexpr int NRED = (OP == V_INIT || OP == V_BI_DOT2) ? 2
+    constexpr int NRED = (OP == V_INIT || OP == V_BI_DOT2 || OP == V_PCG_XRW) ? 2
                          : (OP == V_SUM_X || OP == V_PRECOND_DOT || OP == V_DOT || OP == V_PCG_XR || OP == V_BI_S ||
                             OP == V_BMINUSAX_NORM || OP == V_BI_XR)
                              ? 1
@@ -838,6 +846,9 @@ static void launch_vec_t(hipStream_t st, int op, const VecArgsT<T>& a, bool exac
     case V_DOT: vec_dispatch<V_DOT>(st, a, exact, R); break;
     case V_PCG_P: vec_dispatch<V_PCG_P>(st, a, exact, R); break;
     case V_PCG_XR: vec_dispatch<V_PCG_XR>(st, a, exact, R); break;
+    case V_PCG_XRW:
+        if constexpr (sizeof(T) == 8) vec_dispatch<V_PCG_XRW>(st, a, exact, R);
+        break;
     case V_BI_P: vec_dispatch<V_BI_P>(st, a, exact, R); break;
     case V_SCALE: vec_dispatch<V_SCALE>(st, a, exact, R); break;
     case V_BI_S: vec_dispatch<V_BI_S>(st, a, exact, R); break;
@@ -922,6 +933,10 @@ __device__ void fin_step(int op, DevScalars& S, const DevScalars& I, double v0, 
         S.finalResidual = v0 / S.normFactor;
         ++S.iterations;
         if (!(S.iterations < S.maxIter && !dev_converged(S))) S.done = 1;
+        break;
+    case FIN_PCG_NORM_WRA:  // a solve that is done takes no next step
+        fin_step(FIN_PCG_NORM, S, I, v0, 0.0);
+        if (!S.done) fin_step(FIN_PCG_WRA, S, I, v1, 0.0);
         break;
     case FIN_BI_RHO:
         S.rhoOld = S.rho;
@@ -1042,80 +1057,83 @@ __global__ __launch_bounds__(FIN_THREADS) void k_finalize(int op, int nred, int 
 }
 
 // The finalize of exact sums. Integer bins add up to the same value in any order, so the
-// blocks' partials are read by the whole workgroup: first the blocks' info words (one per
+// blocks' partials are read by FINX_THREADS threads per sum, all sums at once: first the blocks' info words (one per
 // thread, nparts ≤ FINX_THREADS), then only the window of bins any block used, P threads
 // (the window rounded up to a power of two) per partial and FINX_LOADS loads in flight
 // each, a tree over the FINX_THREADS / P groups, and the carries and the conversion over
 // the window on one thread. Latency-bound: two round trips, the tree and ~10 bins in turn.
 // Adding the partials bin by bin on 72 threads and carrying through all 72 bins took 116 µs
-// per launch at 512 partials; a reproducible PCG iteration on 24,480 cells (three of these)
-// went from 375 to 38 µs with this and the smaller grids of vec_exact_blocks.
+// per launch at 512 partials; a reproducible PCG iteration on 24,480 cells (then three of
+// these) went from 375 to 38 µs with this and the smaller grids of vec_exact_blocks, and to
+// 34 with both sums of the iteration's end in one (V_PCG_XRW; 37 with one after the other).
 constexpr int FINX_THREADS = 512;
 constexpr int FINX_LOADS = 8;
 static_assert(RED_BLOCKS_EXACT <= FINX_THREADS, "one info word per thread");
-__global__ __launch_bounds__(FINX_THREADS) void k_finalize_exact(int op, int nred, int nparts, const long long* xpart,
-                                                                 const int* xnf, int maxBlk, DevScalars* Sp,
-                                                                 double* result, DevScalars* hostOut) {
+__global__ __launch_bounds__(FINX_THREADS* MAX_RED) void k_finalize_exact(int op, int nred, int nparts,
+                                                                          const long long* xpart, const int* xnf,
+                                                                          int maxBlk, DevScalars* Sp, double* result,
+                                                                          DevScalars* hostOut) {
     if (op != FIN_STORE && Sp->done) {
         if (threadIdx.x == 0) publish(*Sp, hostOut);
         return;
     }
     __shared__ double vals[MAX_RED];
-    __shared__ long long sum[FINX_THREADS];
-    __shared__ long long bins[NBINS];
-    __shared__ int nfl, lo, hi;
-    const int t = threadIdx.x;
-    for (int q = 0; q < nred; ++q) {
-        if (t == 0) {
-            nfl = 0;
-            lo = NBINS;
-            hi = -1;
-        }
-        __syncthreads();
-        const int f = t < nparts ? xnf[q * maxBlk + t] : exact_info(0, NBINS, -1);
-        const int wlo = wave_min_i((f >> 8) & 0xff), whi = wave_max_i((f >> 16) - 1);
-        if (t % WAVE == 0) {
-            atomicMin(&lo, wlo);
-            atomicMax(&hi, whi);
-        }
-        if (f & 0xff) atomicOr(&nfl, f & 0xff);
-        __syncthreads();
-        const int l = lo, w = hi - lo + 1;
-        int P = 8;
-        while (P < w) P *= 2;  // ≤ 128
-        const int b = t % P, g = t / P, groups = FINX_THREADS / P;
-        long long s = 0;
-        if (b < w) {
-            const long long* src = xpart + size_t(q) * maxBlk * NBINS + l + b;
-            for (int k0 = g; k0 < nparts; k0 += groups * FINX_LOADS) {
-                long long v[FINX_LOADS];
-#pragma unroll
-                for (int u = 0; u < FINX_LOADS; ++u) {
-                    const int k = k0 + u * groups;
-                    v[u] = k < nparts ? src[size_t(k) * NBINS] : 0;
-                }
-#pragma unroll
-                for (int u = 0; u < FINX_LOADS; ++u) s += v[u];
-            }
-        }
-        sum[t] = s;
-        for (int o = groups / 2; o > 0; o /= 2) {
-            __syncthreads();
-            if (g < o) sum[t] += sum[t + o * P];
-        }
-        __syncthreads();
-        if (t < w) bins[l + t] = sum[t];
-        __syncthreads();
-        if (t == 0) vals[q] = exact_to_double(bins, l, hi, nfl);
-        __syncthreads();
+    __shared__ long long sum[FINX_THREADS * MAX_RED];
+    __shared__ long long bins[MAX_RED][NBINS];
+    __shared__ int nfl[MAX_RED], lo[MAX_RED], hi[MAX_RED];
+    const int q = threadIdx.x / FINX_THREADS, t = threadIdx.x % FINX_THREADS;  // q < nred
+    if (t == 0) {
+        nfl[q] = 0;
+        lo[q] = NBINS;
+        hi[q] = -1;
     }
-    if (t == 0) fin_apply(op, nred, vals[0], nred > 1 ? vals[1] : 0.0, Sp, result, hostOut);
+    __syncthreads();
+    const int f = t < nparts ? xnf[q * maxBlk + t] : exact_info(0, NBINS, -1);
+    const int wlo = wave_min_i((f >> 8) & 0xff), whi = wave_max_i((f >> 16) - 1);
+    if (t % WAVE == 0) {
+        atomicMin(&lo[q], wlo);
+        atomicMax(&hi[q], whi);
+    }
+    if (f & 0xff) atomicOr(&nfl[q], f & 0xff);
+    __syncthreads();
+    const int l = lo[q], w = hi[q] - l + 1;
+    int widest = 0;  // one P for all: the tree's barriers are the same for every thread
+    for (int k = 0; k < nred; ++k) widest = max(widest, hi[k] - lo[k] + 1);
+    int P = 8;
+    while (P < widest) P *= 2;  // ≤ 128
+    const int b = t % P, g = t / P, groups = FINX_THREADS / P;
+    long long s = 0;
+    if (b < w) {
+        const long long* src = xpart + size_t(q) * maxBlk * NBINS + l + b;
+        for (int k0 = g; k0 < nparts; k0 += groups * FINX_LOADS) {
+            long long v[FINX_LOADS];
+#pragma unroll
+            for (int u = 0; u < FINX_LOADS; ++u) {
+                const int k = k0 + u * groups;
+                v[u] = k < nparts ? src[size_t(k) * NBINS] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < FINX_LOADS; ++u) s += v[u];
+        }
+    }
+    long long* const mine = sum + q * FINX_THREADS;
+    mine[t] = s;
+    for (int o = groups / 2; o > 0; o /= 2) {
+        __syncthreads();
+        if (g < o) mine[t] += mine[t + o * P];
+    }
+    __syncthreads();
+    if (t < w) bins[q][l + t] = mine[t];
+    __syncthreads();
+    if (t == 0) vals[q] = exact_to_double(bins[q], l, hi[q], nfl[q]);
+    __syncthreads();
+    if (threadIdx.x == 0) fin_apply(op, nred, vals[0], nred > 1 ? vals[1] : 0.0, Sp, result, hostOut);
 }
 
 void launch_finalize(hipStream_t st, int op, int nred, bool exact, int nparts, const RedScratch& R, DevScalars* S,
                      DevScalars* hostOut) {
     if (exact && op != FIN_INNER_START)
-        hipLaunchKernelGGL(k_finalize_exact, dim3(1), dim3(FINX_THREADS), 0, st, op, nred, nparts, R.xpart, R.xnf,
+        hipLaunchKernelGGL(k_finalize_exact, dim3(1), dim3(FINX_THREADS * nred), 0, st, op, nred, nparts, R.xpart, R.xnf,
                            R.maxBlkExact, S, R.result, hostOut);
     else
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, op, nred, nparts, R.part, R.maxBlk, S,

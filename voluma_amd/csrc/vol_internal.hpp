@@ -104,6 +104,7 @@ enum FinOp : int {
     FIN_STORE = 11,    // only store the reduced values (tests/diagnostics)
     FIN_OUTER = 12,    // mixed: outer residual Σ|b − Ax| after x += e; convergence of the whole solve
     FIN_INNER_START = 13,  // mixed: set up the next inner solve in S[1] from S[0]
+    FIN_PCG_NORM_WRA = 14,  // FIN_PCG_NORM on the first value, then FIN_PCG_WRA on the second
 };
 
 // Reduction scratch: fast mode uses `nblk` double partials per reduced quantity;
@@ -205,6 +206,7 @@ enum VecOp : int {
     V_FROMZERO = 15,      // w = ω·(r/d)
     V_FILL_XREF = 16,     // w = xRef of the row's system (batches)
     V_ZSCALE = 17,        // w = ω·(a·rD) in the vector type (the first Jacobi sweep from zero)
+    V_PCG_XRW = 18,       // V_PCG_XR, then w = rD·r (rD null: r) of the new r; red0 = Σ|r|, red1 = Σ w·r
 };
 
 // Vector element type T (double, or float for the inner solve of mixed precision);
