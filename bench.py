@@ -343,7 +343,7 @@ def reference_solvers_leg(va, W, ctx, m, A, db, dx, dzero, args, cpu):
     """The reference's own solver choices on the GPU: GAMG-PCG with its Gauss–Seidel
     smoother (2/2 sweeps) on the pressure system, and its default momentum solver
     (PBiCGStab + DILU) on the momentum matrix of velocity component 0, both as
-    level-scheduled sweeps; with cpu, the momentum solve's CPU baseline too."""
+    level-ordered sweeps; with cpu, the momentum solve's CPU baseline too."""
     out = {}
     short = args.profile_legs  # a kernel-trace run: one short solve of each kind
     ctl = va.SolverControls("PCG", "GAMG", args.tol, 0.0, 3 if short else 1000, gamgSmoother=va.GAMG_GAUSS_SEIDEL)

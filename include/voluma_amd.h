@@ -103,7 +103,7 @@ typedef struct {
 #define VOL_GAMG_JACOBI 0
 /* the reference's smoother (GAMG.cpp:363-384,423-442): x = 0, gamgPreSweeps forward
  * Gauss–Seidel sweeps, coarse correction, gamgPostSweeps backward sweeps, each level
- * run as level-scheduled sweeps; with 2/2 sweeps and exact sums the V-cycle is the
+ * run in level order; with 2/2 sweeps and exact sums the V-cycle is the
  * reference's bit for bit */
 #define VOL_GAMG_GAUSS_SEIDEL 1
 
