@@ -34,8 +34,8 @@
 // looks counts where chunks wait for each other: with a division after the sum, a wait for
 // the stores before the count, an add per LDS address, branches per entry in the polls and
 // the first look at other chunks' values one round trip each, these took 205 and 185 µs
-// (49,000 agglomerated cells of up to 20 entries 310, now 170). PCG with GAMG smoothed by
-// Gauss–Seidel on these meshes: 235 → 57 and 66 → 18 ms; DIC-PCG on 24,273 hexes 34.6 → 7.6
+// (24,000 agglomerated cells of up to 20 entries 310, now 170). PCG with GAMG smoothed by
+// Gauss–Seidel on these meshes: 228 → 53 and 66 → 18 ms; DIC-PCG on 24,273 hexes 34.6 → 7.6
 // ms; three momentum components by PBiCGStab + DILU on 839,664 tets, assembly and factor
 // included, 28.8 → 6.3 ms.
 #include "device_common.hpp"

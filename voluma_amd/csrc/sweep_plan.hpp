@@ -62,11 +62,11 @@ struct SweepPlanHost {
 // only add hops between chunks. Long rows (coarse GAMG levels, few rows a level): 4096.
 // Where that makes at most SWEEP_FEW_CHUNKS chunks, twice as many: a step less per level and
 // chunk is then worth more than the hops (two sweeps, as given and doubled: 16,384 box cells
-// in 6 chunks 54 → 44 µs, 65,536 in 22: 91 → 85, 49,000 agglomerated cells in 12: 206 → 170,
-// 20,000 in 6: 79 → 64; but 262,144 box cells in 86: 150 → 204, 188,000 agglomerated cells
-// in 46: 175 → 203).
+// in 3 chunks 54 → 44 µs, 65,536 in 11: 91 → 85, 24,000 agglomerated cells in 6: 206 → 170,
+// 10,000 in 3: 79 → 65; but 93,000 agglomerated cells in 23: 175 → 203, 262,144 box cells in
+// 43: 150 → 204).
 constexpr int SWEEP_ONE_CELLS = 8192;
-constexpr int SWEEP_FEW_CHUNKS = 24;
+constexpr int SWEEP_FEW_CHUNKS = 12;
 inline int sweepChunks(int n, const std::vector<int>& off, const std::vector<int>& perm, bool longRows) {
     if (n <= SWEEP_ONE_CELLS) return 1;
     auto chunks = [n](int cells) {
