@@ -128,3 +128,27 @@ def test_row_division_over_the_exponent_range(ctx, name, powers):
         va.solve_ldu(va.LduMatrix(lm, d, u, lo), b, x, va.SolverControls("GaussSeidel", "none", 1e-300, 0.0, sweeps,
                                                                         nSweeps=sweeps, sums=va.SUMS_EXACT))
         assert np.array_equal(x, xo) and np.array_equal(np.signbit(x), np.signbit(xo)), sweeps
+
+
+@pytest.mark.parametrize("name", ["one", "two", "wide"])
+def test_infinite_coefficients_keep_the_loops_signs(ctx, name):
+    """Infinite coefficients on faces of a chunk whose rows also read other chunks' values:
+    every infinity and every NaN of the sequential loop, and its bits elsewhere."""
+    n, own, nei = _graph(name)
+    rng = np.random.default_rng(12)
+    u, lo = -rng.uniform(0.5, 1.5, own.size), -rng.uniform(0.5, 1.5, own.size)
+    d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -lo, n)
+    b, x0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    near = np.flatnonzero((np.minimum(own, nei) > n // 2) & (np.maximum(own, nei) < n // 2 + 400))
+    for at, side in zip(rng.choice(near, 6, replace=False), (u, lo) * 3):
+        side[at] = rng.choice([-np.inf, np.inf])
+    lm, om = va.LduMesh(ctx, n, own, nei), O.LduMesh(n, own, nei)
+    A = va.LduMatrix(lm, d, u, lo)
+    for sweeps in (1, 2):
+        xo, _ = om.solve(d, u, lo, b, x0=x0, solver="GaussSeidel", preconditioner="none", tolerance=1e-30,
+                         max_iter=1, n_sweeps=sweeps, mode=O.MODE_EXACT)
+        assert np.isinf(xo).any()
+        x = x0.copy()
+        va.solve_ldu(A, b, x, va.SolverControls("GaussSeidel", "none", 1e-30, 0.0, 1, nSweeps=sweeps,
+                                                sums=va.SUMS_EXACT))
+        assert np.array_equal(x, xo, equal_nan=True), sweeps

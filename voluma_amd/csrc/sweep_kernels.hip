@@ -233,12 +233,15 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
             }
             if (__any(lowest < 0)) {
                 T v[PF], own[PF];
+                bool inf = false;
 #pragma unroll
                 for (int k = 0; k < PF; ++k) {
                     own[k] = at[k] < 0 ? -T(0) : cf[k];
                     v[k] = OP == SW_FAC ? T(1) : copysign(T(0), -cf[k]);  // cf·v = −0
+                    if (OP != SW_FAC) inf = inf | __builtin_isinf(own[k]);
                     asm volatile("" : "+v"(own[k]), "+v"(v[k]));
                 }
+                const bool infinite = __any(inf);
                 // all of them in one round trip; then, once the turn is near (asking
                 // earlier only loads the fabric), the ones not yet published again,
                 // together, until they are
@@ -271,6 +274,11 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
                     const T f = OP != SW_FAC || at[k] < 0 ? cf[k] : -T(0);
                     add[k] = row_term<OP>(f, v[k]);
                     cf[k] = own[k];
+                }
+                if (infinite) {  // ∞·0 is no −0 (a select in every step would come after the values)
+#pragma unroll
+                    for (int k = 0; k < PF; ++k)
+                        if (at[k] >= 0) add[k] = -T(0);
                 }
             }
         }
