@@ -152,3 +152,22 @@ def test_infinite_coefficients_keep_the_loops_signs(ctx, name):
         va.solve_ldu(A, b, x, va.SolverControls("GaussSeidel", "none", 1e-30, 0.0, 1, nSweeps=sweeps,
                                                 sums=va.SUMS_EXACT))
         assert np.array_equal(x, xo, equal_nan=True), sweeps
+
+
+def test_long_chain_is_no_timeout(ctx):
+    """Two million cells in a row, one row per level: a chunk's wait lasts as long as all the
+    chunks before it take (most of a second), which is no failure."""
+    n = 2_000_000
+    own, nei = np.arange(n - 1, dtype=np.int32), np.arange(1, n, dtype=np.int32)
+    rng = np.random.default_rng(13)
+    u = -rng.uniform(0.5, 1.5, n - 1)
+    d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
+    b = rng.uniform(-1, 1, n)
+    lm, om = va.LduMesh(ctx, n, own, nei), O.LduMesh(n, own, nei)
+    A = va.LduMatrix(lm, d, u)
+    for solver, pre in (("GaussSeidel", "none"), ("PCG", "DIC")):
+        xo, _ = om.solve(d, u, None, b, x0=np.zeros(n), solver=solver, preconditioner=pre, tolerance=1e-30, max_iter=1,
+                         mode=O.MODE_EXACT)
+        x = np.zeros(n)
+        va.solve_ldu(A, b, x, va.SolverControls(solver, pre, 1e-30, 0.0, 1, sums=va.SUMS_EXACT))
+        assert np.array_equal(x, xo), solver

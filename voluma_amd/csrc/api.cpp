@@ -614,6 +614,7 @@ void buildDilu(vol_matrix A) {
     if (F.v.nChunks > 1) {
         a.mail = sweepMailbox<double>(c, st, m->n, 1, nullptr);
         a.ticket = c->sweepFault.p + 1;
+        a.polls = sweepPolls(F.v.serial, 1);
         a.fault = c->sweepFault.p;
     }
     launch_sweep<double>(st, SW_FAC, false, F.v, a, 1, nullptr);
@@ -1480,6 +1481,7 @@ void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T
     for (int s = 0; s < k; s += SWEEP_MAX_SWEEPS) {
         const int q = std::min(k - s, SWEEP_MAX_SWEEPS);
         a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
+        a.polls = sweepPolls(E.v.serial, q);
         launch_sweep<T>(C.st, SW_GS, backward, E.v, a, q, C.done);
         a.zero = false;
     }
@@ -1539,9 +1541,11 @@ void precondApply(const Ctx& C, vol_matrix A, const Plan& P, const T* r, T* w, i
         }
         a.mail = sweepMailbox<T>(C.c, C.st, n, 2, C.done);
         a.ticket = C.c->sweepFault.p + 1;
+        a.polls = sweepPolls(F.serial, 1);
         a.fault = C.c->sweepFault.p;
         launch_sweep<T>(C.st, SW_FWD, false, F, a, 1, C.done);
         a.coef = eb;
+        a.polls = sweepPolls(B.serial, 1);
         a.mail += n;
         ++a.ticket;
         launch_sweep<T>(C.st, SW_BWD, true, B, a, 1, C.done);

@@ -98,6 +98,7 @@ struct SweepPlanDev {
         v.halo = halo.p;
         v.maxSlots = H.maxSlots;
         v.maxWidth = H.maxWidth;
+        v.serial = H.serial;
         HIPCHECK(hipStreamSynchronize(st));
     }
 };

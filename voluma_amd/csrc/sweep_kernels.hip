@@ -23,7 +23,8 @@
 // before its turn. Chunks are handed out by a ticket counter in sweep order, so a value
 // is only ever waited for from a workgroup that has started (and waits itself only for
 // earlier ones): whichever workgroups are resident, the earliest unfinished chunk
-// proceeds. A wait past its limit sets *fault and every later wait gives up at once.
+// proceeds. A wait past the plan's limit (sweepPolls) sets *fault and every later wait
+// gives up at once.
 //
 // Measured (MI355X): handing a step over through LDS takes 0.14 µs and a value handed to
 // another workgroup through memory 0.6 µs plus the polling; one CU streams rows at about
@@ -79,8 +80,6 @@ template <> struct Sentinel<float> {
     __device__ static float quiet() { return __uint_as_float(bits | (1u << 22)); }
 };
 
-constexpr unsigned SWEEP_SPIN_LIMIT = 1u << 18;  // polls of one value, ≥ 0.2 s
-
 template <class T> __device__ __forceinline__ T peek(const T* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -89,14 +88,15 @@ template <class T> __device__ __forceinline__ void publish_value(T* p, T v) {
     // a read-modify-write is performed where every XCD sees it
     (void)__hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Whether a wait ends without its value after `spins` polls: past its limit (which it
-// reports), or because another wait has.
-__device__ __forceinline__ bool given_up(unsigned spins, int* fault) {
-    if (spins > SWEEP_SPIN_LIMIT) {
+// Whether a wait ends without its value after `spins` polls, looked at every 64: past its
+// limit (sweepPolls; it reports that), or because another wait has.
+__device__ __forceinline__ bool given_up(unsigned spins, unsigned limit, int* fault) {
+    if ((spins & 63) != 63) return false;
+    if (spins > limit) {
         __hip_atomic_fetch_or(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return true;
     }
-    return (spins & 63) == 63 && __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 // Finished steps of the chunk.
 __device__ __forceinline__ int finished(int* cnt) {
@@ -262,7 +262,7 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
                         __builtin_amdgcn_s_sleep(2);
                         continue;
                     }
-                    if (given_up(++spins, a.fault)) break;
+                    if (given_up(++spins, a.polls, a.fault)) break;
 #pragma unroll
                     for (int k = 0; k < PF; ++k) {
                         asm volatile("" : "+v"(at[k]));  // no address kept over the loop
@@ -329,7 +329,7 @@ __device__ __forceinline__ void sweep_steps(const SweepPlan& P, const SweepArgs<
                 xt[q] = value(lds + unsigned(MULTI && j[q] < 0 ? 0 : j[q]) * unsigned(sizeof(T)));
                 if (MULTI && j[q] < 0) {
                     xt[q] = mailed(j[q]) ? Sentinel<T>::value() : initial(j[q]);
-                    for (unsigned spins = 0; Sentinel<T>::is(xt[q]) && !given_up(spins, a.fault); ++spins)
+                    for (unsigned spins = 0; Sentinel<T>::is(xt[q]) && !given_up(spins, a.polls, a.fault); ++spins)
                         xt[q] = peek(&mail[~j[q]]);
                 }
             }

@@ -42,6 +42,7 @@ struct SweepStep {
 
 struct SweepPlanHost {
     int n = 0, nChunks = 0, maxSlots = 0, maxWidth = 0;
+    int64_t serial = 0;         // Σ 1 + entry groups over the steps: the work if they ran in turn
     std::vector<int> chunkOff;  // first cell of each chunk (nChunks + 1)
     std::vector<int> stepOff;   // first step of each chunk (nChunks + 1)
     std::vector<int> haloOff, halo;  // cells of each chunk's halo
@@ -86,6 +87,18 @@ inline int sweepChunks(int n, const std::vector<int>& off, const std::vector<int
         if (runs * 128 >= n) return chunks(cells);
     }
     return chunks(1536);
+}
+
+// Polls of one value after which a wait of `sweeps` sweeps counts as failed. The earliest
+// unfinished chunk always proceeds, so a wait lasts at most as long as all steps one after
+// the other: 0.4 µs each when the rows are held (a chain of cells: every step a level), 2
+// µs per entry group past those. A poll is a memory round trip (0.3 µs at the least, 0.7
+// measured), so SWEEP_STEP_POLLS per step and group are over ten times that, and
+// SWEEP_BASE_POLLS (0.1–0.2 s) cover what does not grow with the plan. A fixed limit of
+// the base alone ended sweeps over a chain of two million cells (0.8 s) with an error.
+constexpr int64_t SWEEP_BASE_POLLS = int64_t(1) << 18, SWEEP_STEP_POLLS = 16;
+inline uint32_t sweepPolls(int64_t serial, int sweeps) {
+    return uint32_t(std::min<int64_t>(SWEEP_BASE_POLLS + SWEEP_STEP_POLLS * serial * sweeps, 0xfffffff0));
 }
 
 // off/perm: cells by level (levels off[L] .. off[L+1], ascending cells within a level;
@@ -150,6 +163,7 @@ inline SweepPlanHost buildSweepPlan(int n, const std::vector<int>& off, const st
         s.base = int(total);
         total += size_t(s.width) * size_t(s.rowsNeed & ((1 << SWEEP_ROWS_BITS) - 1));
         P.maxWidth = std::max(P.maxWidth, s.width);
+        P.serial += 1 + s.width / SWEEP_GROUP;
         if (total >= (size_t(1) << 31)) throw std::length_error("sweep rows exceed 2^31 entries");
     }
     again = again && nc > 1;

@@ -540,6 +540,7 @@ struct SweepPlan {
     const int* haloOff = nullptr;
     const int* halo = nullptr;
     int n = 0, nChunks = 0, nSteps = 0, maxSlots = 0, maxWidth = 0;
+    long long serial = 0;
 };
 constexpr int SWEEP_MAX_SWEEPS = 4;  // of one launch over several chunks
 enum SweepOp { SW_GS = 0, SW_FWD = 1, SW_BWD = 2, SW_FAC = 3 };
@@ -551,9 +552,11 @@ template <class T> struct SweepArgs {
     T* x = nullptr;           // result; SW_GS, SW_BWD: updated in place
     bool zero = false;        // SW_GS: x is taken as zero
     // several chunks only: the mailbox (n values per sweep) and the chunk ticket of this
-    // launch, both made ready by launch_sweep_prepare; the flag of timed-out waits
+    // launch, both made ready by launch_sweep_prepare; the limit of a wait (sweepPolls) and
+    // the flag of the ones that ran past it
     T* mail = nullptr;
     int* ticket = nullptr;
+    unsigned polls = 0;
     int* fault = nullptr;
 };
 // m mailbox values and SWEEP_TICKETS tickets made ready
