@@ -171,3 +171,27 @@ def test_long_chain_is_no_timeout(ctx):
         x = np.zeros(n)
         va.solve_ldu(A, b, x, va.SolverControls(solver, pre, 1e-30, 0.0, 1, sums=va.SUMS_EXACT))
         assert np.array_equal(x, xo), solver
+
+
+@pytest.mark.parametrize("solver,pre,prec", [("PCG", "DIC", va.FP64), ("PBiCGStab", "DILU", va.FP64),
+                                             ("PCG", "DIC", va.MIXED), ("GaussSeidel", "none", va.FP64)])
+def test_a_timed_out_solve_leaves_nothing_behind(ctx, monkeypatch, solver, pre, prec):
+    """A solve whose waits run past their limit (here one of a single poll) ends in an error,
+    and the next solve of the same matrix is a fresh one's bit for bit: no factor that the
+    failed one left half done."""
+    n, own, nei = _graph("chain")
+    rng = np.random.default_rng(14)
+    u = -rng.uniform(0.5, 1.5, own.size)
+    d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
+    b = rng.uniform(-1, 1, n)
+    lm = va.LduMesh(ctx, n, own, nei)
+    A, fresh = va.LduMatrix(lm, d, u), va.LduMatrix(lm, d, u)
+    ctl = va.SolverControls(solver, pre, 1e-30, 0.0, 2, precision=prec)
+    monkeypatch.setenv("VOLUMA_SWEEP_POLLS", "1")
+    with pytest.raises(va.VolumaError, match="timed out"):
+        va.solve_ldu(A, b, np.zeros(n), ctl)
+    monkeypatch.delenv("VOLUMA_SWEEP_POLLS")
+    x, want = np.zeros(n), np.zeros(n)
+    p, pw = va.solve_ldu(A, b, x, ctl), va.solve_ldu(fresh, b, want, ctl)
+    assert p.iterations == pw.iterations and p.finalResidual == pw.finalResidual
+    assert np.isfinite(want).all() and np.array_equal(x, want)

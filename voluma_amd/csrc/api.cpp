@@ -594,7 +594,8 @@ template <class T> T* sweepMailbox(vol_context c, hipStream_t st, int n, int swe
     return mail;
 }
 
-// DIC/DILU factor of the matrix (LinearSolver.cpp:66-78) and the substitutions' entries.
+// DIC/DILU factor of the matrix (LinearSolver.cpp:66-78) and the substitutions' entries. It
+// is ready once the solve that builds it has seen that no wait ran past its limit.
 void buildDilu(vol_matrix A) {
     vol_mesh m = A->mesh;
     buildDiluPlans(m);
@@ -614,7 +615,7 @@ void buildDilu(vol_matrix A) {
     if (F.v.nChunks > 1) {
         a.mail = sweepMailbox<double>(c, st, m->n, 1, nullptr);
         a.ticket = c->sweepFault.p + 1;
-        a.polls = sweepPolls(F.v.serial, 1);
+        a.polls = c->waitLimit(F.v, 1);
         a.fault = c->sweepFault.p;
     }
     launch_sweep<double>(st, SW_FAC, false, F.v, a, 1, nullptr);
@@ -625,7 +626,6 @@ void buildDilu(vol_matrix A) {
     launch_vec(st, V_RECIP, v, false, c->red);
     launch_dilu_entries(st, F.v, F.src.p, A->upper.p, lower, A->dluR.p, A->dluEf.p);
     launch_dilu_entries(st, B.v, B.src.p, A->upper.p, lower, A->dluR.p, A->dluEb.p);
-    A->diluReady = true;
     A->dilu32Ready = false;
 }
 
@@ -1481,7 +1481,7 @@ void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T
     for (int s = 0; s < k; s += SWEEP_MAX_SWEEPS) {
         const int q = std::min(k - s, SWEEP_MAX_SWEEPS);
         a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
-        a.polls = sweepPolls(E.v.serial, q);
+        a.polls = C.c->waitLimit(E.v, q);
         launch_sweep<T>(C.st, SW_GS, backward, E.v, a, q, C.done);
         a.zero = false;
     }
@@ -1541,11 +1541,11 @@ void precondApply(const Ctx& C, vol_matrix A, const Plan& P, const T* r, T* w, i
         }
         a.mail = sweepMailbox<T>(C.c, C.st, n, 2, C.done);
         a.ticket = C.c->sweepFault.p + 1;
-        a.polls = sweepPolls(F.serial, 1);
+        a.polls = C.c->waitLimit(F, 1);
         a.fault = C.c->sweepFault.p;
         launch_sweep<T>(C.st, SW_FWD, false, F, a, 1, C.done);
         a.coef = eb;
-        a.polls = sweepPolls(B.serial, 1);
+        a.polls = C.c->waitLimit(B, 1);
         a.mail += n;
         ++a.ticket;
         launch_sweep<T>(C.st, SW_BWD, true, B, a, 1, C.done);
@@ -1741,6 +1741,8 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
     }
     setDevice(c);
     hipStream_t st = c->stream;
+    const char* polls = std::getenv("VOLUMA_SWEEP_POLLS");
+    c->sweepPolls = polls ? std::atoi(polls) : -1;
     DevScalars* scal = ws ? ws->scal : c->scal.p;
     Ctx C{c, st, &scal->done, scal};
     if (ws) {
@@ -1879,6 +1881,7 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
             HIPCHECK(hipMemsetAsync(c->sweepFault.p, 0, sizeof(int), st));
             throw VolError(VOL_ERR_HIP, "triangular sweep: a wait for a neighbour's value timed out");
         }
+        if (dilu) A->diluReady = true;
         if (!hs.done) throw VolError(VOL_ERR_HIP, "solver loop did not terminate");
     }
     collectTiming(c);

@@ -762,6 +762,12 @@ struct vol_context_s {
     // then the chunk tickets; pinned copy of the flag read with a solve's scalars
     DevBuf<int> sweepFault;
     int* hostFault = nullptr;
+    // limit of a wait of theirs; VOLUMA_SWEEP_POLLS=<polls> (read by each solve) replaces the
+    // plan's, so that a solve's time-out can be had without a wait that fails
+    int sweepPolls = -1;
+    uint32_t waitLimit(const SweepPlan& P, int sweeps) const {
+        return sweepPolls >= 0 ? uint32_t(sweepPolls) : vol::sweepPolls(P.serial, sweeps);
+    }
     DevBuf<double> sweepMail;  // their mailbox
     RedScratch red;
     DevBuf<double> part, result;
