@@ -417,7 +417,7 @@ std::vector<host::HLevel> buildHierarchyDevice(hipStream_t st, int n, int nf, co
     }
     std::vector<char> paired;  // per level: its maps are valid
     int passes = 0, rounds = 0;
-    while (D.size() < 40) {
+    while (D.size() < MAX_GAMG_LEVELS) {
         DLevel& F = *D.back();
         const int nF = F.n;
         if (nF <= nCoarsest) break;

@@ -417,9 +417,8 @@ void bsellLaunch(hipStream_t st, int op, int xl, const SellArgs32& a) { launch_s
 
 template <class T>
 void bsell(hipStream_t st, int op, int xl, const SellView& V, const T* coef, const T* diag, const T* rD, const T* x,
-           const T* r, T* out, double omega = 1.0, const T* xc = nullptr, const int* agg = nullptr,
-           const BLevel* skip = nullptr, const DevScalars* S = nullptr, T* pushZ = nullptr,
-           const BLevel* pushTo = nullptr) {
+           const T* r, T* out, double omega = 1.0, const BLevel* skip = nullptr, const DevScalars* S = nullptr,
+           T* pushZ = nullptr, const BLevel* pushTo = nullptr) {
     SellArgsT<T> a;
     if (pushZ) {
         a.pushZ = pushZ;
@@ -437,8 +436,6 @@ void bsell(hipStream_t st, int op, int xl, const SellView& V, const T* coef, con
     a.rD = rD;
     a.x = x;
     a.r = r;
-    a.xc = xc;
-    a.agg = agg;
     a.omega = omega;
     a.out = out;
     bsellLaunch(st, op, xl, a);
@@ -482,7 +479,7 @@ template <class T>
 void bvcycle(vol_batch B, const BPlan& P, const T* r0, T* x0, const DevScalars* S) {
     hipStream_t st = B->ctx->stream;
     const int LM = B->nLevMax;
-    const bool useZ = P.nPre == 1, pushing = LM <= BATCH_PUSH_LEVELS;
+    const bool useZ = P.nPre == 1;
     std::vector<int> curL(LM, 0);
     std::vector<T*> first(LM, nullptr);  // what a level's first post-sweep gathers, before the prolongation
     BatchPush<T> push;
@@ -497,40 +494,35 @@ void bvcycle(vol_batch B, const BPlan& P, const T* r0, T* x0, const DevScalars* 
         for (int s = 1; s < P.nPre; ++s) {
             const int dst = (s == 1) ? 0 : 1 - cur;
             bsell<T>(st, OP_JACOBI, s == 1 ? XL_FROMZERO : XL_PLAIN, V, p.coef, p.diag, p.rD,
-                     s == 1 ? nullptr : bufs[cur], r, bufs[dst], P.omega, nullptr, nullptr, &Lv, S);
+                     s == 1 ? nullptr : bufs[cur], r, bufs[dst], P.omega, &Lv, S);
             cur = dst;
         }
         const int freeB = 1 - cur;
         first[l] = useZ ? p.z : bufs[cur];
-        bsell<T>(st, OP_RESID, XL_PLAIN, V, p.coef, p.diag, p.rD, first[l], r, bufs[freeB], P.omega, nullptr, nullptr,
-                 &Lv, S);
+        bsell<T>(st, OP_RESID, XL_PLAIN, V, p.coef, p.diag, p.rD, first[l], r, bufs[freeB], P.omega, &Lv, S);
         const BLevelPtrs<T> pc = blevel(B, l + 1, (T*)nullptr);
         brestrict(st, B->L[l + 1]->nRows, Lv, bufs[freeB], pc.r, useZ ? pc.z : nullptr, pc.rD, P.omega);
         curL[l] = cur;
         depth = l + 1;
-        if (pushing) {
-            push.z[l + 1] = first[l];
-            push.off[l + 1] = Lv.mOff.p;
-            push.list[l + 1] = Lv.mList.p;
-        }
+        push.z[l + 1] = first[l];
+        push.off[l + 1] = Lv.mOff.p;
+        push.list[l + 1] = Lv.mList.p;
     }
     bcoarse(B, S, push);
     for (int l = depth - 1; l >= 0; --l) {
         BLevel& Lv = *B->L[l];
         const SellView V = Lv.sell.view();
         const BLevelPtrs<T> p = blevel(B, l, (T*)nullptr);
-        const BLevelPtrs<T> pc = blevel(B, l + 1, (T*)nullptr);
         const T* r = l == 0 ? r0 : p.r;
         T* xout = l == 0 ? x0 : p.x;
         T* bufs[2] = {p.bufA, p.bufB};
         int src = curL[l], other = 1 - curL[l];
         for (int s = 0; s < P.nPost; ++s) {
-            const bool last = s == P.nPost - 1, down = last && l > 0 && pushing;  // down: nothing reads this x
+            const bool last = s == P.nPost - 1, down = last && l > 0;  // down: nothing reads this x
             T* dst = down ? nullptr : last ? xout : bufs[other];
             const T* in = s == 0 ? first[l] : bufs[src];
-            bsell<T>(st, OP_JACOBI, s == 0 && !pushing ? XL_PROLONG : XL_PLAIN, V, p.coef, p.diag, p.rD, in, r, dst,
-                     P.omega, pc.x, Lv.agg.p, &Lv, S, down ? first[l - 1] : nullptr,
-                     down ? B->L[l - 1].get() : nullptr);
+            bsell<T>(st, OP_JACOBI, XL_PLAIN, V, p.coef, p.diag, p.rD, in, r, dst, P.omega, &Lv, S,
+                     down ? first[l - 1] : nullptr, down ? B->L[l - 1].get() : nullptr);
             if (!last) std::swap(src, other);
         }
     }
@@ -575,8 +567,8 @@ void bpcgIteration(vol_batch B, const BPlan& P, const BKrylov<T>& k, DevScalars*
     }
     launch_bfinalize(st, FIN_PCG_WRA, 1, B->red, S, nullptr);
     bvec<T>(B, V_PCG_P, S, k.w, nullptr, nullptr, nullptr, k.p);
-    bsell<T>(st, OP_AMUL, XL_PLAIN, B->L[0]->sell.view(), p0.coef, p0.diag, nullptr, k.p, nullptr, k.q, 1.0, nullptr,
-             nullptr, B->L[0].get(), S);
+    bsell<T>(st, OP_AMUL, XL_PLAIN, B->L[0]->sell.view(), p0.coef, p0.diag, nullptr, k.p, nullptr, k.q, 1.0,
+             B->L[0].get(), S);
     bvec<T>(B, V_DOT, S, k.q, k.p);
     launch_bfinalize(st, FIN_PCG_WAPA, 1, B->red, S, nullptr);
     bvec<T>(B, V_PCG_XR, S, k.p, k.q, nullptr, k.z0, k.x, k.r, k.z0 ? p0.rD : nullptr, P.omega);
@@ -748,7 +740,7 @@ void bsolve(vol_batch B, const double* b, double* x, const vol_solver_controls& 
                 bloop(B, maxLoops, [&] { bpcgIteration<float>(B, P, k, SI); }, graphKey(B, P, "mixed", nullptr));
                 launch_bmix(st, MIX_ADD, B->red, S, nullptr, nullptr, nullptr, nullptr, x, B->ie.p);
                 bsell<double>(st, OP_AMUL, XL_PLAIN, V, L0.coef.p, B->diag.p, nullptr, x, nullptr, B->wA.p, 1.0,
-                              nullptr, nullptr, &L0, S);
+                              &L0, S);
                 bvec<double>(B, V_BMINUSAX_NORM, S, B->wA.p, b, nullptr, B->vr.p);
                 launch_bfinalize(st, FIN_OUTER, 1, B->red, S, SI);
                 innerRhs();

@@ -531,7 +531,7 @@ inline std::vector<HLevel> buildHierarchy(int n, int nf, const int* own, const i
     L0.adjacency();
     H.push_back(std::move(L0));
     const int nCoarsest = 64;
-    while (H.size() < 40) {
+    while (H.size() < MAX_GAMG_LEVELS) {
         HLevel& F = H.back();
         const int nF = F.n;
         if (nF <= nCoarsest) break;

@@ -10,6 +10,7 @@
 namespace vol {
 
 constexpr int WAVE = 64;   // CDNA wavefront
+constexpr int MAX_GAMG_LEVELS = 40;  // of a hierarchy, the mesh among them
 constexpr int NBINS = 72;  // exact-sum bins (par::ExactSum::NBINS, Comm.h:44)
 
 // ------------------------------------------------------------------ SELL-64 layout
@@ -639,12 +640,12 @@ void launch_bmix(hipStream_t st, int op, const BatchRed& R, const DevScalars* S,
 // Dense assembly + no-pivot LU of every system's coarsest level (one workgroup each).
 void launch_bcoarse_factor(hipStream_t st, const CoarseDesc* D, int nSys, double* lu, double* luT, int* status);
 // Pushed prolongation of the coarsest solves: a system whose coarsest level is l also adds
-// its x to z[l] over the members list[l][off[l][row] ..] of its rows (z[l] null: it does not).
-constexpr int BATCH_PUSH_LEVELS = 16;
+// its x to z[l] over the members list[l][off[l][row] ..] of its rows (z[l] null: it does
+// not). An entry for every level that a hierarchy may have.
 template <class T> struct BatchPush {
-    T* z[BATCH_PUSH_LEVELS] = {};
-    const int* off[BATCH_PUSH_LEVELS] = {};
-    const int* list[BATCH_PUSH_LEVELS] = {};
+    T* z[MAX_GAMG_LEVELS] = {};
+    const int* off[MAX_GAMG_LEVELS] = {};
+    const int* list[MAX_GAMG_LEVELS] = {};
 };
 // Coarsest substitutions: r and x of system s live at rLev[D.level] + D.rowBase.
 void launch_bcoarse_solve(hipStream_t st, const CoarseDesc* D, int nSys, int maxN, const double* lu,
