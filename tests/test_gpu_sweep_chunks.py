@@ -195,3 +195,25 @@ def test_a_timed_out_solve_leaves_nothing_behind(ctx, monkeypatch, solver, pre, 
     p, pw = va.solve_ldu(A, b, x, ctl), va.solve_ldu(fresh, b, want, ctl)
     assert p.iterations == pw.iterations and p.finalResidual == pw.finalResidual
     assert np.isfinite(want).all() and np.array_equal(x, want)
+
+
+def test_any_number_of_sweeps_over_one_chunk(ctx):
+    """More sweeps than a one-chunk schedule holds go in several launches: the oracle's bits
+    after 20, and 20,000 (as one schedule over 2^31 entries) are taken and converge."""
+    n, (a, b) = 8192, _band(8192, 14, 900, 15)
+    keep = (a < b) & (b < n - 1)
+    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
+    own, nei = (e // n).astype(np.int32), (e % n).astype(np.int32)
+    rng = np.random.default_rng(16)
+    u = -rng.uniform(0.5, 1.5, own.size)
+    d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
+    rhs = rng.uniform(-1, 1, n)
+    lm, om = va.LduMesh(ctx, n, own, nei), O.LduMesh(n, own, nei)
+    A = va.LduMatrix(lm, d, u)
+    xo, _ = om.solve(d, u, None, rhs, x0=np.zeros(n), solver="GaussSeidel", preconditioner="none", tolerance=1e-30,
+                     max_iter=1, n_sweeps=20, mode=O.MODE_EXACT)
+    x = np.zeros(n)
+    va.solve_ldu(A, rhs, x, va.SolverControls("GaussSeidel", "none", 1e-30, 0.0, 1, nSweeps=20, sums=va.SUMS_EXACT))
+    assert np.array_equal(x, xo)
+    p = va.solve_ldu(A, rhs, x, va.SolverControls("GaussSeidel", "none", 1e-12, 0.0, 1, nSweeps=20000))
+    assert p.converged

@@ -692,8 +692,8 @@ void multiSweepOrder(int n, const std::vector<int>& l, const std::vector<int>& u
 }
 
 // The plan of Gauss–Seidel sweeps of GAMG level lvl (0: the mesh) in one direction, built
-// on first use: with one chunk the k sweeps as one pipelined schedule, else a single sweep
-// (k = 1).
+// on first use: with one chunk the k ≤ SWEEP_ONE_SWEEPS sweeps as one pipelined schedule,
+// else a single sweep (k = 1).
 const SweepPlanDev& gsPlan(vol_mesh m, int lvl, bool backward, int k) {
     std::lock_guard<std::mutex> guard(m->sweepMu);
     auto& slot = m->gsPlans[{lvl, backward ? 1 : 0, k}];
@@ -1465,24 +1465,23 @@ template <class T>
 void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T* diag, const T* b, T* x, int n,
               bool fromZero) {
     const bool one = n <= SWEEP_ONE_CELLS;
-    const SweepPlanDev& E = gsPlan(A->mesh, lvl, backward, one ? k : 1);
+    const int most = one ? SWEEP_ONE_SWEEPS : SWEEP_MAX_SWEEPS;
     SweepArgs<T> a;
-    a.coef = gsPlanCoef<T>(A, E, lvl, backward, one ? k : 1);
     a.b = b;
     a.diag = diag;
     a.x = x;
     a.zero = fromZero;
-    if (one) {
-        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, 1, C.done);
-        return;
-    }
     a.ticket = C.c->sweepFault.p + 1;
     a.fault = C.c->sweepFault.p;
-    for (int s = 0; s < k; s += SWEEP_MAX_SWEEPS) {
-        const int q = std::min(k - s, SWEEP_MAX_SWEEPS);
-        a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
-        a.polls = C.c->waitLimit(E.v, q);
-        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, q, C.done);
+    for (int s = 0; s < k; s += most) {
+        const int q = std::min(k - s, most);
+        const SweepPlanDev& E = gsPlan(A->mesh, lvl, backward, one ? q : 1);
+        a.coef = gsPlanCoef<T>(A, E, lvl, backward, one ? q : 1);
+        if (!one) {
+            a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
+            a.polls = C.c->waitLimit(E.v, q);
+        }
+        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, one ? 1 : q, C.done);
         a.zero = false;
     }
 }

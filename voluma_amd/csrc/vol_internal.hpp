@@ -544,6 +544,7 @@ struct SweepPlan {
     long long serial = 0;
 };
 constexpr int SWEEP_MAX_SWEEPS = 4;  // of one launch over several chunks
+constexpr int SWEEP_ONE_SWEEPS = 8;  // of one launch over one chunk, whose plan lists each of them
 enum SweepOp { SW_GS = 0, SW_FWD = 1, SW_BWD = 2, SW_FAC = 3 };
 template <class T> struct SweepArgs {
     const T* coef = nullptr;  // per entry of the plan
