@@ -618,7 +618,7 @@ void buildDilu(vol_matrix A) {
         a.polls = c->waitLimit(F.v, 1);
         a.fault = c->sweepFault.p;
     }
-    launch_sweep<double>(st, SW_FAC, false, F.v, a, 1, nullptr);
+    HIPCHECK(launch_sweep<double>(st, SW_FAC, false, F.v, a, 1, nullptr));
     VecArgs v;
     v.n = m->n;
     v.a = A->dluD.p;
@@ -1481,7 +1481,7 @@ void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T
             a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
             a.polls = C.c->waitLimit(E.v, q);
         }
-        launch_sweep<T>(C.st, SW_GS, backward, E.v, a, one ? 1 : q, C.done);
+        HIPCHECK(launch_sweep<T>(C.st, SW_GS, backward, E.v, a, one ? 1 : q, C.done));
         a.zero = false;
     }
 }
@@ -1535,19 +1535,19 @@ void precondApply(const Ctx& C, vol_matrix A, const Plan& P, const T* r, T* w, i
         a.b = r;
         a.x = w;
         if (F.nChunks == 1) {
-            launch_dilu_one<T>(C.st, F, B, a, eb, C.done);
+            HIPCHECK(launch_dilu_one<T>(C.st, F, B, a, eb, C.done));
             return;
         }
         a.mail = sweepMailbox<T>(C.c, C.st, n, 2, C.done);
         a.ticket = C.c->sweepFault.p + 1;
         a.polls = C.c->waitLimit(F, 1);
         a.fault = C.c->sweepFault.p;
-        launch_sweep<T>(C.st, SW_FWD, false, F, a, 1, C.done);
+        HIPCHECK(launch_sweep<T>(C.st, SW_FWD, false, F, a, 1, C.done));
         a.coef = eb;
         a.polls = C.c->waitLimit(B, 1);
         a.mail += n;
         ++a.ticket;
-        launch_sweep<T>(C.st, SW_BWD, true, B, a, 1, C.done);
+        HIPCHECK(launch_sweep<T>(C.st, SW_BWD, true, B, a, 1, C.done));
     } else
         vec<T>(C, V_SCALE, n, false, r, nullptr, nullptr, nullptr, w, nullptr, nullptr,
                P.precond == "diagonal" ? level0(A, (T*)nullptr).rD : nullptr);

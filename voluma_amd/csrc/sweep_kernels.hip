@@ -42,6 +42,8 @@
 #include "device_common.hpp"
 #include "vol_internal.hpp"
 
+#include <atomic>
+
 namespace vol {
 
 namespace {
@@ -464,14 +466,23 @@ template <class T> void launch_sweep_prepare(hipStream_t st, size_t m, T* mail, 
 template void launch_sweep_prepare<double>(hipStream_t, size_t, double*, int*, const int*);
 template void launch_sweep_prepare<float>(hipStream_t, size_t, float*, int*, const int*);
 
-// Launch with dynamic LDS beyond the default limit.
+// Launch with dynamic LDS beyond the default limit, which is raised once per device.
 template <auto Kernel, class... A>
-static void launch_lds(int blocks, int threads, size_t lds, hipStream_t st, A... args) {
-    static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int((SWEEP_MAX_SLOTS + 1) * sizeof(double)));
-    (void)attr;
-    hipLaunchKernelGGL(Kernel, dim3(blocks), dim3(threads), lds, st, args...);
+static hipError_t launch_lds(int blocks, int threads, size_t lds, hipStream_t st, A... args) {
+    static std::atomic<unsigned long long> raised{0};  // a bit per device
+    const void* const f = reinterpret_cast<const void*>(Kernel);
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+    if (!(raised.load(std::memory_order_relaxed) & bit)) {
+        e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int((SWEEP_MAX_SLOTS + 1) * sizeof(double)));
+        if (e != hipSuccess) return e;
+        raised.fetch_or(bit, std::memory_order_relaxed);
+    }
+    void* p[] = {&args...};
+    return hipLaunchKernel(f, dim3(blocks), dim3(threads), p, lds, st);
 }
 
 // Rows of at most 8 entries (mesh cells) run 16 wavefronts; longer ones (coarse GAMG
@@ -479,56 +490,54 @@ static void launch_lds(int blocks, int threads, size_t lds, hipStream_t st, A...
 // chunks beside them; entries past that cost a memory round trip inside the dependence:
 // a level of 5,739 cells with up to 24 took 365 µs with 16 held and 220 with 20).
 template <int OP, bool BACK, class T>
-static void launch_sweep_t(hipStream_t st, const SweepPlan& P, const SweepArgs<T>& a, int sweeps, const int* done) {
+static hipError_t launch_sweep_t(hipStream_t st, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
+                                 const int* done) {
     const size_t lds = (size_t(P.maxSlots) + 1) * sizeof(T);
+    const int blocks = P.nChunks * sweeps;
     if (P.nChunks > 1) {
         if (P.maxWidth <= 8)
-            launch_lds<k_sweep_chunks<OP, BACK, 8, 16, T>>(P.nChunks * sweeps, 16 * WAVE, lds, st, P, a, sweeps, done);
-        else if (P.maxWidth <= 12)
-            launch_lds<k_sweep_chunks<OP, BACK, 12, 8, T>>(P.nChunks * sweeps, 8 * WAVE, lds, st, P, a, sweeps, done);
-        else
-            launch_lds<k_sweep_chunks<OP, BACK, 20, 8, T>>(P.nChunks * sweeps, 8 * WAVE, lds, st, P, a, sweeps, done);
-    } else {
-        if (P.maxWidth <= 8)
-            launch_lds<k_sweep_one<OP, 8, 16, T>>(1, 16 * WAVE, lds, st, P, a, done);
-        else
-            launch_lds<k_sweep_one<OP, 24, 8, T>>(1, 8 * WAVE, lds, st, P, a, done);
+            return launch_lds<k_sweep_chunks<OP, BACK, 8, 16, T>>(blocks, 16 * WAVE, lds, st, P, a, sweeps, done);
+        if (P.maxWidth <= 12)
+            return launch_lds<k_sweep_chunks<OP, BACK, 12, 8, T>>(blocks, 8 * WAVE, lds, st, P, a, sweeps, done);
+        return launch_lds<k_sweep_chunks<OP, BACK, 20, 8, T>>(blocks, 8 * WAVE, lds, st, P, a, sweeps, done);
     }
+    if (P.maxWidth <= 8) return launch_lds<k_sweep_one<OP, 8, 16, T>>(1, 16 * WAVE, lds, st, P, a, done);
+    return launch_lds<k_sweep_one<OP, 24, 8, T>>(1, 8 * WAVE, lds, st, P, a, done);
 }
 
 template <class T>
-void launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
-                  const int* done) {
-    if (P.n <= 0) return;
+hipError_t launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
+                        const int* done) {
+    if (P.n <= 0) return hipSuccess;
     switch (op) {
     case SW_GS:
-        if (backward) launch_sweep_t<SW_GS, true, T>(st, P, a, sweeps, done);
-        else launch_sweep_t<SW_GS, false, T>(st, P, a, sweeps, done);
-        break;
-    case SW_FWD: launch_sweep_t<SW_FWD, false, T>(st, P, a, sweeps, done); break;
-    case SW_BWD: launch_sweep_t<SW_BWD, true, T>(st, P, a, sweeps, done); break;
+        return backward ? launch_sweep_t<SW_GS, true, T>(st, P, a, sweeps, done)
+                        : launch_sweep_t<SW_GS, false, T>(st, P, a, sweeps, done);
+    case SW_FWD: return launch_sweep_t<SW_FWD, false, T>(st, P, a, sweeps, done);
+    case SW_BWD: return launch_sweep_t<SW_BWD, true, T>(st, P, a, sweeps, done);
     default:
-        if constexpr (std::is_same_v<T, double>) launch_sweep_t<SW_FAC, false, T>(st, P, a, sweeps, done);
-        break;
+        if constexpr (std::is_same_v<T, double>) return launch_sweep_t<SW_FAC, false, T>(st, P, a, sweeps, done);
+        return hipErrorInvalidValue;
     }
 }
-template void launch_sweep<double>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<double>&, int, const int*);
-template void launch_sweep<float>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<float>&, int, const int*);
+template hipError_t launch_sweep<double>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<double>&, int,
+                                         const int*);
+template hipError_t launch_sweep<float>(hipStream_t, int, bool, const SweepPlan&, const SweepArgs<float>&, int,
+                                        const int*);
 
 template <class T>
-void launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B, const SweepArgs<T>& a, const T* eb,
-                     const int* done) {
-    if (F.n <= 0) return;
+hipError_t launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B, const SweepArgs<T>& a, const T* eb,
+                           const int* done) {
+    if (F.n <= 0) return hipSuccess;
     const size_t lds = (size_t(F.n) + 1) * sizeof(T);
     if (std::max(F.maxWidth, B.maxWidth) <= 8)
-        launch_lds<k_dilu_one<8, 16, T>>(1, 16 * WAVE, lds, st, F, B, a, eb, done);
-    else
-        launch_lds<k_dilu_one<24, 8, T>>(1, 8 * WAVE, lds, st, F, B, a, eb, done);
+        return launch_lds<k_dilu_one<8, 16, T>>(1, 16 * WAVE, lds, st, F, B, a, eb, done);
+    return launch_lds<k_dilu_one<24, 8, T>>(1, 8 * WAVE, lds, st, F, B, a, eb, done);
 }
-template void launch_dilu_one<double>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<double>&,
-                                      const double*, const int*);
-template void launch_dilu_one<float>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<float>&,
-                                     const float*, const int*);
+template hipError_t launch_dilu_one<double>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<double>&,
+                                            const double*, const int*);
+template hipError_t launch_dilu_one<float>(hipStream_t, const SweepPlan&, const SweepPlan&, const SweepArgs<float>&,
+                                           const float*, const int*);
 
 // Entries of the DIC/DILU factor and substitutions, a wavefront per step. src[e] is a
 // face with its side of the row's own cell (f << 1 | side, 0: upper, 1: lower holds the

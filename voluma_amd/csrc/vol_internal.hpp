@@ -566,12 +566,12 @@ constexpr int SWEEP_TICKETS = 2;
 template <class T> void launch_sweep_prepare(hipStream_t st, size_t m, T* mail, int* tickets, const int* done);
 // `sweeps` sweeps over several chunks; a one-chunk plan holds its whole schedule (sweeps = 1)
 template <class T>
-void launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P, const SweepArgs<T>& a, int sweeps,
-                  const int* done);
+[[nodiscard]] hipError_t launch_sweep(hipStream_t st, int op, bool backward, const SweepPlan& P,
+                                      const SweepArgs<T>& a, int sweeps, const int* done);
 // Forward and backward substitution of one-chunk plans in one launch (a.coef: forward entries)
 template <class T>
-void launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B, const SweepArgs<T>& a, const T* eb,
-                     const int* done);
+[[nodiscard]] hipError_t launch_dilu_one(hipStream_t st, const SweepPlan& F, const SweepPlan& B,
+                                         const SweepArgs<T>& a, const T* eb, const int* done);
 // Entries of the DIC/DILU factor (rD null) and substitutions in a plan's layout
 void launch_dilu_entries(hipStream_t st, const SweepPlan& P, const int* src, const double* upper, const double* lower,
                          const double* rD, double* out);
