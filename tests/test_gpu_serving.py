@@ -207,3 +207,32 @@ def test_bench_pool_same_alone_and_in_the_mix(bench_pool, precision):
         for a, b in zip(xa, xm):
             assert np.array_equal(a, b), k
     server.close()
+
+
+def _chain_server(n, budget_copies):
+    """A server of one worker with two meshes of n cells in a row (no hierarchy), whose
+    budget holds the registered meshes and that many resident copies."""
+    own, nei = np.arange(n - 1, dtype=np.int32), np.arange(1, n, dtype=np.int32)
+    est = n * 400 + (n - 1) * 96 + (1 << 20)
+    server = va.Server(0, slots=1, hbm_budget=est * (1 + budget_copies) + 1000)
+    ids = [server.add_mesh(n, own, nei) for _ in range(2)]
+    d, u, b = np.full(n, 2.5), np.full(n - 1, -1.0), np.ones(n)
+
+    def bytes_after(mesh, solver, pre):
+        server.wait(server.submit(mesh, d, u, None, [b], controls=va.SolverControls(solver, pre, 1e-8)))
+        return server.stats()["bytes_in_use"]
+
+    return server, ids, bytes_after
+
+
+def test_budget_gives_back_what_an_evicted_entry_held():
+    """A mesh that goes and comes back is charged the same both times: the workspace of its
+    sweeps (20,000 cells: several chunks) goes with it."""
+    server, (a, b), bytes_after = _chain_server(20000, 1)
+    bytes_after(a, "PCG", "diagonal")  # the worker's own scratch is charged here
+    seen = []
+    for _ in range(2):
+        bytes_after(b, "PCG", "diagonal")  # does not fit beside a
+        seen.append(bytes_after(a, "PCG", "DIC"))
+    assert seen[0] == seen[1]
+    server.close()

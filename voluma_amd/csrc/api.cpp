@@ -112,6 +112,7 @@ struct vol_mesh_s {
     std::mutex sweepMu;
     std::unique_ptr<SweepPlanDev> diluF, diluB;
     std::map<std::tuple<int, int, int>, std::unique_ptr<SweepPlanDev>> gsPlans;
+    DevBuf<double> sweepMail;  // mailbox of sweeps over several chunks, theirs one after the other
     // geometry of the explicit corrector operators (vol_mesh_set_geometry) and their
     // staging buffers for host pointers
     bool geomSet = false;
@@ -586,11 +587,11 @@ void buildDiluPlans(vol_mesh m) {
 
 // The mailbox of `sweeps` sweeps over n cells (several chunks) and the tickets of up to
 // SWEEP_TICKETS launches made ready in stream order.
-template <class T> T* sweepMailbox(vol_context c, hipStream_t st, int n, int sweeps, const int* done) {
+template <class T> T* sweepMailbox(vol_mesh mesh, hipStream_t st, int n, int sweeps, const int* done) {
     const size_t m = size_t(n) * sweeps;
-    c->sweepMail.alloc((m * sizeof(T) + sizeof(double) - 1) / sizeof(double));
-    T* mail = reinterpret_cast<T*>(c->sweepMail.p);
-    launch_sweep_prepare<T>(st, m, mail, c->sweepFault.p + 1, done);
+    mesh->sweepMail.alloc((m * sizeof(T) + sizeof(double) - 1) / sizeof(double));
+    T* mail = reinterpret_cast<T*>(mesh->sweepMail.p);
+    launch_sweep_prepare<T>(st, m, mail, mesh->ctx->sweepFault.p + 1, done);
     return mail;
 }
 
@@ -613,7 +614,7 @@ void buildDilu(vol_matrix A) {
     a.diag = A->diag.p;
     a.x = A->dluD.p;
     if (F.v.nChunks > 1) {
-        a.mail = sweepMailbox<double>(c, st, m->n, 1, nullptr);
+        a.mail = sweepMailbox<double>(m, st, m->n, 1, nullptr);
         a.ticket = c->sweepFault.p + 1;
         a.polls = c->waitLimit(F.v, 1);
         a.fault = c->sweepFault.p;
@@ -1478,7 +1479,7 @@ void gsSweeps(const Ctx& C, vol_matrix A, int lvl, bool backward, int k, const T
         const SweepPlanDev& E = gsPlan(A->mesh, lvl, backward, one ? q : 1);
         a.coef = gsPlanCoef<T>(A, E, lvl, backward, one ? q : 1);
         if (!one) {
-            a.mail = sweepMailbox<T>(C.c, C.st, n, q, C.done);
+            a.mail = sweepMailbox<T>(A->mesh, C.st, n, q, C.done);
             a.polls = C.c->waitLimit(E.v, q);
         }
         HIPCHECK(launch_sweep<T>(C.st, SW_GS, backward, E.v, a, one ? 1 : q, C.done));
@@ -1538,7 +1539,7 @@ void precondApply(const Ctx& C, vol_matrix A, const Plan& P, const T* r, T* w, i
             HIPCHECK(launch_dilu_one<T>(C.st, F, B, a, eb, C.done));
             return;
         }
-        a.mail = sweepMailbox<T>(C.c, C.st, n, 2, C.done);
+        a.mail = sweepMailbox<T>(m, C.st, n, 2, C.done);
         a.ticket = C.c->sweepFault.p + 1;
         a.polls = C.c->waitLimit(F, 1);
         a.fault = C.c->sweepFault.p;

@@ -768,7 +768,6 @@ struct vol_context_s {
     uint32_t waitLimit(const SweepPlan& P, int sweeps) const {
         return sweepPolls >= 0 ? uint32_t(sweepPolls) : vol::sweepPolls(P.serial, sweeps);
     }
-    DevBuf<double> sweepMail;  // their mailbox
     RedScratch red;
     DevBuf<double> part, result;
     DevBuf<long long> xpart;
