@@ -236,3 +236,17 @@ def test_budget_gives_back_what_an_evicted_entry_held():
         seen.append(bytes_after(a, "PCG", "DIC"))
     assert seen[0] == seen[1]
     server.close()
+
+
+def test_budget_follows_what_an_entry_gives_back():
+    """Requests in turn with and without Gauss–Seidel sweeps on one mesh: each new matrix
+    gives the sweeps' coefficients of the one before back, and they are not charged again
+    on top."""
+    server, (a, _), bytes_after = _chain_server(20000, 4)
+    bytes_after(a, "GaussSeidel", "none")
+    bytes_after(a, "PCG", "diagonal")
+    seen = []
+    for _ in range(3):
+        seen.append((bytes_after(a, "GaussSeidel", "none"), bytes_after(a, "PCG", "diagonal")))
+    assert seen[0] == seen[1] == seen[2] and seen[0][0] > seen[0][1]
+    server.close()

@@ -149,18 +149,16 @@ bool admit(vol_server S, Worker& w, Req* q) {
 }
 
 // Finishes a group of requests (under the lock). grown: device bytes the entry's
-// allocations added while the group ran. When the measured size pushes the total over
+// allocations added while the group ran (negative: gave back, as a new matrix does with
+// the sweep coefficients of the one before). When the measured size pushes the total over
 // the budget, idle entries of the worker go, least recently used first.
 void finish(vol_server S, Worker& w, CacheEntry* e, const std::vector<Req*>& group, int rc, const std::string& err,
             int64_t grown) {
     std::lock_guard<std::mutex> lk(S->mu);
     const uint64_t was = e->bytes;
-    if (!e->measured) {  // the reservation becomes the measured size
-        e->bytes = uint64_t(std::max<int64_t>(grown, 0));
-        e->measured = true;
-    } else if (grown > 0) {
-        e->bytes += uint64_t(grown);
-    }
+    // the first time the reservation becomes the measured size
+    e->bytes = uint64_t(std::max<int64_t>((e->measured ? int64_t(was) : 0) + grown, 0));
+    e->measured = true;
     S->inUse = S->inUse - was + e->bytes;
     while (S->inUse > S->budget) {
         auto victim = w.cache.end();
