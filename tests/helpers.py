@@ -17,6 +17,50 @@ SMALL_MESHES = {
 }
 
 
+def band(n, deg, width, seed):
+    """Faces between cells at most width apart, deg / 2 per cell; what would lie past the last
+    cell ends at it (a long row)."""
+    rng = np.random.default_rng(seed)
+    a = rng.integers(0, n - 1, n * deg // 2)
+    b = np.minimum(a + 1 + rng.integers(0, width, a.size), n - 1)
+    return a, b
+
+
+def sweep_graph(name):
+    """(cells, owner, neighbour) of graphs at the edges of the sweep plans: the largest
+    one-chunk size and its neighbour, a chain (one row per level), rows of every length the
+    kernels treat apart (up to 8, 12 and 20 entries, longer ones, a hub of hundreds), and
+    neighbours anywhere: ``far`` has large halos (16 chunks, 12,993 of 20,400 slots forward;
+    backward over 10,000 values lie past them), in ``scattered`` both directions run over."""
+    rng = np.random.default_rng(5)
+    if name == "chain":
+        n = 8193
+        a, b = np.arange(n - 1), np.arange(1, n)
+    elif name == "one":
+        n, (a, b) = 8192, band(8192, 6, 300, 1)
+    elif name == "two":
+        n, (a, b) = 8193, band(8193, 6, 300, 2)
+    elif name == "wide":
+        n, (a, b) = 12345, band(12345, 14, 900, 3)
+    elif name == "far":
+        n, (a, b) = 30000, band(30000, 16, 30000, 4)
+    elif name == "scattered":
+        n, (a, b) = 100_003, band(100_003, 16, 100_003, 8)
+    elif name == "hub":
+        n, (a, b) = 9001, band(9001, 5, 200, 6)
+        a = np.concatenate([a, np.full(400, 4500), rng.integers(0, 4500, 400)])
+        b = np.concatenate([b, 4501 + rng.permutation(4500)[:400], np.full(400, 4500)])
+    else:
+        m = M.box(23, 21, 19)
+        return m.n_cells, m.owner[: m.n_internal], m.neighbour
+    keep = a < b
+    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
+    rng.shuffle(e)  # face order unrelated to cell order
+    flip = rng.random(e.size) < 0.3  # faces owned by the higher cell too
+    l, u = (e // n).astype(np.int32), (e % n).astype(np.int32)
+    return n, np.where(flip, u, l), np.where(flip, l, u)
+
+
 def sha(a):
     return hashlib.sha256(np.ascontiguousarray(a).tobytes()).hexdigest()
 

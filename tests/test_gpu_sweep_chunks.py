@@ -1,53 +1,15 @@
 """Triangular sweeps over one and several chunks against the oracle's sequential loops, bit
-for bit (exact sums), on graphs at the edges of the sweep plans: the largest one-chunk
-size and its neighbour, a chain (one row per level), rows of every length the kernels
-treat apart (up to 8, 12 and 20 entries, longer ones, a hub of hundreds), neighbours so
-scattered that a chunk's halo does not fit its LDS, and more sweeps than one launch takes.
+for bit (exact sums), on the graphs of ``helpers.sweep_graph`` and with more sweeps than one
+launch takes.
 """
 import numpy as np
 import pytest
 
 import voluma_amd as va
+from helpers import band, sweep_graph
 from oracle import oracle as O
-from voluma_amd import mesh as M
 
 pytestmark = pytest.mark.gpu
-
-
-def _band(n, deg, width, seed):
-    rng = np.random.default_rng(seed)
-    a = rng.integers(0, n - 1, n * deg // 2)
-    b = np.minimum(a + 1 + rng.integers(0, width, a.size), n - 1)
-    return a, b
-
-
-def _graph(name):
-    rng = np.random.default_rng(5)
-    if name == "chain":
-        n = 8193
-        a, b = np.arange(n - 1), np.arange(1, n)
-    elif name == "one":
-        n, (a, b) = 8192, _band(8192, 6, 300, 1)
-    elif name == "two":
-        n, (a, b) = 8193, _band(8193, 6, 300, 2)
-    elif name == "wide":
-        n, (a, b) = 12345, _band(12345, 14, 900, 3)
-    elif name == "far":  # neighbours anywhere: 4096-cell chunks see over 16,300 other cells
-        n = 30000
-        a, b = _band(n, 16, n, 4)
-    elif name == "hub":
-        n, (a, b) = 9001, _band(9001, 5, 200, 6)
-        a = np.concatenate([a, np.full(400, 4500), rng.integers(0, 4500, 400)])
-        b = np.concatenate([b, 4501 + rng.permutation(4500)[:400], np.full(400, 4500)])
-    else:
-        m = M.box(23, 21, 19)
-        return m.n_cells, m.owner[: m.n_internal], m.neighbour
-    keep = a < b
-    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
-    rng.shuffle(e)  # face order unrelated to cell order
-    flip = rng.random(e.size) < 0.3  # faces owned by the higher cell too
-    l, u = (e // n).astype(np.int32), (e % n).astype(np.int32)
-    return n, np.where(flip, u, l), np.where(flip, l, u)
 
 
 @pytest.fixture(scope="module")
@@ -59,7 +21,7 @@ def ctx():
 
 @pytest.mark.parametrize("name", ["chain", "one", "two", "wide", "far", "hub", "box"])
 def test_sweeps_bit_exact_vs_oracle(ctx, name):
-    n, own, nei = _graph(name)
+    n, own, nei = sweep_graph(name)
     rng = np.random.default_rng(9)
     nf = own.size
     u = -rng.uniform(0.5, 1.5, nf)
@@ -84,25 +46,25 @@ def test_sweeps_bit_exact_vs_oracle(ctx, name):
 
 def test_values_before_the_sweep_past_the_halo(ctx):
     """Enough chunks of long scattered rows that a chunk's neighbours do not fit its LDS:
-    what is left of them is read where it lies, from x and from zero."""
-    n = 100_003
-    a, b = _band(n, 16, n, 8)
-    keep = a < b
-    e = np.unique(a[keep].astype(np.int64) * n + b[keep])
-    own, nei = (e // n).astype(np.int32), (e % n).astype(np.int32)
+    what is left of them is read where it lies, from x (at the start of every four sweeps)
+    and, in the GAMG smoother's first sweeps, from the zero that x is taken as."""
+    n, own, nei = sweep_graph("scattered")
     rng = np.random.default_rng(10)
-    u = -rng.uniform(0.5, 1.5, e.size)
+    u = -rng.uniform(0.5, 1.5, own.size)
     d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
     rhs, x0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
-    lm = va.LduMesh(ctx, n, own, nei)
-    om = O.LduMesh(n, own, nei)
+    w = rng.uniform(0.5, 1.5, own.size)
+    lm, om = va.LduMesh(ctx, n, own, nei, w, 20), O.LduMesh(n, own, nei, w, 20)  # the graph, then the coarsest
     A = va.LduMatrix(lm, d, u)
-    for start in (x0, np.zeros(n)):
-        xo, _ = om.solve(d, u, None, rhs, x0=start, solver="symGaussSeidel", preconditioner="none", tolerance=1e-30,
-                         max_iter=2, mode=O.MODE_EXACT)
-        x = start.copy()
-        va.solve_ldu(A, rhs, x, va.SolverControls("symGaussSeidel", "none", 1e-30, 0.0, 2, sums=va.SUMS_EXACT))
-        assert np.array_equal(x, xo)
+    for solver, pre, sweeps, mx in (("GaussSeidel", "none", 2, 4), ("GaussSeidel", "none", 5, 5),
+                                    ("symGaussSeidel", "none", 1, 2), ("PCG", "GAMG", 1, 2)):
+        xo, po = om.solve(d, u, None, rhs, x0=x0, solver=solver, preconditioner=pre, tolerance=1e-30, max_iter=mx,
+                          n_sweeps=sweeps, mode=O.MODE_EXACT, smoother=O.SMOOTHER_GS)
+        x = x0.copy()
+        p = va.solve_ldu(A, rhs, x, va.SolverControls(solver, pre, 1e-30, 0.0, mx, nSweeps=sweeps,
+                                                      sums=va.SUMS_EXACT, gamgSmoother=va.GAMG_GAUSS_SEIDEL))
+        assert p.iterations == po["iterations"] and p.finalResidual == po["finalResidual"], (solver, sweeps)
+        assert np.array_equal(x, xo), (solver, sweeps)
 
 
 @pytest.mark.parametrize("name", ["one", "two"])
@@ -110,7 +72,7 @@ def test_values_before_the_sweep_past_the_halo(ctx):
 def test_row_division_over_the_exponent_range(ctx, name, powers):
     """Rows scaled by powers of two on both sides of the range in which a step divides with
     the reciprocal, and zero numerators of both signs: the oracle's quotients bit for bit."""
-    n, own, nei = _graph(name)
+    n, own, nei = sweep_graph(name)
     rng = np.random.default_rng(11)
     s = 2.0 ** rng.choice(powers, n)
     u, lo = -rng.uniform(0.5, 1.5, own.size), -rng.uniform(0.5, 1.5, own.size)
@@ -134,7 +96,7 @@ def test_row_division_over_the_exponent_range(ctx, name, powers):
 def test_infinite_coefficients_keep_the_loops_signs(ctx, name):
     """Infinite coefficients on faces of a chunk whose rows also read other chunks' values:
     every infinity and every NaN of the sequential loop, and its bits elsewhere."""
-    n, own, nei = _graph(name)
+    n, own, nei = sweep_graph(name)
     rng = np.random.default_rng(12)
     u, lo = -rng.uniform(0.5, 1.5, own.size), -rng.uniform(0.5, 1.5, own.size)
     d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -lo, n)
@@ -179,7 +141,7 @@ def test_a_timed_out_solve_leaves_nothing_behind(ctx, monkeypatch, solver, pre, 
     """A solve whose waits run past their limit (here one of a single poll) ends in an error,
     and the next solve of the same matrix is a fresh one's bit for bit: no factor that the
     failed one left half done."""
-    n, own, nei = _graph("chain")
+    n, own, nei = sweep_graph("chain")
     rng = np.random.default_rng(14)
     u = -rng.uniform(0.5, 1.5, own.size)
     d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
@@ -200,7 +162,7 @@ def test_a_timed_out_solve_leaves_nothing_behind(ctx, monkeypatch, solver, pre, 
 def test_any_number_of_sweeps_over_one_chunk(ctx):
     """More sweeps than a one-chunk schedule holds go in several launches: the oracle's bits
     after 20, and 20,000 (as one schedule over 2^31 entries) are taken and converge."""
-    n, (a, b) = 8192, _band(8192, 14, 900, 15)
+    n, (a, b) = 8192, band(8192, 14, 900, 15)
     keep = (a < b) & (b < n - 1)
     e = np.unique(a[keep].astype(np.int64) * n + b[keep])
     own, nei = (e // n).astype(np.int32), (e % n).astype(np.int32)

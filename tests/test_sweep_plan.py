@@ -3,7 +3,10 @@ address and undefined-behaviour sanitizers (sweep_plan_check.cpp)."""
 import os
 import subprocess
 
+import numpy as np
 import pytest
+
+from helpers import sweep_graph
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "..", "voluma_amd", "csrc")
@@ -32,3 +35,31 @@ def test_wait_limit_covers_every_step_in_turn(check, n):
     got = check("limit", n)
     assert got["steps"] == n and got["chunks"] > 1
     assert got["polls"] * 0.3 >= 10 * 0.4 * n
+
+
+def _write(path, n, own, nei):
+    l, u = np.minimum(own, nei), np.maximum(own, nei)
+    with open(path, "wb") as f:
+        f.write(b"".join(np.asarray(a, np.int32).tobytes() for a in ([n, l.size], l, u)))
+    return path
+
+
+SMALL = {"cell": (1, [], []), "apart": (3, [], []), "pair": (2, [0], [1]), "row": (100, range(99), range(1, 100))}
+
+
+@pytest.mark.parametrize("name", list(SMALL) + ["chain", "one", "two", "wide", "far", "hub", "box", "scattered"])
+@pytest.mark.parametrize("backward", [0, 1])
+def test_plan_gives_the_sequential_loop(check, tmp_path, name, backward):
+    """A plan worked through as the kernels do it (chunk by chunk, the steps of a level in
+    either order, x copied as early or as late as it may be) reads only what is there by
+    then and gives the sequential loop's bits: one sweep, several in one launch, and a
+    substitution, in as many chunks as the rule makes and in others."""
+    small = name in SMALL
+    f = _write(tmp_path / "faces", *(SMALL[name] if small else sweep_graph(name)))
+    for sweeps, old in ((1, 1), (2, 1), (1, 0)) if name == "scattered" else ((1, 1), (2, 1), (4, 1), (1, 0)):
+        for chunks in (0, 1, 2, 7, 70) if small else (0,):
+            got = check("sweep", f, backward, sweeps, chunks, old)
+            if name in ("one", "two"):
+                assert (got["chunks"] == 1) == (name == "one")
+            if name in ("far", "scattered") and old:  # values past the halo
+                assert (got["fromx"] > 10000) == (name == "scattered" or backward == 1)
