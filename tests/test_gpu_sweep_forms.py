@@ -1,76 +1,154 @@
-"""GPU tests of the two forms of the triangular sweeps (Gauss–Seidel solver and GAMG
-smoother, DIC/DILU substitutions): level-scheduled (a launch per level or per run of
-short levels; the default, VOLUMA_SWEEP=levels) and sync-free (one launch per sweep, each
-row waiting for the new values of its neighbours on the sweep's side; VOLUMA_SWEEP=free).
-Each row's arithmetic is the same in both, so solutions, iteration counts and residuals
-must be bit-identical, in FP64 and mixed precision."""
-import os
+"""The triangular sweeps over several chunks in both precisions, against sequential loops.
 
+FP64 with exact sums: the oracle's bits on mid-size meshes, every solver and preconditioner
+that sweeps. FP32 (the inner solve of mixed precision): cut after its first iteration a
+mixed PCG returns x = α·p with p = M⁻¹ b in FP32, so every element must round to one and
+the same α times the p of a sequential float32 loop in numpy; an element that is off by a
+unit in the last place leaves no such α.
+"""
 import numpy as np
 import pytest
 
 import voluma_amd as va
+from helpers import sweep_graph
+from oracle import oracle as O
 from voluma_amd import mesh as M
 from voluma_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
+F = np.float32
 
 
-def _context(sweep):
-    old = os.environ.get("VOLUMA_SWEEP")
-    try:
-        os.environ["VOLUMA_SWEEP"] = sweep
-        return va.Context(0)
-    finally:
-        if old is None:
-            os.environ.pop("VOLUMA_SWEEP", None)
-        else:
-            os.environ["VOLUMA_SWEEP"] = old
+@pytest.fixture(scope="module")
+def ctx():
+    c = va.Context(0)
+    yield c
+    c.close()
 
 
-def _gs_gamg(prec, maxit):
-    return va.SolverControls("PCG", "GAMG", 1e-9, 0.0, maxit, precision=prec, gamgSmoother=va.GAMG_GAUSS_SEIDEL,
-                             gamgPreSweeps=2, gamgPostSweeps=2)
-
-
-PRESSURE = [("gs_gamg_fp64", lambda: _gs_gamg(va.FP64, 12)), ("gs_gamg_mixed", lambda: _gs_gamg(va.MIXED, 12)),
-            ("dic_pcg", lambda: va.SolverControls("PCG", "DIC", 1e-8, 0.0, 60)),
-            ("gauss_seidel", lambda: va.SolverControls("GaussSeidel", "none", 1e-12, 0.0, 4, nSweeps=2)),
-            ("sym_gauss_seidel", lambda: va.SolverControls("symGaussSeidel", "none", 1e-12, 0.0, 3, nSweeps=1))]
-MOMENTUM = [("dilu_bicgstab", lambda: va.SolverControls("PBiCGStab", "DILU", 1e-10, 0.0, 50)),
-            ("dilu_bicgstab_mixed", lambda: va.SolverControls("PBiCGStab", "DILU", 1e-10, 0.0, 50, precision=va.MIXED))]
-
-
-def _solves(sweep, m):
-    ctx = _context(sweep)
-    out = {}
-    lm, A, b = W.pressure_system(ctx, m, seed=1, gamg=True, nonorth=False)
-    for name, ctl in PRESSURE:
-        x = np.zeros(m.n_cells)
-        out[name] = (x, va.solve_ldu(A, b, x, ctl()))
-        print(f"[sweeps]   {sweep} {name}: {out[name][1].iterations} iterations", flush=True)
-    A.close()
-    lm.close()
-    lm, A, b, inp = W.momentum_system(ctx, m, seed=1, comp=0)
-    for name, ctl in MOMENTUM:
-        x = np.ascontiguousarray(inp["U0"][:, 0]).copy()
-        out[name] = (x, va.solve_ldu(A, b, x, ctl()))
-        print(f"[sweeps]   {sweep} {name}: {out[name][1].iterations} iterations", flush=True)
-    A.close()
-    lm.close()
-    ctx.close()
-    return out
+SYM = [("PCG", "GAMG", 8, 1), ("PCG", "DIC", 30, 1), ("GaussSeidel", "none", 4, 2), ("symGaussSeidel", "none", 3, 1)]
 
 
 @pytest.mark.parametrize("mesh", ["tet", "box"])
-def test_sweep_forms_bit_identical(mesh):
+def test_mid_size_meshes_bit_exact_vs_oracle(ctx, mesh):
     m = M.tet(30, 28, 26, 0.2, 3) if mesh == "tet" else M.box(48, 40, 36)
-    print(f"[sweeps] {mesh}: {m.n_cells} cells, level-scheduled", flush=True)
-    ref = _solves("levels", m)
-    print(f"[sweeps] {mesh}: sync-free", flush=True)
-    got = _solves("free", m)
-    for name in ref:
-        (xr, pr), (xg, pg) = ref[name], got[name]
-        assert pg.iterations == pr.iterations and pg.finalResidual == pr.finalResidual, name
-        assert np.array_equal(xg, xr), name
-        print(f"[sweeps] {mesh} {name}: {pr.iterations} iterations, same bits", flush=True)
+    ni = m.n_internal
+    om = O.LduMesh(m.n_cells, m.owner[:ni], m.neighbour, m.agglomeration_weights())
+    lm, A, b = W.pressure_system(ctx, m, seed=1, gamg=True, nonorth=False)
+    lmm, Am, bm, inp = W.momentum_system(ctx, m, seed=1, comp=0)
+    runs = [(A, b, np.zeros(m.n_cells), *c) for c in SYM]
+    runs.append((Am, bm, np.ascontiguousarray(inp["U0"][:, 0]), "PBiCGStab", "DILU", 20, 1))
+    for mat, rhs, x0, solver, pre, mx, nsw in runs:
+        d, u, lo = mat.get()
+        xo, po = om.solve(d, u, None if mat is A else lo, rhs, x0=x0, solver=solver, preconditioner=pre,
+                          tolerance=1e-12, max_iter=mx, n_sweeps=nsw, mode=O.MODE_EXACT, smoother=O.SMOOTHER_GS)
+        x = x0.copy()
+        p = va.solve_ldu(mat, rhs, x, va.SolverControls(solver, pre, 1e-12, 0.0, mx, nSweeps=nsw, sums=va.SUMS_EXACT,
+                                                        gamgSmoother=va.GAMG_GAUSS_SEIDEL))
+        assert p.iterations == po["iterations"] and p.finalResidual == po["finalResidual"], (solver, pre)
+        assert np.array_equal(x, xo), (solver, pre)
+    for o in (A, Am, lm, lmm):
+        o.close()
+
+
+# ------------------------------------------------------------------ sequential float32 loops
+def _rows(n, own, nei):
+    """Per cell its faces in ascending order, the cells behind them and which coefficient
+    is its own row's (0: upper, the owner's)."""
+    nf = own.size
+    cell = np.concatenate([own, nei])
+    face = np.concatenate([np.arange(nf)] * 2)
+    order = np.lexsort((face, cell))
+    off = np.concatenate([[0], np.cumsum(np.bincount(cell, minlength=n))])
+    return off, np.concatenate([nei, own])[order], face[order]
+
+
+def _less(acc, terms):
+    """acc − t0 − t1 − … one after the other."""
+    return np.subtract.reduce(np.concatenate([[acc], terms]))
+
+
+def _dic32(n, own, nei, d, u, r):
+    """DIC in FP32 from an FP64 factor, entries by neighbour up and down the cells."""
+    off, nb, face = _rows(n, own, nei)
+    lower, upper, D = [], [], d.copy()
+    for c in range(n):
+        k = off[c] + np.argsort(nb[off[c]: off[c + 1]], kind="stable")
+        j, a = nb[k], u[face[k]]
+        lower.append((j[j < c], a[j < c]))
+        upper.append((j[j > c][::-1], a[j > c][::-1]))
+        jl, al = lower[c]
+        D[c] = _less(D[c], (al * al) / D[jl])
+    rD = 1.0 / D
+    w = np.zeros(n, F)
+    for c in range(n):
+        j, a = lower[c]
+        w[c] = _less(F(rD[c]) * r[c], (rD[c] * a).astype(F) * w[j])
+    for c in range(n - 1, -1, -1):
+        j, a = upper[c]
+        w[c] = _less(w[c], (rD[c] * a).astype(F) * w[j])
+    return w
+
+
+def _vcycle32(n, own, nei, d, u, r, om, sweeps):
+    """A V-cycle of two levels smoothed by Gauss–Seidel, in FP32 but for the coarsest solve."""
+    off, nb, face = _rows(n, own, nei)
+    a, dg = u[face].astype(F), d.astype(F)
+    x = np.zeros(n, F)
+
+    def sweep(cells):
+        for c in cells:
+            s = slice(off[c], off[c + 1])
+            x[c] = _less(r[c], a[s] * x[nb[s]]) / dg[c]
+
+    for _ in range(sweeps):
+        sweep(range(n))
+    fine, coarse = om.gamg_levels()
+    rc = np.zeros(coarse["n"], F)
+    for c in range(n):
+        s = slice(off[c], off[c + 1])
+        rc[fine["agg"][c]] += _less(r[c] - dg[c] * x[c], a[s] * x[nb[s]])
+    cd, cu, cl = om.gamg_coeffs(d, u, None, 1)
+    Ac = np.diag(cd)
+    Ac[coarse["l"], coarse["u"]], Ac[coarse["u"], coarse["l"]] = cu, cl
+    x += np.linalg.solve(Ac, rc.astype(np.float64)).astype(F)[fine["agg"]]
+    for _ in range(sweeps):
+        sweep(range(n - 1, -1, -1))
+    return x
+
+
+def _one_factor(x, p):
+    """Whether one α has x = float32(α·p) everywhere: α's interval of each element, half a
+    unit in the last place of x to either side, all have a point in common (to 1e-14, for
+    the rounding of the bounds themselves)."""
+    k = p != 0
+    assert np.array_equal(x[~k], p[~k]) and k.sum() > 0.9 * k.size
+    half = 0.5 * np.spacing(np.abs(x[k])).astype(np.float64)
+    a, b = (x[k] - half) / p[k].astype(np.float64), (x[k] + half) / p[k].astype(np.float64)
+    lo, hi = np.minimum(a, b).max(), np.maximum(a, b).min()
+    return lo <= hi + 1e-14 * abs(hi)
+
+
+@pytest.mark.parametrize("pre", ["DIC", "GAMG"])
+@pytest.mark.parametrize("name", ["one", "chain", "two", "wide", "hub", "box"])
+def test_fp32_sweeps_vs_sequential_float32(ctx, name, pre):
+    n, own, nei = sweep_graph(name)
+    rng = np.random.default_rng(21)
+    u = -rng.uniform(0.5, 1.5, own.size)
+    d = (0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)) * 2.0 ** rng.integers(0, 3, n)
+    d[:: 501] *= 2.0 ** 60  # a division outside the range of the reciprocal form
+    b = rng.uniform(-1, 1, n)
+    weights = rng.uniform(0.5, 1.5, own.size)
+    lm, om = va.LduMesh(ctx, n, own, nei, weights, 20), O.LduMesh(n, own, nei, weights, 20)
+    assert len(om.gamg_levels()) == 2
+    A = va.LduMatrix(lm, d, u)
+    x = np.zeros(n)
+    va.solve_ldu(A, b, x, va.SolverControls("PCG", pre, 1e-30, 0.0, 1, precision=va.MIXED,
+                                            gamgSmoother=va.GAMG_GAUSS_SEIDEL))
+    assert np.array_equal(x, x.astype(F))
+    p = _dic32(n, own, nei, d, u, b.astype(F)) if pre == "DIC" else _vcycle32(n, own, nei, d, u, b.astype(F), om, 2)
+    assert _one_factor(x.astype(F), p)
+    p[n // 2] += 3 * np.spacing(p[n // 2])
+    assert not _one_factor(x.astype(F), p)
+    A.close()
+    lm.close()

@@ -1,4 +1,4 @@
-"""GPU tests of the level-scheduled triangular sweeps: the DIC/DILU preconditioner
+"""GPU tests of the triangular sweeps: the DIC/DILU preconditioner
 (LinearSolver.cpp:56-105) and the Gauss–Seidel / symmetric Gauss–Seidel solvers
 (LinearSolver.cpp:238-278). Bar: with exact sums, every solve is bit-identical to the
 oracle's sequential restatement (which the CPU tests pin to the reference's own
@@ -160,9 +160,8 @@ def test_gamg_gauss_seidel_fast_mode_vs_reference(ctx, name):
 
 
 def test_sweeps_with_split_runs_bit_exact_vs_oracle(ctx):
-    """A 48k-cell tet mesh (20³ hexes × 6): its forward levels all hold ≤ 1024 cells, so
-    the one-workgroup runs together cover far more cells than one run's 16384 LDS slots
-    and are cut at level boundaries. Gauss–Seidel (2 sweeps), DILU-PBiCGStab and
+    """A 48k-cell tet mesh (20³ hexes × 6): more cells than one workgroup's LDS holds, in
+    levels of at most 1024, so each level's rows lie in several chunks. Gauss–Seidel (2 sweeps), DILU-PBiCGStab and
     PCG + GAMG smoothed by Gauss–Seidel, with exact sums: bit-identical to the oracle."""
     from voluma_amd import mesh as M
     m = M.tet(20, 20, 20, 0.2, 1)
