@@ -494,8 +494,6 @@ void toFloat(hipStream_t st, const double* a, float* w, size_t n) {
     launch_mix(st, MIX_TO32, int(n), a, w, nullptr, nullptr, nullptr, nullptr, nullptr);
 }
 
-// FP32 copies of the level-0 matrix and, with GAMG, of every coarse level and the tail
-// descriptors (the coarsest LU stays FP64). Values are rounded from the FP64 ones.
 // Forward / backward level order of a graph given by its edges (l[k] < u[k]): cells by
 // level, then by index; offF/offB hold the level offsets.
 void levelOrder(int n, const std::vector<int>& l, const std::vector<int>& u, std::vector<int>& offF,
@@ -754,6 +752,8 @@ void buildDilu32(vol_matrix A) {
     A->dilu32Ready = true;
 }
 
+// FP32 copies of the level-0 matrix and, with GAMG, of every coarse level and the tail
+// descriptors (the coarsest LU stays FP64). Values are rounded from the FP64 ones.
 void buildMixed(vol_matrix A, bool gamg) {
     vol_mesh m = A->mesh;
     hipStream_t st = m->ctx->stream;
@@ -1855,7 +1855,7 @@ void solveDevice(vol_matrix A, const double* b, double* x, const vol_solver_cont
             if (withW) pcgDiagonalStart<double>(C, A, P, k, ex);
             runLoop(c, C, maxLoops, [&] { krylovIteration<double>(C, A, P, k, isPCG, ex, withW); });
         } else {  // Jacobi and Gauss–Seidel solvers, LinearSolver.cpp:238-278
-            A->vw.alloc(n);
+            if (isJac) A->vw.alloc(n);
             const bool sym = P.solver == "symGaussSeidel";
             runLoop(c, C, maxLoops, [&] {
                 if (isGS && !sym)

@@ -1057,11 +1057,12 @@ __global__ __launch_bounds__(FIN_THREADS) void k_finalize(int op, int nred, int 
 }
 
 // The finalize of exact sums. Integer bins add up to the same value in any order, so the
-// blocks' partials are read by FINX_THREADS threads per sum, all sums at once: first the blocks' info words (one per
-// thread, nparts ≤ FINX_THREADS), then only the window of bins any block used, P threads
-// (the window rounded up to a power of two) per partial and FINX_LOADS loads in flight
-// each, a tree over the FINX_THREADS / P groups, and the carries and the conversion over
-// the window on one thread. Latency-bound: two round trips, the tree and ~10 bins in turn.
+// blocks' partials are read by FINX_THREADS threads per sum, all sums at once: first the
+// blocks' info words (one per thread, nparts ≤ FINX_THREADS), then only the window of bins
+// any block used, P threads (the window rounded up to a power of two) per partial and
+// FINX_LOADS loads in flight each, a tree over the FINX_THREADS / P groups, and the carries
+// and the conversion over the window on one thread. Latency-bound: two round trips, the
+// tree and ~10 bins in turn.
 // Adding the partials bin by bin on 72 threads and carrying through all 72 bins took 116 µs
 // per launch at 512 partials; a reproducible PCG iteration on 24,480 cells (then three of
 // these) went from 375 to 38 µs with this and the smaller grids of vec_exact_blocks, and to
