@@ -44,7 +44,7 @@ def test_sweeps_bit_exact_vs_oracle(ctx, name):
         assert np.array_equal(x, xo), (solver, sweeps)
 
 
-def test_values_before_the_sweep_past_the_halo(ctx):
+def test_values_before_the_sweep_past_the_halo(ctx, monkeypatch):
     """Enough chunks of long scattered rows that a chunk's neighbours do not fit its LDS:
     what is left of them is read where it lies, from x (at the start of every four sweeps)
     and, in the GAMG smoother's first sweeps, from the zero that x is taken as."""
@@ -54,6 +54,7 @@ def test_values_before_the_sweep_past_the_halo(ctx):
     d = 0.1 + np.bincount(own, -u, n) + np.bincount(nei, -u, n)
     rhs, x0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
     w = rng.uniform(0.5, 1.5, own.size)
+    monkeypatch.setenv("VOLUMA_AGGLOMERATION", "host")  # the same hierarchy; its hubs take the device 19 s
     lm, om = va.LduMesh(ctx, n, own, nei, w, 20), O.LduMesh(n, own, nei, w, 20)  # the graph, then the coarsest
     A = va.LduMatrix(lm, d, u)
     for solver, pre, sweeps, mx in (("GaussSeidel", "none", 2, 4), ("GaussSeidel", "none", 5, 5),
